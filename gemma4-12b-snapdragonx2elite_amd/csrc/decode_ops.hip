@@ -33,6 +33,7 @@ constexpr int NORM_THREADS = 1024;
 constexpr int ATT_THREADS = 256;
 constexpr int ATT_KPW = 8;        // keys per wave of an attention split (one K row per 8 lanes)
 constexpr int ATT_HPW = 4;        // query heads per attention workgroup (at most)
+constexpr int ATT_MMH = 16;       // query heads per workgroup of the matrix-core attention split
 constexpr int ATT_MAX_HD = 512;   // head dims up to 512 (global layers)
 
 
@@ -480,6 +481,10 @@ __device__ inline uint32_t load_pos(const uint32_t* dyn) {
   return __builtin_amdgcn_readfirstlane(__hip_atomic_load(dyn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
+// Partials of the attention splits: the unnormalised p V sums [nH][nsplit][hd],
+// then (m, l) pairs [nH][nsplit][2].
+__device__ inline float* attn_ml(float* part, int nH, int nsplit, int hd) { return part + (long)nH * nsplit * hd; }
+
 // Decode attention, split along the keys (vk/attn.comp:18-53,
 // flash-decoding). Workgroup (g, s): head group g = hpw query heads of one
 // KV head (they share that KV head's rows, so the rows are read once for all
@@ -702,69 +707,279 @@ attn_split_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, 
   __syncthreads();
   for (int i = t; i < hpw * HD; i += NT) {
     const int h = i / HD, c = i % HD;
-    float* o = part + ((long)(h0 + h) * nsplit + sp) * (HD + 2);
     float v = accp[0][h][c];
 #pragma unroll
     for (int w = 1; w < NW; ++w) v += accp[w][h][c];  // waves in order
-    o[2 + c] = v;
+    part[((long)(h0 + h) * nsplit + sp) * HD + c] = v;
   }
   if (t == 0) {
 #pragma unroll
     for (int h = 0; h < ATT_HPW; ++h) {
       if (h >= hpw) break;
-      float* o = part + ((long)(h0 + h) * nsplit + sp) * (HD + 2);
+      float* o = attn_ml(part, gridDim.x * hpw, nsplit, HD) + 2 * ((long)(h0 + h) * nsplit + sp);
       o[0] = mh[h];
       o[1] = lh[h];
     }
   }
 }
 
-// Head blockIdx.x, dims 64 blockIdx.y .. + 63, one wave (lane = dim):
+// The same split for 16 query heads of one KV head at hd 512 (the k == v
+// global layers), on fp32 matrix cores: scores and p V are 16-row products,
+// v_mfma_f32_16x16x4_f32 takes q and p as they are (fp32; K and V widened
+// from fp16 exactly), and the cache is read once for all 16 heads instead of
+// once per 4. What bounds it: the latency of one round of loads (each
+// workgroup requests its 32 K and V rows, 64 KB, before anything else), then
+// ~4,100 MFMA cycles per wave.
+//
+// Workgroup (g, sp): heads 16 g .., keys [32 sp, 32 sp + 32), 4 waves. For the
+// scores wave w takes the dims [64 w, +64) and [256 + 64 w, +64) of every
+// head and key: RoPE partners (i, i + 256) stay in one lane, and no wave
+// repeats another's q norm (only the sums of squares cross waves, through
+// LDS). Lane l holds row l % 16 (head or key) and, of each 32 dims, the 8
+// from 8 (l / 16): element e of the 8 is step e of the MFMA's k, the same
+// for both operands. The waves' partial scores meet in LDS; every wave then
+// takes the softmax of all 16 heads in the A layout of p V (lane: head
+// l % 16, keys 8 (l / 16) ..), which is a product over the wave's own 128
+// columns of V: lane column c of MFMA e is dim 8 c + e, so a lane's 16-byte
+// V load feeds 8 MFMAs and its results are 8 consecutive dims.
+// Measured at 8101 keys (256 splits, 16.6 MB of cache per layer, kernel
+// trace): 22.6 -> 14.7 us against the 4-head kernel.
+template <bool PREP>
+__global__ void __launch_bounds__(256)
+attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, const float* __restrict__ cs,
+                     const float* __restrict__ sn, uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int stride,
+                     int window, int qoff, int grp, const uint32_t* __restrict__ dyn, float* __restrict__ part,
+                     int nsplit, const float* __restrict__ knw, int koff, int voff) {
+  constexpr int EPL = 8, HD = 512, KCH = 32, NW = 4, SST = KCH + 4;  // SST: score row stride (words)
+  __shared__ __attribute__((aligned(16))) float sc[NW][ATT_MMH][SST];
+  __shared__ __attribute__((aligned(16))) uint16_t fresh[PREP ? NW : 1][2][PREP ? HD : 8];
+  __shared__ float ssq[NW][ATT_MMH];
+  const int h0 = blockIdx.x * ATT_MMH, sp = blockIdx.y, t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int kvh = h0 / grp, j0 = sp * KCH;
+  const long kv0 = (long)kvh * stride * HD;
+  const int li = lane & 15, lg = lane >> 4;
+  // dims of score chunk c (0..3): 8 from sdim(c); chunks c and c + 2 are RoPE partners
+  auto sdim = [&](int c) { return (c >> 1) * (HD / 2) + 64 * wave + (c & 1) * 32 + 8 * lg; };
+
+  // (1) every load of the split, none waiting for the position
+  const uint32_t pos = load_pos(dyn);
+  float q[4][8], wq[4][8], cr[4][8], sr[4][8], kr[EPL], vr[EPL], wk[EPL], crr[EPL], srr[EPL];
+  auto ld8f = [](const float* p, float(&v)[8]) {
+    const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  };
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int d = sdim(c);
+    ld8f(qkv + qoff + (long)(h0 + li) * HD + d, q[c]);
+    ld8f(qnw + d, wq[c]);
+    ld8f(cs + d, cr[c]);
+    ld8f(sn + d, sr[c]);
+  }
+  if constexpr (PREP) {
+    ld_row<EPL>(qkv + koff + kvh * HD, kr);
+    ld_row<EPL>(qkv + voff + kvh * HD, vr);
+    ld_row<EPL>(knw, wk);
+    ld_row<EPL>(cs, crr);
+    ld_row<EPL>(sn, srr);
+  }
+  v4u ku[2][4], vv[8];
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) {
+    const int j = min(j0 + 16 * kt + li, stride - 1);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) ku[kt][c] = *reinterpret_cast<const v4u*>(kc + kv0 + (long)j * HD + sdim(c));
+  }
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const int j = min(j0 + 8 * lg + s, stride - 1);
+    vv[s] = *reinterpret_cast<const v4u*>(vc + kv0 + (long)j * HD + 128 * wave + 8 * li);
+  }
+  const int T = att_len(pos, window, stride);
+  const int n = min(KCH, T - j0);  // <= 0 past the current length: the merge reads only the live splits
+  const int slot = kv_slot(pos, window);
+  const bool fresh_split = PREP && slot < stride && slot >= j0 && slot < j0 + n;  // workgroup-uniform
+
+  // (2) q norm and RoPE of this wave's dims; with the fresh slot in this
+  //     split, this token's K and V through the wave's own LDS rows
+  float s2 = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s2 = fmaf(q[c][e], q[c][e], s2);
+  s2 = slot_sum<16>(s2);
+  if (lg == 0) ssq[wave][li] = s2;
+  if constexpr (PREP) {
+    if (fresh_split) {
+      uint16_t kb[EPL], vb[EPL];
+      fresh_kv<EPL>(kr, vr, wk, crr, srr, kb, vb);
+      v4u k4, v4;
+      __builtin_memcpy(&k4, kb, 16);
+      __builtin_memcpy(&v4, vb, 16);
+      *reinterpret_cast<v4u*>(&fresh[wave][0][EPL * lane]) = k4;
+      *reinterpret_cast<v4u*>(&fresh[wave][1][EPL * lane]) = v4;
+      if (h0 % grp == 0 && wave == 0) {
+        const long o = ((long)kvh * stride + slot) * HD + EPL * lane;
+        *reinterpret_cast<v4u*>(kc + o) = k4;
+        *reinterpret_cast<v4u*>(vc + o) = v4;
+      }
+    }
+  }
+  __syncthreads();
+  if constexpr (PREP) {
+    if (fresh_split) {
+      const int kslot = slot - j0;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+        if (16 * kt + li == kslot) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) ku[kt][c] = *reinterpret_cast<const v4u*>(&fresh[wave][0][sdim(c)]);
+        }
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        if (8 * lg + s == kslot) vv[s] = *reinterpret_cast<const v4u*>(&fresh[wave][1][128 * wave + 8 * li]);
+    }
+  }
+  const float inv = inv_rms(((ssq[0][li] + ssq[1][li]) + ssq[2][li]) + ssq[3][li], HD);
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float lo = __fmul_rn(__fmul_rn(q[c][e], inv), wq[c][e]);
+      const float hi = __fmul_rn(__fmul_rn(q[c + 2][e], inv), wq[c + 2][e]);
+      q[c][e] = __fadd_rn(__fmul_rn(lo, cr[c][e]), __fmul_rn(-hi, sr[c][e]));
+      q[c + 2][e] = __fadd_rn(__fmul_rn(hi, cr[c + 2][e]), __fmul_rn(lo, sr[c + 2][e]));
+    }
+
+  // (3) this wave's part of the scores: D column l % 16 = key, rows 4 (l / 16) .. = heads
+  auto half_at = [](const v4u& u, int e) { return h2f((uint16_t)(e & 1 ? u[e >> 1] >> 16 : u[e >> 1] & 0xFFFFu)); };
+  v4f d[2][2] = {};  // [key tile][chunk parity]
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+        d[kt][c & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[c][e], half_at(ku[kt][c], e), d[kt][c & 1], 0, 0, 0);
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float sum = d[kt][0][v] + d[kt][1][v];
+      sc[wave][4 * lg + v][16 * kt + li] = sum;
+    }
+  __syncthreads();
+
+  // (4) softmax over the split's keys: lane = head li, keys 8 lg .. + 7
+  float p[8];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    v4f x = *reinterpret_cast<const v4f*>(&sc[0][li][8 * lg + 4 * b]);
+#pragma unroll
+    for (int w = 1; w < NW; ++w) x += *reinterpret_cast<const v4f*>(&sc[w][li][8 * lg + 4 * b]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[4 * b + e] = 8 * lg + 4 * b + e < n ? x[e] : -INFINITY;
+  }
+  float m = p[0];
+#pragma unroll
+  for (int s = 1; s < 8; ++s) m = fmaxf(m, p[s]);
+  m = slot_reduce<16, true>(m);
+  float l = 0.0f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    p[s] = p[s] != -INFINITY ? expf(p[s] - m) : 0.0f;
+    l += p[s];
+  }
+  l = slot_sum<16>(l);
+
+  // (5) unnormalised p V over the wave's 128 dims. Rows past the length are
+  //     taken as zero (a never-written cache row may hold a NaN).
+  v4f o[8] = {};
+#pragma unroll
+  for (int s = 0; s < 8; ++s)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float v = 8 * lg + s < n ? half_at(vv[s], e) : 0.0f;
+      o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], v, o[e], 0, 0, 0);
+    }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    float* dst = part + ((long)(h0 + 4 * lg + v) * nsplit + sp) * HD + 128 * wave + 8 * li;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dst[e] = o[e][v];
+  }
+  if (t < ATT_MMH) {
+    float* ml = attn_ml(part, gridDim.x * ATT_MMH, nsplit, HD) + 2 * ((long)(h0 + t) * nsplit + sp);
+    ml[0] = m;
+    ml[1] = l;
+  }
+}
+
+// Head blockIdx.x, dims 64 blockIdx.y .. + 63 (lane = dim), NW waves:
 // out = sum_c acc_c e^(m_c - M) / sum_c l_c e^(m_c - M), M = max_c m_c,
-// over the live splits c. No barrier: the wave loads its dims of the first
-// MB splits and the (m, l) of splits lane, lane + 64, .. before the position
-// (which sets the live split count) arrives, takes M and L with cross-lane
-// reductions (lane c holds split c, c + 64, ..), passes the weights through
-// its own LDS and sums the splits in order. Per head and dim the arithmetic
-// and its order are the same whichever wave does it. ml: nsplit floats of
-// dynamic shared memory. out fp32 or fp16.
-template <int YT, int EPL, int MB>
-__global__ void __launch_bounds__(64) attn_merge_kernel(const float* __restrict__ part, void* __restrict__ out,
-                                                        int nsplit, int kch, int stride, int window,
-                                                        const uint32_t* __restrict__ dyn) {
+// over the live splits c; wave w sums splits w, w + NW, .. in order, then the
+// waves' sums are added in order. The wave loads its dims of its first MB
+// splits and the (m, l) of splits lane, lane + 64, .. before the position
+// (which sets the live split count) arrives, takes M with a cross-lane
+// maximum (lane c holds split c, c + 64, ..); the weights e^(m_c - M) go
+// through LDS. One wave and no barrier up to 32 splits; 8 waves above, where
+// one wave's batches of 32 loads were a serial chain of memory round trips
+// (254 splits of 16 heads, hd 512: 17.4 -> 5.2 us).
+// ml: nsplit floats of dynamic shared memory. out fp32 or fp16.
+template <int YT, int EPL, int MB, int NW>
+__global__ void __launch_bounds__(64 * NW) attn_merge_kernel(const float* __restrict__ part, void* __restrict__ out,
+                                                             int nsplit, int kch, int stride, int window,
+                                                             const uint32_t* __restrict__ dyn) {
   constexpr int HD = 64 * EPL;
   extern __shared__ float ml[];
-  const int h = blockIdx.x, t = threadIdx.x, d = blockIdx.y * 64 + t;
-  const float* w = part + (long)h * nsplit * (HD + 2);
+  __shared__ float red[NW][64], redl[NW];
+  const int h = blockIdx.x, t = threadIdx.x & 63, d = blockIdx.y * 64 + t;
+  const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const float* w = part + (long)h * nsplit * HD;
+  const float2* wml = reinterpret_cast<const float2*>(part + (long)gridDim.x * nsplit * HD) + (long)h * nsplit;
   // indices clamped to the workspace until the live split count is known
   float x[MB];
   auto fetch = [&](int c0, int cmax) {
 #pragma unroll
-    for (int c = 0; c < MB; ++c) x[c] = w[(long)min(c0 + c, cmax) * (HD + 2) + 2 + d];
+    for (int c = 0; c < MB; ++c) x[c] = w[(long)min(c0 + NW * c, cmax) * HD + d];
   };
-  fetch(0, nsplit - 1);
-  const int c_t = min(t, nsplit - 1);
-  const float m_t = w[(long)c_t * (HD + 2)], l_t = w[(long)c_t * (HD + 2) + 1];
+  fetch(wave, nsplit - 1);
+  const float2 ml_t = wml[min(t, nsplit - 1)];
   const int T = att_len(load_pos(dyn), window, stride);
   const int ns = (T + kch - 1) / kch;
-  float M = t < ns ? m_t : -INFINITY;
-  for (int c = t + 64; c < ns; c += 64) M = fmaxf(M, w[(long)c * (HD + 2)]);
+  float M = t < ns ? ml_t.x : -INFINITY;
+  for (int c = t + 64; c < ns; c += 64) M = fmaxf(M, wml[c].x);
   M = reduce64<true>(M);
   float L = 0.0f;
-  for (int c = t; c < ns; c += 64) {
-    const float mc = c == t ? m_t : w[(long)c * (HD + 2)];
-    const float lc = c == t ? l_t : w[(long)c * (HD + 2) + 1];
-    const float wc = expf(mc - M);
+  for (int c = threadIdx.x; c < ns; c += 64 * NW) {
+    const float2 mc = c == t ? ml_t : wml[c];
+    const float wc = expf(mc.x - M);
     ml[c] = wc;
-    L = fmaf(lc, wc, L);
+    L = fmaf(mc.y, wc, L);
   }
   L = reduce64<false>(L);
+  if constexpr (NW > 1) {
+    if (t == 0) redl[wave] = L;
+    __syncthreads();
+    L = redl[0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) L += redl[i];
+  }
   float acc = 0.0f;
-  for (int c0 = 0; c0 < ns; c0 += MB) {
-    if (c0 > 0) fetch(c0, ns - 1);
+  for (int c0 = wave; c0 < ns; c0 += MB * NW) {
+    if (c0 > wave) fetch(c0, ns - 1);
 #pragma unroll
     for (int c = 0; c < MB; ++c)
-      if (c0 + c < ns) acc = fmaf(x[c], ml[c0 + c], acc);
+      if (c0 + NW * c < ns) acc = fmaf(x[c], ml[c0 + NW * c], acc);
+  }
+  if constexpr (NW > 1) {
+    red[wave][t] = acc;
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int i = 1; i < NW; ++i) acc += red[i][t];
   }
   const float v = acc / L;
   if constexpr (YT == Q4_DT_F16) reinterpret_cast<uint16_t*>(out)[h * HD + d] = f2h(v);
@@ -970,21 +1185,37 @@ static int attn_launch(const float* qkv, const float* qnw, const float* cosb, co
 #define Q4_ATT(E, P, W)                                                                                               \
   hipLaunchKernelGGL((attn_split_kernel<E, P, W>), grid, blk, 0, st, qkv, qnw, cosb, sinb, kc, vc, stride, window, \
                      qoff, grp, hpw, dyn, part, ns, knw, koff, voff)
-  // the merge fetches its splits MB at a time: the smallest of 8, 16, 32 that covers them all, or 32
-#define Q4_MRG2(E, MB)                                                                                               \
-  if (h16) hipLaunchKernelGGL((attn_merge_kernel<Q4_DT_F16, E, MB>), dim3(nH, E), dim3(64), msh, st, part, out, ns, \
-                              kch, stride, window, dyn);                                                            \
-  else hipLaunchKernelGGL((attn_merge_kernel<Q4_DT_F32, E, MB>), dim3(nH, E), dim3(64), msh, st, part, out, ns,     \
+  // the merge fetches its splits MB per wave at a time: one wave and the smallest of 8, 16, 32 that covers them all,
+  // else 8 waves of 32
+#define Q4_MRG2(E, MB, W)                                                                                             \
+  if (h16) hipLaunchKernelGGL((attn_merge_kernel<Q4_DT_F16, E, MB, W>), dim3(nH, E), dim3(64 * W), msh, st, part, out, \
+                              ns, kch, stride, window, dyn);                                                         \
+  else hipLaunchKernelGGL((attn_merge_kernel<Q4_DT_F32, E, MB, W>), dim3(nH, E), dim3(64 * W), msh, st, part, out, ns, \
                           kch, stride, window, dyn)
 #define Q4_MRG(E)                  \
-  if (ns <= 8) { Q4_MRG2(E, 8); }  \
-  else if (ns <= 16) { Q4_MRG2(E, 16); } \
-  else { Q4_MRG2(E, 32); }
+  if (ns <= 8) { Q4_MRG2(E, 8, 1); }  \
+  else if (ns <= 16) { Q4_MRG2(E, 16, 1); } \
+  else if (ns <= 32) { Q4_MRG2(E, 32, 1); } \
+  else { Q4_MRG2(E, 32, 8); }
   switch (hd) {
     case 64: if (prep) { Q4_ATT(1, true, 8); } else { Q4_ATT(1, false, 8); } break;
     case 128: if (prep) { Q4_ATT(2, true, 8); } else { Q4_ATT(2, false, 8); } break;
     case 256: if (prep) { Q4_ATT(4, true, 8); } else { Q4_ATT(4, false, 8); } break;
-    default: if (prep) { Q4_ATT(8, true, 4); } else { Q4_ATT(8, false, 4); } break;
+    default:
+      // whole 16-head groups of one KV head fill the matrix cores' 16 rows; other groupings keep the 4-head kernel
+      if (grp % ATT_MMH == 0) {
+        const dim3 mgrid(nH / ATT_MMH, ns);
+        void (*fn)(const float*, const float*, const float*, const float*, uint16_t*, uint16_t*, int, int, int, int,
+                   const uint32_t*, float*, int, const float*, int, int) =
+            prep ? attn_split_mm_kernel<true> : attn_split_mm_kernel<false>;
+        hipLaunchKernelGGL(fn, mgrid, dim3(256), 0, st, qkv, qnw, cosb, sinb, kc, vc, stride, window, qoff, grp, dyn,
+                           part, ns, knw, koff, voff);
+      } else if (prep) {
+        Q4_ATT(8, true, 4);
+      } else {
+        Q4_ATT(8, false, 4);
+      }
+      break;
   }
   Q4_LAUNCHED("attn_split");
   switch (hd) {
