@@ -8,24 +8,20 @@
 //          (vk/coopgemm_i4h.comp, which accumulates in f16; this one
 //          accumulates in fp32)          v_mfma_f32_32x32x16_f16
 //
-// Both kernels stage the activation tile A through an LDS ring filled by
+// The kernels stage the activation tile A through an LDS ring filled by
 // direct-to-LDS loads (global_load_lds_dwordx4: no VGPR round trip, no
-// staging registers) and feed 4 waves (2 x 2, each a (BM/2) x 128 block of
-// 32x32 MFMA tiles) from it. They differ in how the weight operand B
-// arrives:
+// staging registers) and differ in how the weight operand B arrives:
 //  * W8A8 (w8a8_kernel): int8 rows are loaded into registers one and a half
 //    k-steps ahead and written into a second LDS ring; fragments are read
 //    from LDS like A's. Direct-to-LDS loads sustain only ~24 B/clk per CU on
 //    MI355X, half of what the 256x256 tile needs, so the two operands take
 //    the two load paths.
-//  * W4A16 / W4A8 (w4_kernel): each lane loads the 8-byte half of a
-//    32-element int4 unit that its MFMA fragment needs (the panel-64 layout
-//    makes the 32 rows of a fragment 512 contiguous bytes) several k-steps
+//  * W4A16 (w4p_kernel) and W4A8 (w4a8_kernel): each lane loads the 8-byte
+//    half of a 32-element int4 unit that its MFMA fragment needs (the
+//    panel-64 layout makes the 32 rows of a fragment 512 contiguous bytes)
 //    ahead, and dequantizes (f16) or requantizes (int8) it straight into
 //    fragment registers. B never touches LDS, which leaves LDS bandwidth to
-//    A: with the 128-row tiles that M = 512 needs, staging both operands in
-//    LDS would need more than the ~128 B/clk LDS read bandwidth per CU.
-//    The k order inside a fragment is permuted consistently for A and B
+//    A. The k order inside a fragment is permuted consistently for A and B
 //    (a dot product does not care) so each lane's 16 k-values come from one
 //    contiguous half-unit.
 //
@@ -49,8 +45,6 @@
 #include "q4mi_common.h"
 
 namespace q4 {
-
-enum { OP_W8A8 = 0, OP_W4A16 = 1, OP_W4A8 = 2 };
 
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -79,30 +73,12 @@ __device__ inline int lds_off(int r, int c) { return r * 64 + ((c ^ swz(r)) << 4
 
 __device__ inline uint32_t pk_h2(v2h v) { return __builtin_bit_cast(uint32_t, v); }
 
-// One device word (8 int4 codes, k order e = 0..7 at nibble (e&1)*4 + (e>>1))
-// -> 8 f16 values f16((q - 8) * s) in k order. Low nibbles: 0x6400 | q =
-// 1024 + q; high nibbles: 0x6400 | 16q = 1024 + 16q. Both become q - 8
-// exactly, then one RNE multiply by s: the reference's
-// float16_t((float(q) - 8.0) * scl) (vk/coopgemm_i4h.comp:24).
-__device__ inline v4u dequant_word_f16(uint32_t w, v2h sv) {
-  const v2h off_lo = {(_Float16)1032.0f, (_Float16)1032.0f};
-  const v2h sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-  const v2h off_hi = {(_Float16)72.0f, (_Float16)72.0f};
-  const uint32_t w8 = w >> 8;
-  v2h p0 = __builtin_bit_cast(v2h, (w & 0x000F000Fu) | 0x64006400u);
-  v2h p1 = __builtin_bit_cast(v2h, (w & 0x00F000F0u) | 0x64006400u);
-  v2h p2 = __builtin_bit_cast(v2h, (w8 & 0x000F000Fu) | 0x64006400u);
-  v2h p3 = __builtin_bit_cast(v2h, (w8 & 0x00F000F0u) | 0x64006400u);
-  p0 = (p0 - off_lo) * sv;
-  p1 = (p1 * sixteenth - off_hi) * sv;
-  p2 = (p2 - off_lo) * sv;
-  p3 = (p3 * sixteenth - off_hi) * sv;
-  return v4u{pk_h2(p0), pk_h2(p1), pk_h2(p2), pk_h2(p3)};
-}
-
-// Pair P (codes e = 2P, 2P + 1 in k order) of dequant_word_f16, in three VALU
-// operations: high nibbles use 0x5400 | 16q = 64 + q (ulp 1/16), so both
-// halves become q - 8 with one exact add before the RNE multiply by s. mlo =
+// Pair P (codes e = 2P, 2P + 1 in k order, nibble (e & 1) * 4 + (e >> 1)) of a
+// device word -> two f16((q - 8) * s), the reference's
+// float16_t((float(q) - 8.0) * scl) (vk/coopgemm_i4h.comp:24), in three VALU
+// operations: low nibbles use 0x6400 | q = 1024 + q, high nibbles
+// 0x5400 | 16q = 64 + q (ulp 1/16), so both halves become q - 8 with one
+// exact add before the RNE multiply by s. mlo =
 // 0x64006400 and mhi = 0x54005400 come in VGPRs: v_and_or_b32 takes no
 // literal constants, and the masks go to SGPRs.
 template <int P>
@@ -1372,202 +1348,243 @@ __global__ void __launch_bounds__(256 * KG) w4p_kernel(const GemmArgs g, int spl
   }
 }
 
-// ---- W4A16 / W4A8 ---------------------------------------------------------------
-// BM x 256 tile, K step one 64-byte A row (32 f16 for W4A16, 64 int8 for
-// W4A8). A: S-stage LDS ring of direct loads (k-step j + S goes into the
-// stage k-step j used). B: each lane's half-units for its FN tiles, loaded
-// three k-steps ahead into a 4-deep register ring, converted to fragments
-// one k-step ahead.
-//   W4A16, slice s (16 k), lane half h: B = dequant(word 2h + s of the unit
-//     of block kt) = k 16h + 8s .. + 8; A = chunk 2h + s of the row.
-//   W4A8, slice s (32 k = block 2kt + s), half h: B = requant(words 2h,
-//     2h + 1 of that block's unit) = k 32s + 16h .. + 16; A = chunk 2s + h.
-template <int OP, int BM>
-__global__ void __launch_bounds__(256) w4_kernel(const GemmArgs g, int split) {
-  constexpr bool F16 = (OP == OP_W4A16);
-  constexpr int BN = 256, WM = BM / 2, WN = 128, FM = WM / 32, FN = 4;
-  constexpr int S = BM == 128 ? 8 : 6;        // A ring stages
-  constexpr int NA = BM / 64;                 // A direct loads per thread per k-step
-  constexpr int NBLK = F16 ? 1 : 2;           // int4 blocks per k-step
-  constexpr int NBR = 2 * NBLK * FN;          // B loads per thread per k-step (half-unit + scale per block per tile)
-  constexpr int AST = BM * 64;
-  constexpr int EPI = 4 * WM * EST * 4;
-  constexpr int LA = S * AST > EPI ? S * AST : EPI;
-  static_assert(S >= 5, "the wait counts assume A(j + 2) is issued before B(j + 1)");
-  __shared__ __attribute__((aligned(16))) uint8_t ldsA[LA];
-  typedef typename std::conditional<F16, v16f, v16i>::type acc_t;
+// ---- W4A8, waves split along K ----------------------------------------------------
+// BM x BN tile, 8 waves (two per SIMD). Every wave computes the whole tile
+// over its share of the k-steps of 64 (wave w takes steps w, w + 8, ..), so a
+// weight is requantized once per M-tile and the grid can be narrow in N:
+// with the waves side by side in N and M a 256-column tile gave the chunk
+// shape (M 128, N 15360) 60 workgroups, each one wave per SIMD bound by its
+// own requantization. Measured against that kernel: M 128, N 15360, K 3840
+// 146.6 -> 20.6 us; M 128, N 3840, K 15360 537 -> 23.2 us (15 workgroups
+// before); M 20, N 15360 142 -> 12.9 us; M 1024, N 15360 292 -> 144 us.
+// A: a two-stage LDS ring per wave (direct loads, no barrier in the k-loop:
+// a wave reads only what it loaded). B: half-units and ratios two steps ahead
+// in a three-set register ring, requantized to fragments in pairs
+// (requant_half). The MFMAs are w8a8's: lane half h of k-slice s holds
+// k 32 s + 16 h .. + 16. The waves' int32 sums meet in LDS (integer adds: the
+// result does not depend on their order), and all 8 waves run the epilogue.
+// What bounds it: the direct loads of A (BM x K bytes per workgroup).
+//
+// Low 8 bits of the two halves of 1536 + rint((q - 8) r): one pair of codes
+// as in dequant_pair_f16 (q - 8 exact), then one fused multiply-add whose
+// single rounding, at an f16 ulp of 1 in [1024, 2048), is rint of the exact
+// product with ties to even. Holds while |8 r| < 127.5 (no clamp acts).
+template <int P>
+__device__ inline uint32_t requant_pair(uint32_t w, v2h rv, uint32_t mlo, uint32_t mhi) {
+  const uint32_t x = P >= 2 ? w >> 8 : w;
+  const v2h magic = {(_Float16)1536.0f, (_Float16)1536.0f};
+  v2h p;
+  if constexpr (P & 1) {
+    const v2h off = {(_Float16)-72.0f, (_Float16)-72.0f};
+    p = __builtin_bit_cast(v2h, (x & 0x00F000F0u) | mhi) + off;
+  } else {
+    const v2h off = {(_Float16)-1032.0f, (_Float16)-1032.0f};
+    p = __builtin_bit_cast(v2h, (x & 0x000F000Fu) | mlo) + off;
+  }
+  return pk_h2(__builtin_elementwise_fma(p, rv, magic));
+}
+// requant_words_i8 for ratios that need no clamp (see above)
+__device__ inline v4i requant_half(v2u u, uint32_t rbits, uint32_t mlo, uint32_t mhi) {
+  const v2h rv = __builtin_bit_cast(v2h, rbits | (rbits << 16));
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t w = u[i];
+    o[2 * i] = __builtin_amdgcn_perm(requant_pair<1>(w, rv, mlo, mhi), requant_pair<0>(w, rv, mlo, mhi), 0x06040200u);
+    o[2 * i + 1] = __builtin_amdgcn_perm(requant_pair<3>(w, rv, mlo, mhi), requant_pair<2>(w, rv, mlo, mhi), 0x06040200u);
+  }
+  return v4i{(int)o[0], (int)o[1], (int)o[2], (int)o[3]};
+}
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int M = g.M, N = g.N, K = g.K;
+constexpr int W4A8_WAVES = 8;
+template <int BM, int BN>
+__global__ void __launch_bounds__(64 * W4A8_WAVES) w4a8_kernel(const GemmArgs g) {
+  constexpr int NW = W4A8_WAVES, FM = BM / 32, FN = BN / 32;
+  constexpr int NA = BM / 16;        // A direct loads per step (16 rows of 64 bytes each)
+  constexpr int NB = 4 * FN;         // B loads per lane per step: n-tile x block x (half-unit, ratio)
+  constexpr int AST = BM * 64, RING = NW * 2 * AST;
+  constexpr int OST = BN + 4;        // sum row stride (words)
+  constexpr int LDSB = RING > BM * OST * 4 ? RING : BM * OST * 4;
+  static_assert(LDSB <= 160 * 1024 && NA + 2 * NB < 64, "LDS and wait count");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[LDSB];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int M = g.M, N = g.N, K = g.K, nblk = K / BLK, nk = K / 64;
   int tm, tn;
   tile_of(blockIdx.x, gridDim.x, (M + BM - 1) / BM, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
-  const int nblk = K / BLK;
-  const int nk_all = F16 ? nblk : nblk / 2;
-  const int kz = blockIdx.y;
-  const int k_lo = (int)((long)kz * nk_all / split), nk = (int)((long)(kz + 1) * nk_all / split) - k_lo;
-  const long a_row_bytes = F16 ? 2L * K : (long)K;
+  const int h = lane >> 5, frow = lane & 31;
+  uint8_t* const ring = lds + wave * (2 * AST);
 
   const uint8_t* asrc[NA];
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
-    const int r = (wave * NA + i) * 16 + (lane >> 2);
-    asrc[i] = reinterpret_cast<const uint8_t*>(g.A) + (long)min(m0 + r, M - 1) * a_row_bytes + (long)k_lo * 64 +
-              (((lane & 3) ^ swz(r)) << 4);
+    const int r = 16 * i + (lane >> 2);
+    asrc[i] = reinterpret_cast<const uint8_t*>(g.A) + (long)min(m0 + r, M - 1) * K + (((lane & 3) ^ swz(r)) << 4);
   }
-  // B: tile j covers rows n0 + wn * 128 + 32 j + lane % 32; lane half h = lane / 32
-  const int h = lane >> 5;
-  const uint8_t* Bu = reinterpret_cast<const uint8_t*>(g.B);
-  long bidx[FN];  // panel index of (row, block k_lo * NBLK)
+  const uint8_t* bsrc[FN];
+  const uint8_t* rsrc[FN];
 #pragma unroll
-  for (int j = 0; j < FN; ++j) bidx[j] = panel_index(min(n0 + wn * WN + 32 * j + (lane & 31), N - 1), k_lo * NBLK, nblk);
-
-  v2u ru[4][FN][NBLK];
-  uint32_t rs[4][FN][NBLK];
-#define W4_LOAD_B(set_, kt_)                                                                         \
-  do {                                                                                               \
-    const long bo_ = (long)min((kt_), nk - 1) * NBLK * PANEL;                                        \
-    _Pragma("unroll") for (int j = 0; j < FN; ++j)                                                   \
-      _Pragma("unroll") for (int b = 0; b < NBLK; ++b) {                                             \
-        const long ix_ = bidx[j] + bo_ + b * PANEL;                                                  \
-        ru[set_][j][b] = ld8(Bu + ix_ * 16 + 8 * h);                                                 \
-        rs[set_][j][b] = ld2(g.bsc + ix_);                                                           \
-      }                                                                                              \
-  } while (0)
-#define W4_LOAD_A(kt_)                                                                               \
-  do {                                                                                               \
-    const long ko_ = (long)min((kt_), nk - 1) * 64;                                                  \
-    uint8_t* st_ = ldsA + ((kt_) % S) * AST;                                                         \
-    _Pragma("unroll") for (int i = 0; i < NA; ++i) dma16(asrc[i] + ko_, st_ + (wave * NA + i) * 1024); \
-  } while (0)
-
-  acc_t acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = acc_t{};
-
-  const int frow = lane & 31;
-  auto rdA = [&](int stage, int i, int s) {
-    const int c = F16 ? 2 * h + s : 2 * s + h;
-    return *reinterpret_cast<const v4i*>(ldsA + stage * AST + lds_off(wm * WM + 32 * i + frow, c));
-  };
-  v4i fa[2][2][FM], fb[2][2][FN];  // [buffer][k-slice][tile]
-#define W4_MAKE_B(buf_, set_)                                                                        \
-  do {                                                                                               \
-    _Pragma("unroll") for (int j = 0; j < FN; ++j) {                                                 \
-      pin(ru[set_][j][0]);                                                                           \
-      pin(rs[set_][j][0]);                                                                           \
-      if constexpr (F16) {                                                                           \
-        const _Float16 s_ = __builtin_bit_cast(_Float16, (uint16_t)rs[set_][j][0]);                   \
-        const v2h sv_ = {s_, s_};                                                                    \
-        fb[buf_][0][j] = __builtin_bit_cast(v4i, dequant_word_f16(ru[set_][j][0].x, sv_));           \
-        fb[buf_][1][j] = __builtin_bit_cast(v4i, dequant_word_f16(ru[set_][j][0].y, sv_));           \
-      } else {                                                                                       \
-        pin(ru[set_][j][NBLK - 1]);                                                                  \
-        pin(rs[set_][j][NBLK - 1]);                                                                  \
-        _Pragma("unroll") for (int b = 0; b < NBLK; ++b) fb[buf_][b][j] = __builtin_bit_cast(v4i,   \
-            requant_words_i8(ru[set_][j][b].x, ru[set_][j][b].y, h2f((uint16_t)rs[set_][j][b])));      \
-      }                                                                                              \
-    }                                                                                                \
-  } while (0)
-
-  // prologue in the steady-state issue order: A0 .. A(S-4), [B0 A(S-3)], [B1 A(S-2)], [B2 A(S-1)]
-#pragma unroll
-  for (int s = 0; s < S - 3; ++s) W4_LOAD_A(s);
-  W4_LOAD_B(0, 0);
-  W4_LOAD_A(S - 3);
-  W4_LOAD_B(1, 1);
-  W4_LOAD_A(S - 2);
-  W4_LOAD_B(2, 2);
-  W4_LOAD_A(S - 1);
-  vmwait<3 * NA + 2 * NBR>();  // B0 and A0 .. A(S-4) landed
-  W4_MAKE_B(0, 0);
-  __builtin_amdgcn_s_barrier();  // stages 0 and 1 visible
-#pragma unroll
-  for (int sl = 0; sl < 2; ++sl)
-#pragma unroll
-    for (int i = 0; i < FM; ++i) fa[0][sl][i] = rdA(0, i, sl);
-  lgkm0();
-  __builtin_amdgcn_s_barrier();  // stage 0 read by every wave: the first k-step may refill it
-
-  constexpr int NMF = 2 * FM * FN;
-#define W4_KSTEP(cur, nxt, bset_load, bset_make)                                                     \
-  do {                                                                                               \
-    W4_LOAD_B(bset_load, kt + 3);                                                                    \
-    W4_LOAD_A(kt + S);                                                                               \
-    vmwait<3 * NA + 2 * NBR>(); /* B(kt + 1) landed, and A(kt + 2) before it */                      \
-    const int st1 = (kt + 1) % S;                                                                    \
-    _Pragma("unroll") for (int sl = 0; sl < 2; ++sl)                                                 \
-      _Pragma("unroll") for (int i = 0; i < FM; ++i) fa[nxt][sl][i] = rdA(st1, i, sl);               \
-    W4_MAKE_B(nxt, bset_make);                                                                       \
-    _Pragma("unroll") for (int sl = 0; sl < 2; ++sl)                                                 \
-      _Pragma("unroll") for (int i = 0; i < FM; ++i)                                                 \
-        _Pragma("unroll") for (int j = 0; j < FN; ++j) {                                             \
-          if constexpr (F16)                                                                         \
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, fa[cur][sl][i]), \
-                          __builtin_bit_cast(v8h, fb[cur][sl][j]), acc[i][j], 0, 0, 0);              \
-          else                                                                                       \
-            acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[cur][sl][i], fb[cur][sl][j], acc[i][j], 0, 0, 0); \
-        }                                                                                            \
-    if constexpr (F16) { /* W4A8 (not a throughput path) is left to the default scheduler */       \
-      __builtin_amdgcn_sched_group_barrier(0x100, 2 * FM, 0);                                        \
-      _Pragma("unroll") for (int q = 0; q < NMF; ++q) {                                              \
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                           \
-        __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);                                           \
-      }                                                                                              \
-    }                                                                                                \
-    lgkm0();                                                                                         \
-    __builtin_amdgcn_s_barrier(); /* k-step kt + 2 visible; stage kt free */                         \
-  } while (0)
-  // register ring: B(kt) in set kt % 4; fragment buffers alternate with kt % 2
-  int kt = 0;
-  for (; kt + 3 < nk; kt += 4) {
-    W4_KSTEP(0, 1, 3, 1);
-    ++kt;
-    W4_KSTEP(1, 0, 0, 2);
-    ++kt;
-    W4_KSTEP(0, 1, 1, 3);
-    ++kt;
-    W4_KSTEP(1, 0, 2, 0);
-    kt -= 3;
+  for (int j = 0; j < FN; ++j) {
+    const long u = panel_index(min(n0 + 32 * j + frow, N - 1), 0, nblk);
+    bsrc[j] = reinterpret_cast<const uint8_t*>(g.B) + u * 16 + 8 * h;
+    rsrc[j] = reinterpret_cast<const uint8_t*>(g.bsc) + u * 2;
   }
-  if (kt < nk) {
-    W4_KSTEP(0, 1, 3, 1);
-    ++kt;
-    if (kt < nk) {
-      W4_KSTEP(1, 0, 0, 2);
-      ++kt;
-      if (kt < nk) W4_KSTEP(0, 1, 1, 3);
-    }
-  }
-#undef W4_KSTEP
-#undef W4_LOAD_A
-#undef W4_LOAD_B
-#undef W4_MAKE_B
-  vmwait<0>();
-  // keep the last k-steps' (unused) B registers live until their loads landed:
-  // otherwise the compiler may reuse them for epilogue addresses
-#pragma unroll
-  for (int s = 0; s < 4; ++s)
+  uint32_t mlo = 0x64006400u, mhi = 0x54005400u;  // requant_pair's VGPR operands
+  asm volatile("" : "+v"(mlo), "+v"(mhi));
+
+  // the wave's steps: k-steps wave, wave + NW, .. (possibly none); loads past the last one repeat it
+  const int ns = (nk - wave + NW - 1) / NW;
+  auto kstep_of = [&](int s) { return min(wave + NW * s, nk - 1); };
+  v2u ru[3][FN][2];
+  uint32_t rr[3][FN][2];
+  auto load_b = [&](auto setc, int s) {
+    constexpr int set = decltype(setc)::value;
+    const long blk = 2L * kstep_of(s);
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int b = 0; b < NBLK; ++b) {
-        pin(ru[s][j][b]);
-        pin(rs[s][j][b]);
+      for (int b = 0; b < 2; ++b) {
+        ru[set][j][b] = ld8(bsrc[j] + (blk + b) * (PANEL * 16));
+        rr[set][j][b] = ld2(rsrc[j] + (blk + b) * (PANEL * 2));
       }
-  __builtin_amdgcn_s_barrier();  // every direct load landed before the strips reuse LDS
+  };
+  auto load_a = [&](int s) {
+    const long ko = 64L * kstep_of(s);
+    uint8_t* st = ring + (s & 1) * AST;
+#pragma unroll
+    for (int i = 0; i < NA; ++i) dma16(asrc[i] + ko, st + i * 1024);
+  };
+  auto pin_b = [&](auto setc) {
+    constexpr int set = decltype(setc)::value;
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        pin(ru[set][j][b]);
+        pin(rr[set][j][b]);
+      }
+  };
 
-  uint32_t* strip = reinterpret_cast<uint32_t*>(ldsA) + wave * (WM * EST);
-  if constexpr (F16) {
-    if (split > 1)
-      epilogue<2, WM>(g, strip, acc, m0 + wm * WM, n0 + wn * WN, g.P + (long)kz * M * N);
-    else
-      epilogue<1, WM>(g, strip, acc, m0 + wm * WM, n0 + wn * WN, nullptr);
-  } else {
-    epilogue<0, WM>(g, strip, acc, m0 + wm * WM, n0 + wn * WN, nullptr);
+  v16i acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = v16i{};
+
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  load_b(I0{}, 0);
+  load_a(0);
+  load_b(I1{}, 1);
+  int s = 0;
+  auto step = [&](auto setc, auto setlc) {
+    constexpr int set = decltype(setc)::value;
+    lgkm0();  // the previous step's fragment reads, before its stage is loaded again
+    load_a(s + 1);
+    load_b(setlc, s + 2);
+    vmwait<NA + 2 * NB>();  // A(s), B(s) landed; B(s+1), A(s+1), B(s+2) in flight
+    pin_b(setc);
+    v4i fb[2][FN];
+    uint32_t rmax = 0;
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        rmax = max(rmax, rr[set][j][b] & 0x7FFFu);
+        fb[b][j] = requant_half(ru[set][j][b], rr[set][j][b], mlo, mhi);
+      }
+    if (__builtin_amdgcn_ballot_w64(rmax >= 0x4BF8u)) {  // some |8 r| >= 127.5, infinite or NaN: the clamped form
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          fb[b][j] = __builtin_bit_cast(v4i, requant_words_i8(ru[set][j][b].x, ru[set][j][b].y,
+                                                              h2f((uint16_t)rr[set][j][b])));
+    }
+    const uint8_t* st = ring + (s & 1) * AST;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const v4i fa = *reinterpret_cast<const v4i*>(st + lds_off(32 * i + frow, 2 * b + h));
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb[b][j], acc[i][j], 0, 0, 0);
+      }
+    ++s;
+  };
+  while (s + 2 < ns) {
+    step(I0{}, I2{});
+    step(I1{}, I0{});
+    step(I2{}, I1{});
+  }
+  if (s < ns) step(I0{}, I2{});
+  if (s < ns) step(I1{}, I0{});
+  vmwait<0>();
+  pin_b(I0{});
+  pin_b(I1{});
+  pin_b(I2{});
+  __syncthreads();  // every wave's loads landed and fragments read before the sums take the LDS
+
+  int* const sum = reinterpret_cast<int*>(lds);
+  for (int i = tid; i < BM * OST; i += 64 * NW) sum[i] = 0;
+  __syncthreads();
+  if (ns > 0) {
+    const int rh = 4 * h;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        int e[16];
+        __builtin_memcpy(e, &acc[i][j], sizeof(e));  // (see store_tile_strip)
+        int* p = sum + (32 * i + rh) * OST + 32 * j + frow;
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          __hip_atomic_fetch_add(p + (8 * (v >> 2) + (v & 3)) * OST, e[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+  }
+  __syncthreads();
+
+  // epilogue: 4 columns per thread, as epilogue<0>
+  constexpr int TPR = BN / 4, RPP = 64 * NW / TPR;  // threads per row, rows per pass
+  const int n = n0 + 4 * (tid % TPR);
+  float swv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (g.Y) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int ne = min(n + e, N - 1);
+      swv[e] = g.sw_f16 ? h2f(reinterpret_cast<const uint16_t*>(g.sw)[ne]) : reinterpret_cast<const float*>(g.sw)[ne];
+    }
+  }
+#pragma unroll
+  for (int it = 0; it < BM / RPP; ++it) {
+    const int row = it * RPP + tid / TPR, m = m0 + row;
+    if (m >= M) break;
+    int c[4];
+    __builtin_memcpy(c, sum + row * OST + 4 * (tid % TPR), sizeof(c));
+    const long o = (long)m * N + n;
+    const bool vec = n + 3 < N && (o & 3) == 0;
+    if (g.C) {
+      if (vec) {
+        *reinterpret_cast<v4i*>(g.C + o) = v4i{c[0], c[1], c[2], c[3]};
+      } else {
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) g.C[o + e] = c[e];
+      }
+    }
+    if (g.Y) {
+      const float sam = g.sa[m];
+      uint16_t hv[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) hv[e] = f2h_after_f32(__fmul_rn(__fmul_rn((float)c[e], sam), swv[e]));
+      if (vec) {
+        *reinterpret_cast<ushort4*>(g.Y + o) = make_ushort4(hv[0], hv[1], hv[2], hv[3]);
+      } else {
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) g.Y[o + e] = hv[e];
+      }
+    }
   }
 }
 
@@ -1667,7 +1684,7 @@ __global__ void __launch_bounds__(256) quant_act_kernel(const void* __restrict__
 
 // W4A8's int8 weights computed once: unit u (row n, block b) of the
 // panel-64 words -> W8[n][32 b .. 32 b + 31] = the bytes requant_words_i8
-// gives for that unit (the values w4_kernel forms on the fly, per M-tile).
+// gives for that unit (the values w4a8_kernel forms on the fly, per M-tile).
 __global__ void __launch_bounds__(256) w4a8_weights_kernel(const uint4* __restrict__ wq,
                                                            const uint16_t* __restrict__ ratio, int N, int K,
                                                            int8_t* __restrict__ W8) {
@@ -1726,9 +1743,17 @@ static void launch_w4p(const GemmArgs& g, int split, hipStream_t st) {
   else hipLaunchKernelGGL((w4p_kernel<BM, false, KG>), grid, dim3(256 * KG), 0, st, g, split);
 }
 
-template <int OP, int BM>
-static void launch_w4(const GemmArgs& g, int split, hipStream_t st) {
-  hipLaunchKernelGGL((w4_kernel<OP, BM>), dim3(tiles(g.M, g.N, BM), split), dim3(256), 0, st, g, split);
+// W4A8 tile: the largest of 128 x 64, 128 x 32, 64 x 64, 64 x 32 (64-row tiles
+// alone up to 64 rows) whose grid gives at least W4A8_MIN_WGS workgroups,
+// else 64 x 32: one 128-row workgroup fills a CU, and a smaller tile repeats
+// the requantization (fewer rows) or the loads of A (fewer columns).
+constexpr int W4A8_MIN_WGS = 192;
+template <int BM, int BN>
+static bool launch_w4a8(const GemmArgs& g, bool force, hipStream_t st) {
+  const long wgs = (long)ceil_div(g.M, BM) * ceil_div(g.N, BN);
+  if (!force && wgs < W4A8_MIN_WGS) return false;
+  hipLaunchKernelGGL((w4a8_kernel<BM, BN>), dim3((unsigned)wgs), dim3(64 * W4A8_WAVES), 0, st, g);
+  return true;
 }
 
 size_t w4a16_partials_bytes(int M, int N, int K) {
@@ -1916,10 +1941,11 @@ int q4_gemm_w4a8(const int8_t* A, const uint32_t* wq, const uint16_t* ratio, con
   Q4_ARG(((uintptr_t)A & 15) == 0 && ((uintptr_t)wq & 15) == 0, "A and wq must be 16-byte aligned");
   Q4_ARG((((uintptr_t)Y | (uintptr_t)C) & 15) == 0, "Y and C must be 16-byte aligned (vector stores)");
   GemmArgs g{A, wq, ratio, sa, sw, sw_dtype == Q4_DT_F16, Y, C, nullptr, M, N, K};
-  // 128-row tiles only: with 256 rows the requant register ring does not fit
-  // without spills, and a spill of a register whose load is still in flight
-  // would store it before the data arrives
-  launch_w4<OP_W4A8, 128>(g, 1, as_stream(stream));
+  const hipStream_t st = as_stream(stream);
+  const bool tall = M > 64;
+  if (!(tall && launch_w4a8<128, 64>(g, false, st)) && !(tall && launch_w4a8<128, 32>(g, false, st)) &&
+      !launch_w4a8<64, 64>(g, false, st))
+    launch_w4a8<64, 32>(g, true, st);
   Q4_LAUNCHED("gemm_w4a8");
   return Q4_OK;
 }

@@ -307,6 +307,35 @@ def test_w4a8_weights_once_then_w8a8_bit_identical(gpu, N, K):
     assert torch.equal(C4, C8) and torch.equal(Y4, Y8)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64),          # one k-step: seven waves without work
+                                   (17, 31, 448),       # seven k-steps, one row tile, partial columns
+                                   (64, 12300, 576),    # 64 x 64 tiles, nine k-steps
+                                   (65, 12300, 512),    # 128 x 64 tiles, a 63-row pad
+                                   (129, 6200, 1088),   # 128 x 64 tiles, one row in the second row tile
+                                   (100, 6200, 1600),   # 128 x 32 tiles, four rounds of the ring
+                                   (300, 520, 3840)])   # 64 x 32 tiles
+@pytest.mark.parametrize("ratios", ["plain", "any bits"])
+def test_w4a8_tiles_any_ratio(gpu, M, N, K, ratios):
+    """Every W4A8 tile, partial tiles and wave shares of the k-steps, against
+    the weights formed once and the W8A8 product on them, bit for bit; with
+    ratios of any fp16 bits (clamped, negative, infinite, NaN) too."""
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    rows = -(-N // 64) * 64
+    wq = torch.randint(-2 ** 31, 2 ** 31 - 1, (rows * K // 8,), dtype=torch.int32, device="cuda", generator=gen)
+    if ratios == "plain":
+        r = torch.rand(rows * K // 32, device="cuda", generator=gen).mul_(15.9).half()
+    else:
+        r = torch.randint(-2 ** 15, 2 ** 15 - 1, (rows * K // 32,), dtype=torch.int16, device="cuda",
+                          generator=gen).view(torch.float16)
+    A = torch.randint(-127, 128, (M, K), dtype=torch.int8, device="cuda", generator=gen)
+    sa = torch.rand(M, device="cuda", generator=gen) + 0.5
+    sw = torch.rand(N, device="cuda", generator=gen) * 1e-4
+    Y4, C4 = gpu.gemm_w4a8(A, wq, r, sa, sw, N, want_c=True)
+    Y8, C8 = gpu.gemm_w8a8(A, gpu.w4a8_weights(wq, r, N, K), sa, sw, want_c=True)
+    assert torch.equal(C4, C8) and torch.equal(Y4, Y8)
+    assert torch.equal(gpu.gemm_w4a8(A, wq, r, sa, sw, N), Y4)
+
+
 # ----------------------------------------------------------------- W4A16
 @pytest.mark.parametrize("M,N,K", [(64, 256, 32), (100, 320, 96), (40, 300, 224), (128, 3840, 15360),
                                    (512, 15360, 3840), (512, 3840, 15360), (1024, 8192, 256), (2048, 8192, 96),
