@@ -890,6 +890,20 @@ static GemvFns pick(int R, int U, int xt, int st, int yt) {
     default: return pick_u<8>(U, xt, st, yt);
   }
 }
+// Groups of 4 rows (single launches only, see unsplit_rows())
+template <int XT, int ST, int YT>
+static gemv_fn pick4_u(int U) {
+  return U == 2 ? gemv_kernel<4, 2, XT, ST, YT> : U == 4 ? gemv_kernel<4, 4, XT, ST, YT> : gemv_kernel<4, 8, XT, ST, YT>;
+}
+template <int XT>
+static gemv_fn pick4_x(int U, int st, int yt) {
+  if (st == Q4_SCALE_E4M3)
+    return yt == Q4_DT_F16 ? pick4_u<XT, Q4_SCALE_E4M3, Q4_DT_F16>(U) : pick4_u<XT, Q4_SCALE_E4M3, Q4_DT_F32>(U);
+  return yt == Q4_DT_F16 ? pick4_u<XT, Q4_SCALE_F16, Q4_DT_F16>(U) : pick4_u<XT, Q4_SCALE_F16, Q4_DT_F32>(U);
+}
+static gemv_fn pick4(int U, int xt, int st, int yt) {
+  return xt == Q4_DT_F16 ? pick4_x<Q4_DT_F16>(U, st, yt) : pick4_x<Q4_DT_F32>(U, st, yt);
+}
 
 typedef void (*gemv_nx_fn)(const NormIn, const uint4*, const void*, float, void*, int, int, int, int, int, int);
 typedef void (*gemv_batch_nx_fn)(const NormIn, int, const GemvSegs, int);
@@ -1123,6 +1137,30 @@ static GemvPlan plan(int N, int K, int split_req, int x_dtype) {
   return p;
 }
 
+// Rows per workgroup of an automatic split-K plan run unsplit instead, 0
+// where the split stays. A matrix of few rows whose whole x fits the staging
+// (the plan split it to fill the chip, not because it had to) takes groups
+// of 4 rows up to one workgroup per CU (1024 rows), else 8: with 4 rows, 64
+// block slots per workgroup, so a lane has 2 blocks at K = 3840 and 8 at
+// 15360, all requested at once, and no partials, ticket or cross-workgroup
+// fence is left. Per launch in a graph, split-K / 8 rows / 4 rows, fp32 x:
+// 512 x 3840 10.4 / 4.0 / 3.5 us, 1024 x 15360 12.7 / 8.5 / 7.2, 1856 x 15360
+// 27.8 / 8.7 / 9.9; fp16 x: 512 x 3840 10.4 / 3.7 / 3.6, 1856 x 15360 29.0 /
+// 6.3 / 8.3 (16 rows are slower throughout).
+// The split queries still name the split (an explicit split runs as asked).
+static int unsplit_rows(const GemvPlan& pl, int split_req, int NP, int nblk, int x_dtype) {
+  if (split_req > 0 || pl.split == 1 || nblk > GEMV_LDS_MAX / x_block_bytes(x_dtype)) return 0;
+  if (tune_value(Q4_TUNE_GEMV_ROWS) >= 0 || tune_value(Q4_TUNE_GEMV_BAL) >= 0) return 0;
+  return NP / 4 <= 256 ? 4 : 8;
+}
+// All of a lane's blocks in flight at once, up to 8
+static int unsplit_units(int nblk, int R) {
+  const int v = tune_value(Q4_TUNE_GEMV_UNITS);
+  if (v == 4 || v == 8) return v;
+  const int per_lane = ceil_div(nblk, (64 / R) * GEMV_WAVES);
+  return per_lane <= 2 && R == 4 ? 2 : per_lane <= 4 ? 4 : 8;
+}
+
 }  // namespace q4
 
 using namespace q4;
@@ -1221,6 +1259,14 @@ static int gemv_launch(const void* x, int x_dtype, const uint32_t* wq, const voi
   }
   Q4_ARG(pl.ws == 0 || (ws && ws_size >= pl.ws), "GEMV N=%d K=%d split=%d needs a %zu-byte workspace (got %zu)", N,
          K, pl.split, pl.ws, ws ? ws_size : (size_t)0);
+  if (const int R = nx ? 0 : unsplit_rows(pl, split, pad_rows(N), K / BLK, x_dtype)) {
+    pl.R = R;
+    pl.split = 1;
+    pl.nb_max = K / BLK;
+    pl.U = unsplit_units(pl.nb_max, R);
+    pl.lds = x_stage_lds(pl.nb_max, x_dtype, R);
+    pl.ws = 0;
+  }
   // row groups: NP / R of the plan, at most one per row (pair, when gated)
   const int unit = gated ? 2 : 1;
   int groups = pad_rows(N) / pl.R;
@@ -1250,7 +1296,7 @@ static int gemv_launch(const void* x, int x_dtype, const uint32_t* wq, const voi
     Q4_LAUNCHED("gemv_normadd");
     return Q4_OK;
   }
-  gemv_fn fn = pick(pl.R, pl.U, x_dtype, scale_fmt, y_dtype).one;
+  gemv_fn fn = pl.R == 4 ? pick4(pl.U, x_dtype, scale_fmt, y_dtype) : pick(pl.R, pl.U, x_dtype, scale_fmt, y_dtype).one;
   hipLaunchKernelGGL(fn, dim3(groups / hv, pl.split), dim3(GEMV_THREADS * hv), pl.lds * hv, as_stream(stream), x,
                      reinterpret_cast<const uint4*>(wq), scales, outscale, y, N, K / BLK, pl.split, part, cnt, gated, gq,
                      gr);
@@ -1545,11 +1591,13 @@ int q4_gemv_noalloc(const void* x, int x_dtype, const uint32_t* wq, const void* 
   Q4_ARG(groups <= GEMV_MAX_TICKETS, "split-K GEMV supports at most %d row groups", GEMV_MAX_TICKETS);
   void* ws = nullptr;
   if (int e = scratch_addr(&ws)) return e;
-  // the tickets of this call's row groups start at zero (a fill kernel, not a
-  // memset node, so the call can be captured in a graph)
-  hipLaunchKernelGGL(zero_words_kernel, dim3(ceil_div(groups, 256)), dim3(256), 0, as_stream(stream),
-                     reinterpret_cast<uint32_t*>(ws), groups);
-  Q4_LAUNCHED("zero_words");
+  if (!unsplit_rows(pl, split, pad_rows(N), K / BLK, x_dtype)) {
+    // the tickets of this call's row groups start at zero (a fill kernel, not a
+    // memset node, so the call can be captured in a graph)
+    hipLaunchKernelGGL(zero_words_kernel, dim3(ceil_div(groups, 256)), dim3(256), 0, as_stream(stream),
+                       reinterpret_cast<uint32_t*>(ws), groups);
+    Q4_LAUNCHED("zero_words");
+  }
   return gemv_launch(x, x_dtype, wq, scales, scale_fmt, inv, y, y_dtype, N, K, split, ws, GEMV_SCRATCH_BYTES, stream,
                      0);
 }

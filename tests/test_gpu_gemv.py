@@ -368,3 +368,33 @@ def test_gemv_paired_row_groups_bit_identical(gpu, N, K, rows, tune):
     assert O.normwise_rel_err(to_np(outs["1"][2]), O.gemv_ref(q2, s2, x)) <= TOL_F32
     ref_act = D.gelumul_ref(O.gemv_ref(q, s, x), O.gemv_ref(q2, s2, x))
     assert O.normwise_rel_err(to_np(outs["1"][3]).astype(np.float64), ref_act) <= 5e-5
+
+
+# ------------------------------------------------- few rows, the whole K in one workgroup
+@pytest.mark.parametrize("N", [2, 62, 66, 512, 1916])
+@pytest.mark.parametrize("K", [1024, 2080, 4128, 8192, 16384, 16416, 32768])
+def test_gemv_few_rows(gpu, N, K):
+    """Automatic plans of matrices with few rows: 4-row groups with 1 to 16
+    blocks per lane, at and around the counts where the units in flight and
+    (K = 16384 / 16416, fp32 x) the longest staged x change; fp16 and fp32
+    x, both scale formats, gated pairs, and the same bits without a caller's
+    workspace."""
+    rng = np.random.default_rng(N + K)
+    q, s, x = _case(rng, N, K)
+    wq, sc = upload_int4(q, s)
+    sc8, inv = gpu.scales_e4m3(torch.from_numpy(s).cuda(), N, K)
+    e8, _, _ = O.e4m3_lift(s)
+    s8 = O.e4m3_decode(e8).astype(np.float32)
+    for xin in (x, x.astype(np.float32)):
+        xt = torch.from_numpy(xin).cuda()
+        y = gpu.gemv(xt, wq, sc, N, K, y_dtype=torch.float32)
+        assert O.normwise_rel_err(to_np(y), O.gemv_ref(q, s, xin)) <= TOL_F32
+        y8 = gpu.gemv(xt, wq, sc8, N, K, scale_fmt=gpu.SCALE_E4M3, inv=inv, y_dtype=torch.float32)
+        assert O.normwise_rel_err(to_np(y8), O.gemv_ref(q, s8, xin, inv)) <= TOL_F32
+        yh = gpu.gemv(xt, wq, sc, N, K, y_dtype=torch.float16)
+        assert torch.equal(yh, y.half())
+        act = gpu.gemv_gated(xt, wq, sc, N, K, act_dtype=torch.float32)
+        g, u = y[0::2].double(), y[1::2].double()
+        ref = 0.5 * g * (1 + torch.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3))) * u
+        # fp32 gelu of the same y: 1 + tanh cancels for negative gates, so its error is absolute, a few 2^-24 of |g u|
+        assert bool(((act.double() - ref).abs() <= 1e-6 * (g * u).abs() + 1e-30).all())
