@@ -78,6 +78,7 @@ SIGNATURES = {
     "q4_gemm_w4a8": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _vp]),
     "q4_w8_packed_bytes": (_sz, [_i, _i]),
     "q4_w8_pack": (_i, [_vp, _i, _i, _vp, _vp]),
+    "q4_w8_fold_packed": (_i, [_vp, _vp, _i, _i, _vp, _vp, _vp, _vp]),
     "q4_gemm_w8a8_packed": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _vp]),
     "q4_gemm_w8a8_packed_stamped": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _vp, _sz, _vp]),
     "q4_gemm_w8a8_packed_workgroups": (_sz, [_i, _i, _i]),

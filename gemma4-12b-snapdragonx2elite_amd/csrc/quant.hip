@@ -11,53 +11,103 @@
 namespace q4 {
 
 // ---- int4 block quantizer (src/vk_engine.py:126-131) ---------------------
-// One thread per (row, block) unit, lanes along rows, so the panel-64 unit
-// and scale stores of a wave are contiguous.
-__global__ void quantize_kernel(const float* __restrict__ W, int N, int K, int nblk,
-                                uint4* __restrict__ wq, uint16_t* __restrict__ sc16,
-                                float* __restrict__ sc32) {
-  long u = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long units = (long)pad_rows(N) * nblk;
-  if (u >= units) return;
-  int r = (int)(u % PANEL);
-  long pb = u / PANEL;
-  int b = (int)(pb % nblk);
-  int n = (int)(pb / nblk) * PANEL + r;
-  if (n >= N) {  // padded row: code 8 (= weight 0), scale 0
-    wq[u] = make_uint4(0x88888888u, 0x88888888u, 0x88888888u, 0x88888888u);
-    sc16[u] = 0;
-    return;
-  }
-  const float4* src = reinterpret_cast<const float4*>(W + (long)n * K + (long)b * BLK);
-  float v[BLK];
+// A workgroup quantizes 64 rows (one panel) x 8 blocks; each wave takes 16
+// rows, one row's 8 blocks (1 KB) per load, all 16 loads requested before the
+// first is used: lane l holds 4 consecutive elements of block l / 8, the
+// block's maximum is an 8-lane reduction, and lane pairs join their nibbles
+// to device words. Units and fp16 scales go through LDS to the panel order
+// (64 rows of a block contiguous), fp32 scales are stored from the lanes.
+// Bound by the read of W: 15360 x 3840 (236 MB in, 41 MB out) 72.6 -> 59.6 us
+// against a thread per block, whose 16-byte loads of a wave lay 64 rows apart.
+// The code is rint(v / sc) of the correctly rounded quotient; v times the
+// approximate reciprocal differs from it by less than 2e-6 (|v / sc| <= 7,
+// three roundings and the 1-ulp reciprocal), so only values that close to a
+// rounding tie, or not finite, take the division.
+constexpr int QB = 8;   // blocks per workgroup tile
+__global__ void __launch_bounds__(256) quantize_kernel(const float* __restrict__ W, int N, int K, int nblk,
+                                                       uint4* __restrict__ wq, uint16_t* __restrict__ sc16,
+                                                       float* __restrict__ sc32) {
+  constexpr int RW = 16;  // rows per wave
+  __shared__ __attribute__((aligned(16))) uint32_t words[PANEL][QB * 4 + 4];
+  __shared__ uint16_t scs[QB][PANEL];
+  const int ct = ceil_div(nblk, QB);
+  const int p = blockIdx.x / ct, b0 = (blockIdx.x % ct) * QB;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lb = lane >> 3;
+  const int b = b0 + lb;
+  const bool bok = b < nblk;
+  float4 v[RW];
 #pragma unroll
-  for (int i = 0; i < BLK / 4; ++i) {
-    float4 t = src[i];
-    v[4 * i + 0] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+  for (int i = 0; i < RW; ++i) {
+    const int n = p * PANEL + wave * RW + i;
+    v[i] = bok && n < N ? *reinterpret_cast<const float4*>(W + (long)n * K + (long)b0 * BLK + 4 * lane)
+                        : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   }
-  float amax = 0.0f;
+  // nibble shifts of this lane's elements e = 4 (lane & 1) + c of its word
+  const int odd = lane & 1;
 #pragma unroll
-  for (int i = 0; i < BLK; ++i) amax = fmaxf(amax, fabsf(v[i]));
-  const float sc = fmaxf(__fdiv_rn(amax, 7.0f), 1e-8f);
-  uint32_t w[4] = {0u, 0u, 0u, 0u};
+  for (int i = 0; i < RW; ++i) {
+    const int r = wave * RW + i, n = p * PANEL + r;
+    const float x[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+    const float amax = reduce8<true>(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
+    const float sc = fmaxf(__fdiv_rn(amax, 7.0f), 1e-8f);
+    const float inv = __builtin_amdgcn_rcpf(sc);
+    float c[4];
+    bool near = false;
 #pragma unroll
-  for (int k = 0; k < BLK; ++k) {
-    float c = rintf(__fdiv_rn(v[k], sc)) + 8.0f;
-    c = fminf(fmaxf(c, 0.0f), 15.0f);
-    w[k >> 3] |= ((uint32_t)c & 15u) << (4 * nib_pos(k & 7));
+    for (int e = 0; e < 4; ++e) {
+      const float t = x[e] * inv;
+      c[e] = rintf(t);
+      near |= !(fabsf(t - c[e]) < 0.499996f);
+    }
+    if (near) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) c[e] = rintf(__fdiv_rn(x[e], sc));
+    }
+    uint32_t w = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      w |= ((uint32_t)fminf(fmaxf(c[e] + 8.0f, 0.0f), 15.0f) & 15u) << (4 * nib_pos(e));
+    w <<= 8 * odd;   // elements 4..7 sit two nibbles above 0..3
+    w |= __float_as_uint(dpp_f<DPP_XOR1>(__uint_as_float(w)));
+    const bool live = n < N;
+    if (!odd) words[r][lane >> 1] = live ? w : 0x88888888u;   // padded row: code 8 (= weight 0), scale 0
+    if ((lane & 7) == 0) {
+      scs[lb][r] = live ? f2h_after_f32(sc) : (uint16_t)0;
+      if (sc32 && live && bok) sc32[(long)n * nblk + b] = sc;
+    }
   }
-  wq[u] = make_uint4(w[0], w[1], w[2], w[3]);
-  sc16[u] = f2h_after_f32(sc);
-  if (sc32) sc32[(long)n * nblk + b] = sc;
+  __syncthreads();
+#pragma unroll
+  for (int bb = wave; bb < QB; bb += 4) {
+    if (b0 + bb >= nblk) break;
+    const long u = ((long)p * nblk + b0 + bb) * PANEL + lane;
+    wq[u] = *reinterpret_cast<const uint4*>(&words[lane][4 * bb]);
+    sc16[u] = scs[bb][lane];
+  }
 }
 
 // ---- e4m3 scale lift (src/vk_engine.py:133-137) ---------------------------
-__global__ void absmax_bits_kernel(const float* __restrict__ x, long n, uint32_t* __restrict__ out) {
+__global__ void zero_word_kernel(uint32_t* __restrict__ p) { *p = 0u; }
+
+// One atomic per workgroup and 256 workgroups of 1024 threads: atomics on one
+// address are served one after the other, and one per wave of 4096 waves was
+// most of the kernel's time (7.4 MB: 49.2 -> 5.3 us).
+__global__ void __launch_bounds__(1024) absmax_bits_kernel(const float* __restrict__ x, long n,
+                                                           uint32_t* __restrict__ out) {
+  __shared__ float red[16];
   float m = 0.0f;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-    m = fmaxf(m, fabsf(x[i]));
+  const long stride = (long)gridDim.x * 1024;
+  long i = (long)blockIdx.x * 1024 + threadIdx.x;
+  for (; i + 3 * stride < n; i += 4 * stride)  // four independent loads in flight
+    m = fmaxf(m, fmaxf(fmaxf(fabsf(x[i]), fabsf(x[i + stride])), fmaxf(fabsf(x[i + 2 * stride]), fabsf(x[i + 3 * stride]))));
+  for (; i < n; i += stride) m = fmaxf(m, fabsf(x[i]));
   m = reduce64<true>(m);
-  if ((threadIdx.x & 63) == 0) atomicMax(out, __float_as_uint(m));  // m >= 0: bit order == value order
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    m = reduce16<true>(red[threadIdx.x & 15]);
+    if (threadIdx.x == 0) atomicMax(out, __float_as_uint(m));  // m >= 0: bit order == value order
+  }
 }
 
 // float32 in [0, 448] -> e4m3fn byte, round-half-to-even. Normal band:
@@ -80,73 +130,143 @@ __device__ inline int lift_shift(const uint32_t* maxbits) {
   return e - 1;
 }
 
-__global__ void e4m3_lift_kernel(const float* __restrict__ sc32, int N, int nblk, const uint32_t* __restrict__ maxbits,
-                                 uint8_t* __restrict__ sc8, float* __restrict__ inv_out) {
-  long u = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long units = (long)pad_rows(N) * nblk;
+// A workgroup lifts 64 rows (one panel) x 32 blocks: rows are read along the
+// blocks (128 bytes per row) and stored in panel order through LDS (15360 x
+// 120 scales: 11.5 -> 4.2 us against lanes along the rows).
+__global__ void __launch_bounds__(256) e4m3_lift_kernel(const float* __restrict__ sc32, int N, int nblk,
+                                                        const uint32_t* __restrict__ maxbits,
+                                                        uint8_t* __restrict__ sc8, float* __restrict__ inv_out) {
+  constexpr int TB = 32;
+  __shared__ __attribute__((aligned(4))) uint8_t out[TB][PANEL + 4];
+  const int ct = ceil_div(nblk, TB);
+  const int p = blockIdx.x / ct, b0 = (blockIdx.x % ct) * TB;
+  const int c = threadIdx.x & (TB - 1), r0 = threadIdx.x / TB;
+  float x[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int n = p * PANEL + 8 * i + r0;
+    x[i] = n < N && b0 + c < nblk ? sc32[(long)n * nblk + b0 + c] : 0.0f;  // padded rows: scale 0
+  }
   const int shift = lift_shift(maxbits);
-  if (u == 0 && inv_out) *inv_out = ldexpf(1.0f, -shift);
-  if (u >= units) return;
-  int r = (int)(u % PANEL);
-  long pb = u / PANEL;
-  int b = (int)(pb % nblk);
-  int n = (int)(pb / nblk) * PANEL + r;
-  if (n >= N) { sc8[u] = 0; return; }
+  if (blockIdx.x == 0 && threadIdx.x == 0 && inv_out) *inv_out = ldexpf(1.0f, -shift);
   const float p2 = __int_as_float((shift + 127) << 23);  // 2^shift, exact
-  float v = __fmul_rn(sc32[(long)n * nblk + b], p2);
-  v = fminf(fmaxf(v, 0.0f), 448.0f);
-  sc8[u] = (uint8_t)e4m3_encode_pos(v);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int n = p * PANEL + 8 * i + r0;
+    const float v = fminf(fmaxf(__fmul_rn(x[i], p2), 0.0f), 448.0f);
+    out[c][8 * i + r0] = n < N ? (uint8_t)e4m3_encode_pos(v) : (uint8_t)0;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < TB * 16; i += 256) {
+    const int bb = i >> 4, w = i & 15;
+    if (b0 + bb < nblk)
+      *reinterpret_cast<uint32_t*>(sc8 + ((long)p * nblk + b0 + bb) * PANEL + 4 * w) =
+          *reinterpret_cast<const uint32_t*>(&out[bb][4 * w]);
+  }
 }
 
 // ---- W8A8 fold (src/vk_engine.py:152-157) --------------------------------
-// One workgroup per weight row.
-__device__ inline void unit_codes(uint4 unit, float* qm8) {
-  uint32_t w[4] = {unit.x, unit.y, unit.z, unit.w};
-#pragma unroll
-  for (int k = 0; k < BLK; ++k) qm8[k] = (float)(int)((w[k >> 3] >> (4 * nib_pos(k & 7))) & 15u) - 8.0f;
+// A workgroup folds 8 rows: thread (r = t % 8, block t / 8 + 32 i), so the 8
+// rows of a block are one 128-byte line of units, read by one workgroup (a
+// workgroup per row fetched every line into the L2 of all 8 XCDs). The row
+// maximum needs only the block's largest |code| (products round
+// monotonically). The 32 quotients of a block take 9 values: k s for k = 0..8
+// with either sign, so a thread rounds 8 quotients, packs the 16 codes' bytes
+// into 4 words and looks the codes up with byte permutes. W8 is row-major
+// [N][K] or, PACKED, the layout of the packed W8A8 GEMM (1 KB per 32 rows x
+// 32 k: 16-byte chunk l is row l % 32, k half l / 32; rows padded to 32 and
+// K to 128 with zeros), which saves the pass that packs it.
+// 15360 x 3840: 59.6 us for the row-major fold and 18.3 for its packing
+// before, 24.1 us in one pass (96 MB).
+__device__ inline uint32_t fold_byte(float v) {
+  return (uint32_t)(int)fminf(fmaxf(v, -127.0f), 127.0f) & 0xFFu;
+}
+// bytes of the 4 codes in the low nibbles of c's bytes; t: the 16 codes' bytes
+__device__ inline uint32_t fold_lookup(uint32_t c, const uint32_t (&t)[4]) {
+  const uint32_t lo = __builtin_amdgcn_perm(t[1], t[0], c & 0x07070707u);
+  const uint32_t hi = __builtin_amdgcn_perm(t[3], t[2], c & 0x07070707u);
+  return __builtin_amdgcn_perm(hi, lo, ((c >> 1) & 0x04040404u) | 0x03020100u);  // byte i of hi where bit 3 is set
 }
 
+template <bool PACKED>
 __global__ void __launch_bounds__(256) w8_fold_kernel(const uint4* __restrict__ wq, const float* __restrict__ sc32,
                                                       int N, int K, int nblk, int8_t* __restrict__ W8,
-                                                      float* __restrict__ sw32, uint16_t* __restrict__ sw16) {
-  __shared__ float red[4];
-  const int n = blockIdx.x;
+                                                      float* __restrict__ sw32, uint16_t* __restrict__ sw16,
+                                                      int kslices) {
+  constexpr int FR = 8, FB = 256 / FR;
+  __shared__ float red[4][FR];
+  const int r = threadIdx.x & (FR - 1), n = blockIdx.x * FR + r, bt = threadIdx.x / FR;
+  const bool live = n < N;
+  const long u0 = panel_index(n < N ? n : N - 1, 0, nblk);
+  const float* srow = sc32 + (long)(live ? n : N - 1) * nblk;
   float amax = 0.0f;
-  for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-    float q[BLK];
-    unit_codes(wq[panel_index(n, b, nblk)], q);
-    const float s = sc32[(long)n * nblk + b];
+  for (int b = bt; b < nblk; b += FB) {
+    const uint4 w = wq[u0 + (long)b * PANEL];
+    const float s = srow[b];
+    typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+    v2us mx = {8, 8}, mn = {8, 8};  // the block's largest and smallest code (and 8 = weight 0)
 #pragma unroll
-    for (int k = 0; k < BLK; ++k) amax = fmaxf(amax, fabsf(__fmul_rn(q[k], s)));
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t wi = i == 0 ? w.x : i == 1 ? w.y : i == 2 ? w.z : w.w;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const v2us c = __builtin_bit_cast(v2us, (wi >> (4 * k)) & 0x000F000Fu);
+        mx = __builtin_elementwise_max(mx, c);
+        mn = __builtin_elementwise_min(mn, c);
+      }
+    }
+    const int far = max(max((int)mx.x, (int)mx.y) - 8, 8 - min((int)mn.x, (int)mn.y));
+    amax = fmaxf(amax, fabsf(__fmul_rn((float)far, s)));
   }
-  amax = reduce64<true>(amax);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
+  amax = slot_reduce<8, true>(amax);
+  if ((threadIdx.x & 63) < FR) red[threadIdx.x >> 6][r] = amax;
   __syncthreads();
-  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  amax = fmaxf(fmaxf(red[0][r], red[1][r]), fmaxf(red[2][r], red[3][r]));
   const float sw = fmaxf(__fdiv_rn(amax, 127.0f), 1e-12f);
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < FR && live) {
     if (sw32) sw32[n] = sw;
     if (sw16) sw16[n] = f2h_after_f32(sw);
   }
-  for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-    float q[BLK];
-    unit_codes(wq[panel_index(n, b, nblk)], q);
-    const float s = sc32[(long)n * nblk + b];
-    uint32_t o[8];
+  if (!PACKED && !live) return;
+  const int nb_out = PACKED ? kslices : nblk;
+  for (int b = bt; b < nb_out; b += FB) {
+    uint32_t o[8] = {};
+    if (live && b < nblk) {
+      const uint4 wv = wq[u0 + (long)b * PANEL];
+      const float s = srow[b];
+      uint32_t t[4];
+      uint32_t pos[9], neg[9];
+      pos[0] = fold_byte(__fmul_rn(0.0f, s));  // 0, or -127 for a scale that is not finite
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      uint32_t word = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float v = rintf(__fdiv_rn(__fmul_rn(q[4 * j + e], s), sw));
-        v = fminf(fmaxf(v, -127.0f), 127.0f);
-        word |= ((uint32_t)(int)v & 0xFFu) << (8 * e);
+      for (int k = 1; k <= 8; ++k) {
+        const float v = rintf(__fdiv_rn(__fmul_rn((float)k, s), sw));
+        pos[k] = fold_byte(v);
+        neg[k] = fold_byte(-v);
       }
-      o[j] = word;
+      t[0] = neg[8] | (neg[7] << 8) | (neg[6] << 16) | (neg[5] << 24);
+      t[1] = neg[4] | (neg[3] << 8) | (neg[2] << 16) | (neg[1] << 24);
+      t[2] = pos[0] | (pos[1] << 8) | (pos[2] << 16) | (pos[3] << 24);
+      t[3] = pos[4] | (pos[5] << 8) | (pos[6] << 16) | (pos[7] << 24);
+      const uint32_t w[4] = {wv.x, wv.y, wv.z, wv.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        // low nibbles hold elements 0, 4, 1, 5 and high nibbles 2, 6, 3, 7 of the word
+        const uint32_t lo = fold_lookup(w[i] & 0x0F0F0F0Fu, t), hi = fold_lookup((w[i] >> 4) & 0x0F0F0F0Fu, t);
+        o[2 * i] = __builtin_amdgcn_perm(hi, lo, 0x06040200u);
+        o[2 * i + 1] = __builtin_amdgcn_perm(hi, lo, 0x07050301u);
+      }
     }
-    uint4* dst = reinterpret_cast<uint4*>(W8 + (long)n * K + (long)b * BLK);
+    uint4* dst;
+    long half;
+    if constexpr (PACKED) {
+      dst = reinterpret_cast<uint4*>(W8 + ((long)(n >> 5) * kslices + b) * 1024) + (n & 31);
+      half = 32;
+    } else {
+      dst = reinterpret_cast<uint4*>(W8 + (long)n * K + (long)b * BLK);
+      half = 1;
+    }
     dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
-    dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
+    dst[half] = make_uint4(o[4], o[5], o[6], o[7]);
   }
 }
 
@@ -255,8 +375,9 @@ int q4_quantize(const float* W, int N, int K, uint32_t* wq, uint16_t* sc16, floa
   Q4_ARG(W && wq && sc16, "null pointer");
   Q4_ARG(((uintptr_t)W & 15) == 0 && ((uintptr_t)wq & 15) == 0, "W and wq must be 16-byte aligned");
   const int nblk = K / BLK;
-  long units = (long)pad_rows(N) * nblk;
-  hipLaunchKernelGGL(quantize_kernel, dim3(ceil_div(units, 256)), dim3(256), 0, as_stream(stream), W, N, K, nblk,
+  const long wgs = (long)(pad_rows(N) / PANEL) * ceil_div(nblk, QB);
+  Q4_ARG(wgs < (1L << 31), "matrix too large");
+  hipLaunchKernelGGL(quantize_kernel, dim3((unsigned)wgs), dim3(256), 0, as_stream(stream), W, N, K, nblk,
                      reinterpret_cast<uint4*>(wq), sc16, sc32);
   Q4_LAUNCHED("quantize");
   return Q4_OK;
@@ -268,14 +389,14 @@ int q4_scales_e4m3(const float* sc32, int N, int K, uint8_t* sc8, float* inv_dev
   Q4_ARG(sc32 && sc8 && work, "null pointer");
   const int nblk = K / BLK;
   long n = (long)N * nblk;
-  Q4_HIP(hipMemsetAsync(work, 0, sizeof(uint32_t), as_stream(stream)));
-  int grid = ceil_div(n, 256);
-  if (grid > 1024) grid = 1024;
-  hipLaunchKernelGGL(absmax_bits_kernel, dim3(grid), dim3(256), 0, as_stream(stream), sc32, n, work);
+  hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(1), 0, as_stream(stream), work);
+  Q4_LAUNCHED("zero_word");
+  const long grid = min((n + 4095) / 4096, 256L);
+  hipLaunchKernelGGL(absmax_bits_kernel, dim3((unsigned)grid), dim3(1024), 0, as_stream(stream), sc32, n, work);
   Q4_LAUNCHED("absmax_bits");
-  long units = (long)pad_rows(N) * nblk;
-  hipLaunchKernelGGL(e4m3_lift_kernel, dim3(ceil_div(units, 256)), dim3(256), 0, as_stream(stream), sc32, N, nblk,
-                     work, sc8, inv_dev);
+  const long wgs = (long)(pad_rows(N) / PANEL) * ceil_div(nblk, 32);
+  hipLaunchKernelGGL(e4m3_lift_kernel, dim3((unsigned)wgs), dim3(256), 0, as_stream(stream), sc32, N, nblk, work, sc8,
+                     inv_dev);
   Q4_LAUNCHED("e4m3_lift");
   return Q4_OK;
 }
@@ -286,9 +407,23 @@ int q4_w8_fold(const uint32_t* wq, const float* sc32, int N, int K, int8_t* W8, 
   if (int st = check_wk(N, K)) return st;
   Q4_ARG(wq && sc32 && W8, "null pointer");
   Q4_ARG(((uintptr_t)W8 & 15) == 0 && ((uintptr_t)wq & 15) == 0, "W8 and wq must be 16-byte aligned");
-  hipLaunchKernelGGL(w8_fold_kernel, dim3(N), dim3(256), 0, as_stream(stream), reinterpret_cast<const uint4*>(wq),
-                     sc32, N, K, K / BLK, W8, sw32, sw16);
+  hipLaunchKernelGGL(w8_fold_kernel<false>, dim3(ceil_div(N, 8)), dim3(256), 0, as_stream(stream),
+                     reinterpret_cast<const uint4*>(wq), sc32, N, K, K / BLK, W8, sw32, sw16, 0);
   Q4_LAUNCHED("w8_fold");
+  return Q4_OK;
+}
+
+int q4_w8_fold_packed(const uint32_t* wq, const float* sc32, int N, int K, int8_t* W8p, float* sw32, uint16_t* sw16,
+                      void* stream) {
+  clear_error();
+  if (int st = check_wk(N, K)) return st;
+  Q4_ARG(wq && sc32 && W8p, "null pointer");
+  Q4_ARG(((uintptr_t)W8p & 15) == 0 && ((uintptr_t)wq & 15) == 0, "W8p and wq must be 16-byte aligned");
+  const int rows = ceil_div(N, 32) * 32;
+  const int kslices = (int)(q4_w8_packed_bytes(N, K) / ((size_t)rows * 32));
+  hipLaunchKernelGGL(w8_fold_kernel<true>, dim3(rows / 8), dim3(256), 0, as_stream(stream),
+                     reinterpret_cast<const uint4*>(wq), sc32, N, K, K / BLK, W8p, sw32, sw16, kslices);
+  Q4_LAUNCHED("w8_fold_packed");
   return Q4_OK;
 }
 

@@ -118,6 +118,15 @@ def w8_fold(wq: torch.Tensor, sc32: torch.Tensor, N: int, K: int):
     return W8, sw32, sw16
 
 
+def w8_fold_packed(wq: torch.Tensor, sc32: torch.Tensor, N: int, K: int):
+    """:func:`w8_fold` with the int8 weights in :func:`w8_pack`'s layout, in one pass."""
+    W8p = torch.empty(int(lib().q4_w8_packed_bytes(N, K)), dtype=torch.int8, device=wq.device)
+    sw32 = torch.empty(N, dtype=torch.float32, device=wq.device)
+    sw16 = torch.empty(N, dtype=torch.float16, device=wq.device)
+    call("q4_w8_fold_packed", _p(wq), _p(sc32.contiguous()), N, K, _p(W8p), _p(sw32), _p(sw16), _stream())
+    return W8p, sw32, sw16
+
+
 def w4a8_ratio(sc32: torch.Tensor, sw32: torch.Tensor, N: int, K: int) -> torch.Tensor:
     _, se = dev_sizes(N, K)
     ratio = torch.empty(se, dtype=torch.float16, device=sc32.device)

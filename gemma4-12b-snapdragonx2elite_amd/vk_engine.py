@@ -120,17 +120,16 @@ def quant(W, pf: bool = True, fp8: bool | None = None, prefill_i8: bool | None =
     inv = 1.0
     bs16 = Buf(tensor=sc16)
     bs = bs16
-    if fp8:
+    w8 = sw8 = None
+    if prefill_i8 and pf:
+        # int8 weights kept in the packed layout the W8A8 kernel reads (the
+        # reference keeps Wi8T [K, N], src/vk_engine.py:155)
+        W8p, _sw32, sw16 = ops.w8_fold_packed(wq, sc32, N, K)
+        w8, sw8 = Buf(tensor=W8p), Buf(tensor=sw16)
+    if fp8:   # last: it waits for the GPU to read inv
         sc8, inv = ops.scales_e4m3(sc32, N, K)
         bs = Buf(tensor=sc8)
     split = ops.auto_split(N, K)
-    w8 = sw8 = None
-    if prefill_i8 and pf:
-        W8, _sw32, sw16 = ops.w8_fold(wq, sc32, N, K)
-        # int8 weights kept in the packed layout the W8A8 kernel reads (the
-        # reference keeps Wi8T [K, N], src/vk_engine.py:155)
-        w8, sw8 = Buf(tensor=ops.w8_pack(W8)), Buf(tensor=sw16)
-        del W8
     return QW(Buf(tensor=wq), bs, split, nblk, float(inv), bs16, w8, sw8)
 
 

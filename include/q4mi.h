@@ -353,6 +353,10 @@ int q4_gemm_w8a8(const int8_t* A, const int8_t* W8, const float* sa,
  * vk/coopgemm_w8a8.comp:18-37 (weights as folded at src/vk_engine.py:152-157). */
 size_t q4_w8_packed_bytes(int N, int K);
 int q4_w8_pack(const int8_t* W8, int N, int K, int8_t* W8p, void* stream);
+/* q4_w8_fold with W8 in that layout (the bytes of q4_w8_fold then
+ * q4_w8_pack), in one pass; W8p: q4_w8_packed_bytes(N, K) bytes. */
+int q4_w8_fold_packed(const uint32_t* wq, const float* sc32, int N, int K,
+                      int8_t* W8p, float* sw32, uint16_t* sw16, void* stream);
 int q4_gemm_w8a8_packed(const int8_t* A, const int8_t* W8p, const float* sa,
                         const void* sw, int sw_dtype, uint16_t* Y,
                         int32_t* C, int M, int N, int K, void* stream);

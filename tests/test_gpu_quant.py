@@ -92,3 +92,38 @@ def test_casts_bit_exact(gpu):
     assert (to_np(h).view(np.uint16) == x.astype(np.float16).view(np.uint16)).all()
     back = gpu.cast_f16_f32(h)
     assert (to_np(back) == x.astype(np.float16).astype(np.float32)).all()
+
+
+@pytest.mark.parametrize("N,K", [(1, 32), (63, 96), (64, 256), (65, 288), (200, 2080), (300, 15360)])
+@pytest.mark.parametrize("kind", ["weights", "ties", "special"])
+def test_quantizer_and_fold_edges_bit_exact(gpu, N, K, kind):
+    """Partial panels, block tiles and fold passes; values on and next to the
+    rounding ties of the codes; blocks of zeros, denormal and huge values.
+    Codes, scales and the folded weights equal numpy's bit for bit, and the
+    one-pass packed fold equals fold then pack."""
+    rng = np.random.default_rng(N + K)
+    W = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    if kind == "ties":   # multiples of half a code step, moved by up to 3 ulp
+        sc = np.maximum(np.abs(W.reshape(N, -1, 32)).max(2) / np.float32(7), np.float32(1e-8))
+        t = (rng.integers(-14, 15, (N, K // 32, 32)) / 2).astype(np.float32)
+        t[:, :, 0] = 7.0
+        W = (t * sc[:, :, None]).astype(np.float32).reshape(N, K)
+        W = (W.view(np.int32) + rng.integers(-3, 4, (N, K)) * (W != 0)).astype(np.int32).view(np.float32)
+    elif kind == "special":
+        W[:, :32] = 0.0
+        W[0, -1] = 3e38
+        W[-1, :16] = 1e-39
+    q, sc = O.quant_codes(W)
+    wq, sc16, sc32 = gpu.quantize(torch.from_numpy(W).cuda())
+    assert (to_np(wq).view(np.uint32).reshape(-1) == O.pack_dev(q).view(np.uint32).reshape(-1)).all()
+    assert (to_np(sc32).view(np.uint32) == sc.view(np.uint32)).all()
+    assert (to_np(sc16).view(np.uint16).reshape(-1) == O.scales_dev(sc.astype(np.float16)).view(np.uint16).reshape(-1)).all()
+    W8, sw = O.w8_fold(q, sc)
+    gW8, gsw32, gsw16 = gpu.w8_fold(wq, sc32, N, K)
+    assert (to_np(gW8) == W8).all() and (to_np(gsw32).view(np.uint32) == sw.view(np.uint32)).all()
+    pW8, psw32, psw16 = gpu.w8_fold_packed(wq, sc32, N, K)
+    assert torch.equal(pW8, gpu.w8_pack(gW8)) and torch.equal(psw32, gsw32) and torch.equal(psw16, gsw16)
+    sc8, inv = gpu.scales_e4m3(sc32, N, K)
+    e8, inv_ref, _ = O.e4m3_lift(sc)
+    assert inv == inv_ref
+    assert (to_np(sc8).reshape(-1) == O.scales_dev(e8).view(np.uint8).reshape(-1)).all()
