@@ -61,6 +61,7 @@ struct GemmArgs {
   float* P;             // W4A16 split-K: fp32 partials [split][M][N]
   int M, N, K;
   unsigned long long* stamps;  // stamped W8A8 only: 4 words per workgroup
+  int gated;            // W4A16: Y [M][N / 2] = gelu(even columns) * odd columns
 };
 
 // LDS byte offset of 16-byte chunk c (0..3) of staged 64-byte row r. The XOR
@@ -144,11 +145,18 @@ __device__ inline void tile_of(int w, int G, int ntm, int& tm, int& tn) {
 
 constexpr int EST = 68;  // epilogue strip row stride (words): 64 columns + 4 to stagger banks
 
+// The activation of a gate/up pair: gelu(f16(g)) f16(u), the separate gate and
+// up GEMMs' fp16 outputs through gelumul_kernel (vk/gelumul.comp:7-8).
+__device__ inline uint16_t gated_f16(float g, float u) {
+  return f2h(__fmul_rn(gelu_tanh(h2f(f2h(g))), h2f(f2h(u))));
+}
+
 // Epilogue: the wave's WM x (32 FN) accumulator block goes through a
 // 64-column LDS strip per 64 columns (so each stored row segment is a full 128-byte line of
 // f16 Y) and is stored row-contiguously, 4 columns per lane. MODE 0: int32
 // accumulators -> Y = f16((f32(C) * sa) * sw) and/or C; MODE 1: fp32 -> f16
-// Y; MODE 2: fp32 -> fp32 partials P.
+// Y; MODE 2: fp32 -> fp32 partials P; MODE 3: fp32 gate/up column pairs ->
+// f16 activations [M][N / 2] (gated_f16).
 template <int MODE, int WM, int FN = 4, class acc_t>
 __device__ inline void epilogue(const GemmArgs& g, uint32_t* strip, const acc_t (&acc)[WM / 32][FN], int mw, int nw,
                                 float* P) {
@@ -196,7 +204,17 @@ __device__ inline void epilogue(const GemmArgs& g, uint32_t* strip, const acc_t 
       if (m < M) {
         const long o = (long)m * N + n;
         const bool vec = n + 3 < N && (o & 3) == 0;
-        if constexpr (MODE == 2) {
+        if constexpr (MODE == 3) {  // N is even, so a pair starts inside N or not at all
+          const long og = (long)m * (N / 2) + n / 2;
+          const uint16_t a = gated_f16(__builtin_bit_cast(float, qv[0]), __builtin_bit_cast(float, qv[1]));
+          const uint16_t b = gated_f16(__builtin_bit_cast(float, qv[2]), __builtin_bit_cast(float, qv[3]));
+          if (n + 3 < N && (og & 1) == 0) {
+            *reinterpret_cast<uint32_t*>(g.Y + og) = a | ((uint32_t)b << 16);
+          } else {
+            if (n < N) g.Y[og] = a;
+            if (n + 2 < N) g.Y[og + 1] = b;
+          }
+        } else if constexpr (MODE == 2) {
           if (vec) {
             *reinterpret_cast<v4u*>(P + o) = q;
           } else {
@@ -1094,29 +1112,34 @@ __global__ void __launch_bounds__(256) w8q_kernel(const GemmArgs g) {
 // paired): for an odd count the second group runs one k-step fewer and
 // then joins the first group's last barrier without any MFMA, so no
 // operand is multiplied that a one-group launch would not multiply (a
-// surplus step on zero scales would turn an Inf in X into NaN). Group 1
-// then hands its accumulators to group 0 through LDS, and group 0 adds them
-// (acc0 + acc1) and runs the epilogue.
-template <int BM, bool TAIL, int KG = 1>
-__global__ void __launch_bounds__(256 * KG) w4p_kernel(const GemmArgs g, int split) {
-  constexpr int S = 4, FM = BM / 32, FN = 2;
+// surplus step on zero scales would turn an Inf in X into NaN). The groups
+// then exchange halves of their accumulators through LDS, add them (acc0 +
+// acc1) and each runs the epilogue of its half.
+// NWV = 2 (with KG = 2) narrows the tile to 128 columns: two waves per group,
+// four per workgroup, the same k-loop per wave with each A row loaded by half
+// as many waves (twice the loads of A). A short grid then needs half the
+// splits to fill the chip, so half the fp32 partials are written and read
+// again: see w4a16_plan.
+template <int BM, bool TAIL, int KG = 1, int NWV = 4>
+__global__ void __launch_bounds__(64 * NWV * KG) w4p_kernel(const GemmArgs g, int split) {
+  constexpr int S = 4, FM = BM / 32, FN = 2, BN = 64 * NWV;
   constexpr int AST = BM * 128;      // bytes per A stage
-  constexpr int NA = BM / 32;        // A direct loads per wave per k-step
+  constexpr int NA = BM / 8 / NWV;   // A direct loads per wave per k-step
   constexpr int NB = FN * 2 * 2;     // B loads per lane per k-step: n-tile x block x (half-unit, scale)
-  constexpr int EPI = 4 * 64 * EST * 4;
+  constexpr int EPI = KG * NWV * 64 * EST * 4;
   constexpr int RING = KG * S * AST;
-  constexpr int XCH = KG > 1 ? 4 * FM * FN * 16 * 64 * 4 : 0;  // group 1's accumulators
+  constexpr int XCH = KG > 1 ? NWV * FM * FN * 16 * 64 * 4 : 0;  // half of each group's accumulators
   constexpr int LDSB = RING > EPI ? (RING > XCH ? RING : XCH) : (EPI > XCH ? EPI : XCH);
   static_assert(KG == 1 || (KG == 2 && BM == 128), "two k-groups at 128-row tiles");
   __shared__ __attribute__((aligned(16))) uint8_t ldsA[LDSB];
 
   // grp through readfirstlane: wave-uniform, so the group's k range stays in SGPRs
-  const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3,
-            grp = KG > 1 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
+  const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % NWV,
+            grp = KG > 1 ? __builtin_amdgcn_readfirstlane(tid / (64 * NWV)) : 0;
   const int M = g.M, N = g.N, K = g.K;
   int tm, tn;
   tile_of(blockIdx.x, gridDim.x, (M + BM - 1) / BM, tm, tn);
-  const int m0 = tm * BM, n0 = tn * 256;
+  const int m0 = tm * BM, n0 = tn * BN;
   const int nblk = K / BLK;
   const int nk_all = (nblk + 1) / 2;
   const int kz = blockIdx.y;
@@ -1305,46 +1328,71 @@ __global__ void __launch_bounds__(256 * KG) w4p_kernel(const GemmArgs g, int spl
       }
   __syncthreads();  // every direct load landed and every fragment read before the strips reuse LDS
 
+  // With two k-groups, group q finishes m-tiles [q FM / 2, (q + 1) FM / 2):
+  // each hands its accumulators of the other half over through LDS (16-byte
+  // piece c of tile (i, j) of wave w, lane l, at float ((((q NWV + w) FM / 2 +
+  // i) FN + j) 4 + c) 64 + l) 4) and adds acc0 + acc1, so both halves of the
+  // workgroup convert and store (one group doing it all took 6 us of M 512, N
+  // 15360: 57.7 -> 56.7 us; M 1024 113.4 -> 110.3).
+  constexpr int FH = FM / KG;  // m-tiles this wave finishes
+  v16f out[KG > 1 ? FH : 1][FN];
   if constexpr (KG > 1) {
-    // group 1's accumulators to group 0: tile (i, j) of wave w, 16-byte piece
-    // c, lane l at float ((((w * FM + i) * FN + j) * 4 + c) * 64 + l) * 4
     float* xch = reinterpret_cast<float*>(ldsA);
-    if (grp) {
+    auto piece = [&](int q, int i, int j, int c) {
+      return xch + ((((q * NWV + wave) * FH + i) * FN + j) * 4 + c) * 256 + lane * 4;
+    };
+    auto hand_over = [&](auto qc) {  // to group q, its m-tiles
+      constexpr int q = decltype(qc)::value;
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < FH; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
-            const v4f t = {acc[i][j][4 * c], acc[i][j][4 * c + 1], acc[i][j][4 * c + 2], acc[i][j][4 * c + 3]};
-            *reinterpret_cast<v4f*>(xch + ((((wave * FM + i) * FN + j) * 4 + c) * 64 + lane) * 4) = t;
+            const v16f& t = acc[q * FH + i][j];
+            *reinterpret_cast<v4f*>(piece(q, i, j, c)) = v4f{t[4 * c], t[4 * c + 1], t[4 * c + 2], t[4 * c + 3]};
           }
-    }
+    };
+    auto take = [&](auto qc) {
+      constexpr int q = decltype(qc)::value;
+#pragma unroll
+      for (int i = 0; i < FH; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const v4f t = *reinterpret_cast<const v4f*>(piece(q, i, j, c));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[i][j][4 * c + e] = acc[q * FH + i][j][4 * c + e] + t[e];
+          }
+    };
+    if (grp) hand_over(I0{});
+    else hand_over(I1{});
     __syncthreads();
-    if (!grp) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const v4f t = *reinterpret_cast<const v4f*>(xch + ((((wave * FM + i) * FN + j) * 4 + c) * 64 + lane) * 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[i][j][4 * c + e] += t[e];
-          }
-    }
+    if (grp) take(I1{});
+    else take(I0{});
     __syncthreads();  // the exchange is read before the strips reuse LDS
-    if (grp) return;
   }
+  auto fin = [&](int i, int j) -> const v16f& {
+    if constexpr (KG > 1) return out[i][j];
+    else return acc[i][j];
+  };
 
-  uint32_t* strip = reinterpret_cast<uint32_t*>(ldsA) + wave * (64 * EST);
+  uint32_t* strip = reinterpret_cast<uint32_t*>(ldsA) + (grp * NWV + wave) * (64 * EST);
+  const int mw = m0 + grp * (BM / KG), nw = n0 + 64 * wave;
 #pragma unroll
-  for (int c = 0; c < FM / 2; ++c) {
-    const v16f sub[2][FN] = {{acc[2 * c][0], acc[2 * c][1]}, {acc[2 * c + 1][0], acc[2 * c + 1][1]}};
-    if (g.P)  // split-K partials (also at split 1 for the gated entry point)
-      epilogue<2, 64, FN>(g, strip, sub, m0 + 64 * c, n0 + 64 * wave, g.P + (long)kz * M * N);
+  for (int c = 0; c < FH / 2; ++c) {
+    const v16f sub[2][FN] = {{fin(2 * c, 0), fin(2 * c, 1)}, {fin(2 * c + 1, 0), fin(2 * c + 1, 1)}};
+    if constexpr (KG > 1) {
+      if (g.gated) {
+        epilogue<3, 64, FN>(g, strip, sub, mw + 64 * c, nw, nullptr);
+        continue;
+      }
+    }
+    if (g.P)  // split-K partials
+      epilogue<2, 64, FN>(g, strip, sub, mw + 64 * c, nw, g.P + (long)kz * M * N);
     else
-      epilogue<1, 64, FN>(g, strip, sub, m0 + 64 * c, n0 + 64 * wave, nullptr);
+      epilogue<1, 64, FN>(g, strip, sub, mw + 64 * c, nw, nullptr);
   }
 }
 
@@ -1416,20 +1464,21 @@ __global__ void __launch_bounds__(64 * W4A8_WAVES) w4a8_kernel(const GemmArgs g)
   const int h = lane >> 5, frow = lane & 31;
   uint8_t* const ring = lds + wave * (2 * AST);
 
-  const uint8_t* asrc[NA];
+  // Wave-uniform bases (the tile's first A row, its panel) plus 32-bit lane
+  // offsets inside the tile: a load costs no vector address arithmetic
+  const uint8_t* const Ab = reinterpret_cast<const uint8_t*>(g.A) + (long)m0 * K;
+  uint32_t aoff[NA];
 #pragma unroll
   for (int i = 0; i < NA; ++i) {
     const int r = 16 * i + (lane >> 2);
-    asrc[i] = reinterpret_cast<const uint8_t*>(g.A) + (long)min(m0 + r, M - 1) * K + (((lane & 3) ^ swz(r)) << 4);
+    aoff[i] = (uint32_t)min(r, M - 1 - m0) * (uint32_t)K + (((lane & 3) ^ swz(r)) << 4);
   }
-  const uint8_t* bsrc[FN];
-  const uint8_t* rsrc[FN];
+  const long up = panel_index(n0 & ~(PANEL - 1), 0, nblk);
+  const uint8_t* const Bb = reinterpret_cast<const uint8_t*>(g.B) + up * 16;
+  const uint8_t* const Rb = reinterpret_cast<const uint8_t*>(g.bsc) + up * 2;
+  uint32_t bo[FN];  // the lane's row of each n-tile within the panel
 #pragma unroll
-  for (int j = 0; j < FN; ++j) {
-    const long u = panel_index(min(n0 + 32 * j + frow, N - 1), 0, nblk);
-    bsrc[j] = reinterpret_cast<const uint8_t*>(g.B) + u * 16 + 8 * h;
-    rsrc[j] = reinterpret_cast<const uint8_t*>(g.bsc) + u * 2;
-  }
+  for (int j = 0; j < FN; ++j) bo[j] = (uint32_t)min(n0 + 32 * j + frow, N - 1) & (PANEL - 1);
   uint32_t mlo = 0x64006400u, mhi = 0x54005400u;  // requant_pair's VGPR operands
   asm volatile("" : "+v"(mlo), "+v"(mhi));
 
@@ -1445,15 +1494,15 @@ __global__ void __launch_bounds__(64 * W4A8_WAVES) w4a8_kernel(const GemmArgs g)
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        ru[set][j][b] = ld8(bsrc[j] + (blk + b) * (PANEL * 16));
-        rr[set][j][b] = ld2(rsrc[j] + (blk + b) * (PANEL * 2));
+        ru[set][j][b] = ld8_so(Bb + (blk + b) * (PANEL * 16), bo[j] * 16 + 8 * h);
+        rr[set][j][b] = ld2_so(Rb + (blk + b) * (PANEL * 2), bo[j] * 2);
       }
   };
   auto load_a = [&](int s) {
     const long ko = 64L * kstep_of(s);
     uint8_t* st = ring + (s & 1) * AST;
 #pragma unroll
-    for (int i = 0; i < NA; ++i) dma16(asrc[i] + ko, st + i * 1024);
+    for (int i = 0; i < NA; ++i) dma16_so(Ab + ko, aoff[i], st + i * 1024);
   };
   auto pin_b = [&](auto setc) {
     constexpr int set = decltype(setc)::value;
@@ -1608,8 +1657,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restr
 
 // Gate/up rows interleaved (row 2i gate i, 2i + 1 up i): Y[o] = f16(gelu(g)
 // u) with g = f16(sum over splits of P[s][2o]), u = f16(... P[s][2o + 1]),
-// split order: the separate gate and up GEMMs' fp16 outputs through
-// gelumul_kernel (vk/gelumul.comp:7-8), bit for bit at the same split. An
+// split order: bit for bit the separate GEMMs' results at the same split. An
 // output row m holds P columns m N .. + N, so output o reads partial 2o. 4
 // outputs per thread.
 __global__ void __launch_bounds__(256) splitk_reduce_gated_kernel(const float* __restrict__ P,
@@ -1617,16 +1665,14 @@ __global__ void __launch_bounds__(256) splitk_reduce_gated_kernel(const float* _
   const long o = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
   if (o >= n) return;
   const long np = 2 * n;  // partials per split
-  auto act = [](float g, float u) {
-    return f2h(__fmul_rn(gelu_tanh(h2f(f2h(g))), h2f(f2h(u))));
-  };
   if (o + 3 < n && (np & 3) == 0) {  // 16-byte loads need 16-byte split strides
     v4f a = *reinterpret_cast<const v4f*>(P + 2 * o), b = *reinterpret_cast<const v4f*>(P + 2 * o + 4);
     for (int s = 1; s < split; ++s) {
       a += *reinterpret_cast<const v4f*>(P + (long)s * np + 2 * o);
       b += *reinterpret_cast<const v4f*>(P + (long)s * np + 2 * o + 4);
     }
-    *reinterpret_cast<ushort4*>(Y + o) = make_ushort4(act(a.x, a.y), act(a.z, a.w), act(b.x, b.y), act(b.z, b.w));
+    *reinterpret_cast<ushort4*>(Y + o) = make_ushort4(gated_f16(a.x, a.y), gated_f16(a.z, a.w), gated_f16(b.x, b.y),
+                                                             gated_f16(b.z, b.w));
   } else {
     for (long e = o; e < min(o + 4, n); ++e) {
       float gs = P[2 * e], us = P[2 * e + 1];
@@ -1634,7 +1680,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_gated_kernel(const float* _
         gs += P[(long)s * np + 2 * e];
         us += P[(long)s * np + 2 * e + 1];
       }
-      Y[e] = act(gs, us);
+      Y[e] = gated_f16(gs, us);
     }
   }
 }
@@ -1736,11 +1782,45 @@ static int w4a16_kgroups(int M, int N, int K, int split) {
   return kg;
 }
 
-template <int BM, int KG = 1>
+// Launch plan of a W4A16 GEMM. `narrow`: two k-groups of two waves on 128 x
+// 128 tiles, taken where the wide plan would split K at one group: the groups
+// take the place of half the splits, each with at least W4A16_NARROW_KSTEPS
+// k-steps. The k-loop is the same per wave (~1600 cycles per k-step at the
+// 1.7 to 2.1 GHz the chip holds under it); the gain is in the partials, which
+// the GEMM writes and the next kernel reads at HBM speed. Per GEMM with its
+// reduction at M 128, wide / narrow: N 30720, K 3840 45.7 / 40.2 us, 8192 x 3840
+// 23.5 / 20.4, 3840 x 4096 20.8 / 18.7, 3840 x 15360 31.1 / 28.6; M 256, 15360 x
+// 3840 42.7 / 36.7; the gated gate/up GEMM (30720 x 3840) leaves no partials
+// and no second kernel (36.8 + 6.8 -> 41.0 us in a kernel trace).
+// Never more splits than the wide plan, whose partials size the workspace.
+struct W4Plan {
+  int split, bm, kg;
+  bool narrow;
+};
+constexpr int W4A16_NARROW_KSTEPS = 8;
+static W4Plan w4a16_plan(int M, int N, int K) {
+  W4Plan p{w4a16_split(M, N, K), pick_bm(M, N), 1, false};
+  p.kg = w4a16_kgroups(M, N, K, p.split);
+  const bool tuned = tune_value(Q4_TUNE_W4A16_SPLIT) >= 0 || tune_value(Q4_TUNE_W4A16_KG) >= 0;
+  if (!tuned && p.bm == 128 && p.kg == 1 && p.split > 1) {
+    const int nk = (K / 32 + 1) / 2, t = ceil_div(M, 128) * ceil_div(N, 128);
+    const int s = min(ceil_div(240, t), nk / (2 * W4A16_NARROW_KSTEPS));
+    if (s >= 1 && s < p.split) p = W4Plan{s, 128, 2, true};
+  }
+  return p;
+}
+
+template <int BM, int KG, int NWV>
 static void launch_w4p(const GemmArgs& g, int split, hipStream_t st) {
-  const dim3 grid(tiles(g.M, g.N, BM), split);
-  if (g.K % 64) hipLaunchKernelGGL((w4p_kernel<BM, true, KG>), grid, dim3(256 * KG), 0, st, g, split);
-  else hipLaunchKernelGGL((w4p_kernel<BM, false, KG>), grid, dim3(256 * KG), 0, st, g, split);
+  const dim3 grid(ceil_div(g.M, BM) * ceil_div(g.N, 64 * NWV), split), blk(64 * NWV * KG);
+  if (g.K % 64) hipLaunchKernelGGL((w4p_kernel<BM, true, KG, NWV>), grid, blk, 0, st, g, split);
+  else hipLaunchKernelGGL((w4p_kernel<BM, false, KG, NWV>), grid, blk, 0, st, g, split);
+}
+static void launch_w4a16(const GemmArgs& g, const W4Plan& p, hipStream_t st) {
+  if (p.narrow) launch_w4p<128, 2, 2>(g, p.split, st);
+  else if (p.bm == 256) launch_w4p<256, 1, 4>(g, p.split, st);
+  else if (p.kg == 2) launch_w4p<128, 2, 4>(g, p.split, st);
+  else launch_w4p<128, 1, 4>(g, p.split, st);
 }
 
 // W4A8 tile: the largest of 128 x 64, 128 x 32, 64 x 64, 64 x 32 (64-row tiles
@@ -1762,26 +1842,27 @@ size_t w4a16_partials_bytes(int M, int N, int K) {
 }
 
 int w4a16_partials(const uint16_t* X, const uint32_t* wq, const uint16_t* sc16, int M, int N, int K, void* ws,
-                   size_t ws_bytes, hipStream_t st, int* split_out) {
+                   size_t ws_bytes, hipStream_t st, int* split_out, uint16_t* gated_y) {
   Q4_ARG(M > 0 && N > 0 && K > 0 && K % 32 == 0, "bad W4A16 shape M=%d N=%d K=%d (K must be a multiple of 32)", M,
          N, K);
   Q4_ARG(X && wq && sc16 && ws, "null pointer");
   Q4_ARG(((uintptr_t)X & 15) == 0 && ((uintptr_t)wq & 15) == 0 && ((uintptr_t)ws & 15) == 0,
          "X, wq and the workspace must be 16-byte aligned");
-  const int split = w4a16_split(M, N, K);
+  const W4Plan pl = w4a16_plan(M, N, K);
   Q4_ARG(ws_bytes >= w4a16_partials_bytes(M, N, K), "W4A16 partials workspace too small: %zu < %zu bytes", ws_bytes,
          w4a16_partials_bytes(M, N, K));
   Q4_ARG(2L * M * K < (1L << 31) && (long)pad_rows(N) * (K / BLK) * 16 < (1L << 31),
          "W4A16 needs X and the int4 weights under 2 GiB (32-bit offsets)");
   GemmArgs g{X, wq, sc16, nullptr, nullptr, 0, nullptr, nullptr, reinterpret_cast<float*>(ws), M, N, K};
-  if (pick_bm(M, N) == 256)
-    launch_w4p<256>(g, split, st);
-  else if (w4a16_kgroups(M, N, K, split) == 2)
-    launch_w4p<128, 2>(g, split, st);
-  else
-    launch_w4p<128>(g, split, st);
+  const bool direct = gated_y && pl.split == 1 && pl.kg == 2;
+  if (direct) {  // one pass: the activation in the epilogue
+    g.P = nullptr;
+    g.Y = gated_y;
+    g.gated = 1;
+  }
+  launch_w4a16(g, pl, st);
   Q4_LAUNCHED("gemm_w4a16 (partials)");
-  *split_out = split;
+  *split_out = direct ? 0 : pl.split;
   return Q4_OK;
 }
 
@@ -1965,18 +2046,17 @@ int q4_gemm_w4a16_ws(const uint16_t* X, const uint32_t* wq, const uint16_t* sc16
   Q4_ARG(((uintptr_t)X & 15) == 0 && ((uintptr_t)wq & 15) == 0, "X and wq must be 16-byte aligned");
   Q4_ARG(((uintptr_t)Y & 7) == 0, "Y must be 8-byte aligned");
   Q4_ARG(!ws || ((uintptr_t)ws & 15) == 0, "workspace must be 16-byte aligned");
-  int split = w4a16_split(M, N, K);
-  if (split > 1 && (!ws || ws_bytes < (size_t)split * M * N * sizeof(float))) split = 1;  // no room: one pass
+  W4Plan pl = w4a16_plan(M, N, K);
+  // no room for the wide plan's partials: one pass (whatever this plan would need)
+  const int wide = w4a16_split(M, N, K);
+  if (pl.split > 1 && (!ws || ws_bytes < (size_t)wide * M * N * sizeof(float)))
+    pl = W4Plan{1, pick_bm(M, N), w4a16_kgroups(M, N, K, 1), false};
+  const int split = pl.split;
   GemmArgs g{X, wq, sc16, nullptr, nullptr, 0, Y, nullptr, split > 1 ? reinterpret_cast<float*>(ws) : nullptr,
              M, N, K};
   Q4_ARG(2L * M * K < (1L << 31) && (long)pad_rows(N) * (K / BLK) * 16 < (1L << 31),
          "W4A16 needs X and the int4 weights under 2 GiB (32-bit offsets)");
-  if (pick_bm(M, N) == 256)
-    launch_w4p<256>(g, split, as_stream(stream));
-  else if (w4a16_kgroups(M, N, K, split) == 2)
-    launch_w4p<128, 2>(g, split, as_stream(stream));
-  else
-    launch_w4p<128>(g, split, as_stream(stream));
+  launch_w4a16(g, pl, as_stream(stream));
   Q4_LAUNCHED("gemm_w4a16");
   if (split > 1) {
     const long n = (long)M * N;
@@ -2000,7 +2080,8 @@ int q4_gemm_w4a16_gated(const uint16_t* X, const uint32_t* wq, const uint16_t* s
   Q4_ARG(Y, "null pointer");
   Q4_ARG(((uintptr_t)Y & 7) == 0, "Y must be 8-byte aligned");
   int split = 0;
-  if (int st = w4a16_partials(X, wq, sc16, M, N, K, ws, ws_bytes, as_stream(stream), &split)) return st;
+  if (int st = w4a16_partials(X, wq, sc16, M, N, K, ws, ws_bytes, as_stream(stream), &split, Y)) return st;
+  if (split == 0) return Q4_OK;  // written by the GEMM
   const long n = (long)M * (N / 2);
   hipLaunchKernelGGL(splitk_reduce_gated_kernel, dim3(ceil_div(n, 1024)), dim3(256), 0, as_stream(stream),
                      reinterpret_cast<const float*>(ws), Y, n, split);

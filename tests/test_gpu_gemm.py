@@ -442,6 +442,40 @@ def test_w4a16_gated_equals_separate_gemms_and_gelumul(gpu, M, I, K, dev_interle
     assert np.abs(A.astype(np.float64) - act).max() <= np.abs(act).max() * 2.0 ** -9
 
 
+@pytest.mark.parametrize("M,N,K", [(100, 660, 1056),     # unsplit, 9 and 8 k-steps, the last one half a step
+                                   (37, 14, 4096),       # one partial column tile, four splits
+                                   (128, 3848, 4096),    # a last tile of 8 columns
+                                   (300, 520, 2080),     # three row tiles, two splits
+                                   (128, 30720, 3840)])  # the chunk's gate/up, unsplit
+def test_w4a16_narrow_tiles(gpu, M, N, K, tune):
+    """128-column tiles of two k-groups (the automatic plan of these shapes)
+    against the 256-column one-group plan and the oracle, plain and gated; an
+    Inf in X reaches the same outputs as there (0 * Inf: NaN), and no others."""
+    rng = np.random.default_rng(M + N + K)
+    q, s = synth_int4(rng, N, K)
+    wq, sc = upload_int4(q, s)
+    Xh = rng.standard_normal((M, K)).astype(np.float16)
+    X = torch.from_numpy(Xh).cuda()
+    Y = to_np(gpu.gemm_w4a16(X, wq, sc, N)).astype(np.float64)
+    A = to_np(gpu.gemm_w4a16_gated(X, wq, sc, N)).astype(np.float64)
+    Xh[3, K - 1] = np.inf
+    Xi = torch.from_numpy(Xh).cuda()
+    Yi = to_np(gpu.gemm_w4a16(Xi, wq, sc, N)).astype(np.float64)
+    tune("w4a16_kg", "1")
+    Y1 = to_np(gpu.gemm_w4a16(X, wq, sc, N)).astype(np.float64)
+    Yi1 = to_np(gpu.gemm_w4a16(Xi, wq, sc, N)).astype(np.float64)
+    assert np.abs(Y - Y1).max() <= np.abs(Y1).max() * 2.0 ** -9   # sums in another order, one fp16 step
+    assert (np.isnan(Yi) == np.isnan(Yi1)).all() and (np.isinf(Yi) == np.isinf(Yi1)).all()
+    assert np.isfinite(np.delete(Yi, 3, 0)).all()
+    if N <= 4096:
+        ref = O.gemm_w4a16_ref(to_np(X), q, s).astype(np.float16).astype(np.float64)
+        assert np.abs(Y - ref).max() <= np.abs(ref).max() * 2.0 ** -9
+        act = D.gelumul_ref(ref[:, 0::2], ref[:, 1::2])
+    else:
+        act = D.gelumul_ref(Y[:, 0::2], Y[:, 1::2])
+    assert np.abs(A - act).max() <= np.abs(act).max() * 2.0 ** -9
+
+
 @pytest.mark.parametrize("M,N,K,fuse_norm", [(128, 3840, 4096, True), (128, 3840, 15360, True),
                                               (100, 320, 96, False), (37, 256, 224, True), (512, 1024, 1920, True)])
 def test_w4a16_normadd_equals_gemm_then_normadd(gpu, M, N, K, fuse_norm):
