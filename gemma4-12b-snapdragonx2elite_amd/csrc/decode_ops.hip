@@ -724,26 +724,29 @@ attn_split_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, 
 }
 
 // The same split for 16 query heads of one KV head at hd 512 (the k == v
-// global layers), on fp32 matrix cores: scores and p V are 16-row products,
-// v_mfma_f32_16x16x4_f32 takes q and p as they are (fp32; K and V widened
-// from fp16 exactly), and the cache is read once for all 16 heads instead of
-// once per 4. What bounds it: the latency of one round of loads (each
-// workgroup requests its 32 K and V rows, 64 KB, before anything else), then
-// ~4,100 MFMA cycles per wave.
+// global layers), on the matrix cores: scores and p V are 16-row products and
+// the cache is read once for all 16 heads instead of once per 4. q and p stay
+// fp32 values: each is split into fp16 hi + lo parts (~22 bits) after an exact
+// power-of-two scaling (q: a head's largest element to [2^13, 2^14); p: 2^14),
+// so that both parts are normal numbers, and the two products with the fp16
+// cache are exact in the fp32 accumulators.
 //
-// Workgroup (g, sp): heads 16 g .., keys [32 sp, 32 sp + 32), 4 waves. For the
-// scores wave w takes the dims [64 w, +64) and [256 + 64 w, +64) of every
-// head and key: RoPE partners (i, i + 256) stay in one lane, and no wave
-// repeats another's q norm (only the sums of squares cross waves, through
-// LDS). Lane l holds row l % 16 (head or key) and, of each 32 dims, the 8
-// from 8 (l / 16): element e of the 8 is step e of the MFMA's k, the same
-// for both operands. The waves' partial scores meet in LDS; every wave then
-// takes the softmax of all 16 heads in the A layout of p V (lane: head
-// l % 16, keys 8 (l / 16) ..), which is a product over the wave's own 128
-// columns of V: lane column c of MFMA e is dim 8 c + e, so a lane's 16-byte
-// V load feeds 8 MFMAs and its results are 8 consecutive dims.
+// Workgroup (g, sp): heads 16 g .., keys [32 sp, 32 sp + 32), 4 waves. All
+// loads come first (37 per wave, 64 KB of K and V per workgroup): this round
+// trip bounds the kernel. Wave w norms and rotates heads 4 w .. 4 w + 3 in
+// row layout and shares their parts through LDS. For the scores it then takes
+// the dims [128 w, +128) of every head and key: lane l holds row l % 16 (head
+// or key) and, of each 32 dims, the 8 from 8 (l / 16). The waves' partial
+// scores meet in LDS; every wave takes the softmax of all 16 heads in the A
+// layout of p V (lane: head l % 16, keys 8 (l / 16) ..), a product over the
+// wave's own 128 columns of V: column c of MFMA e is dim 8 c + e, so a lane's
+// 16-byte V loads of 8 keys hold the B operands of 8 MFMAs, transposed in the
+// lane by byte permutes, and its results are 8 consecutive dims.
 // Measured at 8101 keys (256 splits, 16.6 MB of cache per layer, kernel
-// trace): 22.6 -> 14.7 us against the 4-head kernel.
+// trace): 22.6 us with the 4-head kernel, 14.7 with the same split on the
+// fp32 matrix instruction (16x16x4: 8 times the MFMA cycles, K and V widened
+// first, every lane loading the norm and RoPE rows), 12.1 us. Error against 64
+// bits with fp32 outputs, 8101 keys: 3.7e-7 (4 heads), 2.9e-7, 2.5e-7.
 template <bool PREP>
 __global__ void __launch_bounds__(256)
 attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, const float* __restrict__ cs,
@@ -751,39 +754,32 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
                      int window, int qoff, int grp, const uint32_t* __restrict__ dyn, float* __restrict__ part,
                      int nsplit, const float* __restrict__ knw, int koff, int voff) {
   constexpr int EPL = 8, HD = 512, KCH = 32, NW = 4, SST = KCH + 4;  // SST: score row stride (words)
+  constexpr int QP = HD + 8;         // q row pitch (halves): 16 rows of a 16-byte column in distinct banks
+  constexpr int HPW = ATT_MMH / NW;  // heads a wave prepares
+  constexpr float PSC = 16384.0f;    // scale of p's parts
+  __shared__ __attribute__((aligned(16))) uint16_t qs[2][ATT_MMH][QP];  // hi, lo
   __shared__ __attribute__((aligned(16))) float sc[NW][ATT_MMH][SST];
   __shared__ __attribute__((aligned(16))) uint16_t fresh[PREP ? NW : 1][2][PREP ? HD : 8];
-  __shared__ float ssq[NW][ATT_MMH];
+  __shared__ float qinv[ATT_MMH];    // inverse of each head's scale
   const int h0 = blockIdx.x * ATT_MMH, sp = blockIdx.y, t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int kvh = h0 / grp, j0 = sp * KCH;
   const long kv0 = (long)kvh * stride * HD;
   const int li = lane & 15, lg = lane >> 4;
-  // dims of score chunk c (0..3): 8 from sdim(c); chunks c and c + 2 are RoPE partners
-  auto sdim = [&](int c) { return (c >> 1) * (HD / 2) + 64 * wave + (c & 1) * 32 + 8 * lg; };
+  auto sdim = [&](int c) { return 128 * wave + 32 * c + 8 * lg; };  // the lane's 8 dims of score chunk c
 
   // (1) every load of the split, none waiting for the position
   const uint32_t pos = load_pos(dyn);
-  float q[4][8], wq[4][8], cr[4][8], sr[4][8], kr[EPL], vr[EPL], wk[EPL], crr[EPL], srr[EPL];
-  auto ld8f = [](const float* p, float(&v)[8]) {
-    const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-  };
+  float q[HPW][EPL], wq[EPL], cr[EPL], sr[EPL], kr[EPL], vr[EPL], wk[EPL];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int d = sdim(c);
-    ld8f(qkv + qoff + (long)(h0 + li) * HD + d, q[c]);
-    ld8f(qnw + d, wq[c]);
-    ld8f(cs + d, cr[c]);
-    ld8f(sn + d, sr[c]);
-  }
+  for (int i = 0; i < HPW; ++i) ld_row<EPL>(qkv + qoff + (long)(h0 + HPW * wave + i) * HD, q[i]);
+  ld_row<EPL>(qnw, wq);
+  ld_row<EPL>(cs, cr);
+  ld_row<EPL>(sn, sr);
   if constexpr (PREP) {
     ld_row<EPL>(qkv + koff + kvh * HD, kr);
     ld_row<EPL>(qkv + voff + kvh * HD, vr);
     ld_row<EPL>(knw, wk);
-    ld_row<EPL>(cs, crr);
-    ld_row<EPL>(sn, srr);
   }
   v4u ku[2][4], vv[8];
 #pragma unroll
@@ -802,19 +798,41 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
   const int slot = kv_slot(pos, window);
   const bool fresh_split = PREP && slot < stride && slot >= j0 && slot < j0 + n;  // workgroup-uniform
 
-  // (2) q norm and RoPE of this wave's dims; with the fresh slot in this
-  //     split, this token's K and V through the wave's own LDS rows
-  float s2 = 0.0f;
+  // (2) q norm and RoPE of this wave's heads, their scaled parts to LDS; with
+  //     the fresh slot in this split, this token's K and V through the wave's
+  //     own LDS rows
+  auto halves = [](const float(&v)[8], v4u& hi, v4u& lo) {
+    v8h h, l;
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+    for (int e = 0; e < 8; ++e) {
+      h[e] = (_Float16)v[e];
+      l[e] = (_Float16)(v[e] - (float)h[e]);
+    }
+    hi = __builtin_bit_cast(v4u, h);
+    lo = __builtin_bit_cast(v4u, l);
+  };
 #pragma unroll
-    for (int e = 0; e < 8; ++e) s2 = fmaf(q[c][e], q[c][e], s2);
-  s2 = slot_sum<16>(s2);
-  if (lg == 0) ssq[wave][li] = s2;
+  for (int i = 0; i < HPW; ++i) {
+    row_norm_rope<EPL>(q[i], wq, cr, sr);
+    float mx = 0.0f;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) mx = fmaxf(mx, fabsf(q[i][e]));
+    mx = reduce64<true>(mx);
+    // exponent field of the scale that takes mx to [2^13, 2^14); its inverse stays a normal number
+    const int ex = min(max(267 - (int)(__float_as_uint(mx) >> 23), 1), 253);
+    const float scale = __uint_as_float((uint32_t)ex << 23);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) q[i][e] *= scale;
+    v4u hi, lo;
+    halves(q[i], hi, lo);
+    *reinterpret_cast<v4u*>(&qs[0][HPW * wave + i][EPL * lane]) = hi;
+    *reinterpret_cast<v4u*>(&qs[1][HPW * wave + i][EPL * lane]) = lo;
+    if (lane == 0) qinv[HPW * wave + i] = __uint_as_float((uint32_t)(254 - ex) << 23);
+  }
   if constexpr (PREP) {
     if (fresh_split) {
       uint16_t kb[EPL], vb[EPL];
-      fresh_kv<EPL>(kr, vr, wk, crr, srr, kb, vb);
+      fresh_kv<EPL>(kr, vr, wk, cr, sr, kb, vb);
       v4u k4, v4;
       __builtin_memcpy(&k4, kb, 16);
       __builtin_memcpy(&v4, vb, 16);
@@ -842,27 +860,18 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
         if (8 * lg + s == kslot) vv[s] = *reinterpret_cast<const v4u*>(&fresh[wave][1][128 * wave + 8 * li]);
     }
   }
-  const float inv = inv_rms(((ssq[0][li] + ssq[1][li]) + ssq[2][li]) + ssq[3][li], HD);
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float lo = __fmul_rn(__fmul_rn(q[c][e], inv), wq[c][e]);
-      const float hi = __fmul_rn(__fmul_rn(q[c + 2][e], inv), wq[c + 2][e]);
-      q[c][e] = __fadd_rn(__fmul_rn(lo, cr[c][e]), __fmul_rn(-hi, sr[c][e]));
-      q[c + 2][e] = __fadd_rn(__fmul_rn(hi, cr[c + 2][e]), __fmul_rn(lo, sr[c + 2][e]));
-    }
 
   // (3) this wave's part of the scores: D column l % 16 = key, rows 4 (l / 16) .. = heads
-  auto half_at = [](const v4u& u, int e) { return h2f((uint16_t)(e & 1 ? u[e >> 1] >> 16 : u[e >> 1] & 0xFFFFu)); };
-  v4f d[2][2] = {};  // [key tile][chunk parity]
+  v4f d[2][2] = {};  // [key tile][part]
 #pragma unroll
   for (int c = 0; c < 4; ++c)
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
+    for (int pt = 0; pt < 2; ++pt) {
+      const v8h a = *reinterpret_cast<const v8h*>(&qs[pt][li][sdim(c)]);
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
-        d[kt][c & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[c][e], half_at(ku[kt][c], e), d[kt][c & 1], 0, 0, 0);
+        d[kt][pt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(v8h, ku[kt][c]), d[kt][pt], 0, 0, 0);
+    }
 #pragma unroll
   for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -873,6 +882,7 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
   __syncthreads();
 
   // (4) softmax over the split's keys: lane = head li, keys 8 lg .. + 7
+  const float qi = qinv[li];
   float p[8];
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
@@ -880,7 +890,7 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
 #pragma unroll
     for (int w = 1; w < NW; ++w) x += *reinterpret_cast<const v4f*>(&sc[w][li][8 * lg + 4 * b]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) p[4 * b + e] = 8 * lg + 4 * b + e < n ? x[e] : -INFINITY;
+    for (int e = 0; e < 4; ++e) p[4 * b + e] = 8 * lg + 4 * b + e < n ? x[e] * qi : -INFINITY;
   }
   float m = p[0];
 #pragma unroll
@@ -891,24 +901,35 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
   for (int s = 0; s < 8; ++s) {
     p[s] = p[s] != -INFINITY ? expf(p[s] - m) : 0.0f;
     l += p[s];
+    p[s] *= PSC;
   }
   l = slot_sum<16>(l);
 
   // (5) unnormalised p V over the wave's 128 dims. Rows past the length are
   //     taken as zero (a never-written cache row may hold a NaN).
-  v4f o[8] = {};
+  v4u ph, pl;
+  halves(p, ph, pl);
+  if (n < KCH) {
 #pragma unroll
-  for (int s = 0; s < 8; ++s)
+    for (int s = 0; s < 8; ++s)
+      if (8 * lg + s >= n) vv[s] = v4u{0u, 0u, 0u, 0u};
+  }
+  v4f o[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float v = 8 * lg + s < n ? half_at(vv[s], e) : 0.0f;
-      o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], v, o[e], 0, 0, 0);
-    }
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+    const int w = e >> 1;
+    const v4u bt = {__builtin_amdgcn_perm(vv[1][w], vv[0][w], sel), __builtin_amdgcn_perm(vv[3][w], vv[2][w], sel),
+                    __builtin_amdgcn_perm(vv[5][w], vv[4][w], sel), __builtin_amdgcn_perm(vv[7][w], vv[6][w], sel)};
+    const v8h bh = __builtin_bit_cast(v8h, bt);
+    o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, ph), bh, v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+    o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, pl), bh, o[e], 0, 0, 0);
+  }
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     float* dst = part + ((long)(h0 + 4 * lg + v) * nsplit + sp) * HD + 128 * wave + 8 * li;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) dst[e] = o[e][v];
+    for (int e = 0; e < 8; ++e) dst[e] = o[e][v] * (1.0f / PSC);
   }
   if (t < ATT_MMH) {
     float* ml = attn_ml(part, gridDim.x * ATT_MMH, nsplit, HD) + 2 * ((long)(h0 + t) * nsplit + sp);
