@@ -1568,8 +1568,10 @@ __global__ void __launch_bounds__(64 * W4A8_WAVES) w4a8_kernel(const GemmArgs g)
     step(I1{}, I0{});
     step(I2{}, I1{});
   }
-  if (s < ns) step(I0{}, I2{});
-  if (s < ns) step(I1{}, I0{});
+  if (s < ns) {
+    step(I0{}, I2{});
+    if (s < ns) step(I1{}, I0{});
+  }
   vmwait<0>();
   pin_b(I0{});
   pin_b(I1{});
