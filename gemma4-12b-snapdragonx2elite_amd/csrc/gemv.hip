@@ -597,9 +597,11 @@ gemv_multi_kernel(const uint16_t* __restrict__ X, int M, const uint4* __restrict
 // g % T, row c, block g / T of the step; 1 KB of contiguous weights per
 // wave for T = 4), and a 4 x 4 transpose of the words across the four
 // 16-lane rows (two v_permlane32_swap, two v_permlane16_swap) hands lane
-// (c, g) word g of the 4 units of its column, one per MFMA. Steps go to
+// (c, g) word g of the 4 units of its column, one per MFMA. The lane loads its
+// unit's scale too (one load where every lane loaded the four scales of its
+// column), and three permlane swaps hand all four to each lane. Steps go to
 // the waves round-robin (the 4 waves read adjacent blocks together); U
-// steps of loads stay in flight (x slices, the unit, 4 scales per step;
+// steps of loads stay in flight (x slices, the unit, its scale per step;
 // explicit wait counts as in the GEMV), and the 4 waves' partial sums meet
 // in LDS in wave order (deterministic).
 __device__ inline v8h codes_to_h8(uint32_t w) {
@@ -623,11 +625,19 @@ __device__ inline v4u transpose_rows(v4u a) {
   return v4u{q01[0], q01[1], q23[0], q23[1]};
 }
 
-// Scale bits at a uniform base + the lane's offset + OFF bytes.
-template <int ST, int OFF>
+// The value of lane (c, t), t = 0..3, in every lane (c, g).
+__device__ inline v4u share_rows(uint32_t a) {
+  const auto p = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+  const auto q = __builtin_amdgcn_permlane16_swap(p[0], p[0], false, false);
+  const auto r = __builtin_amdgcn_permlane16_swap(p[1], p[1], false, false);
+  return v4u{q[0], q[1], r[0], r[1]};
+}
+
+// Scale bits at a uniform base + the lane's offset.
+template <int ST>
 __device__ inline uint32_t mm_scale(const uint8_t* sbase, uint32_t voff) {
-  if constexpr (ST == Q4_SCALE_F16) return ld2_so_off<OFF>(sbase, voff);
-  else return ld1_so_off<OFF>(sbase, voff);
+  if constexpr (ST == Q4_SCALE_F16) return ld2_so(sbase, voff);
+  else return ld1_so(sbase, voff);
 }
 
 template <int T, int U, int ST, int YT>
@@ -635,7 +645,7 @@ __global__ void __launch_bounds__(GEMV_THREADS)
 gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict__ wq, const void* __restrict__ scv,
                float outscale, void* __restrict__ Y, int N, int nblk, int kspan, float* __restrict__ part) {
   constexpr int BPS = 4 / T;                      // blocks per step
-  constexpr int L = BPS + 1 + 4;                  // loads per step: x slices, the unit, 4 scales
+  constexpr int L = BPS + 2;                      // loads per step: x slices, the unit and its scale
   constexpr int SB = ST == Q4_SCALE_F16 ? 2 : 1;  // scale bytes
   static_assert(U * L < 64, "vmcnt range");
   __shared__ v4f red[GEMV_WAVES][T][64];
@@ -652,11 +662,10 @@ gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict_
   const uint8_t* sbase = reinterpret_cast<const uint8_t*>(scv) + (pu + (long)kb0 * PANEL) * SB;
   const uint32_t xo = (uint32_t)min(c, M - 1) * (uint32_t)(nblk * BLK * 2) + g * 16;
   const int lrow = 16 * (g % T) + c, lblk = g / T;  // the unit lane (c, g) loads: row, block within the step
-  const uint32_t so = c * SB;
   const int nsteps = (nb + BPS - 1) / BPS;
   const int rounds = ((nsteps + GEMV_WAVES - 1) / GEMV_WAVES + U - 1) / U;
   v4u xr[U][BPS], wr[U];
-  uint32_t sr[U][4];
+  uint32_t sr[U];
   auto issue = [&](int u, int s) {
     const int b0 = (wave + GEMV_WAVES * s) * BPS;  // first block of the step
     static_for<0, BPS>([&](auto ic) {
@@ -664,10 +673,7 @@ gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict_
       xr[u][i] = ld16_so(xbase + (long)min(b0 + i, nb - 1) * (BLK * 2), xo);
     });
     wr[u] = ld16_so(wbase, (uint32_t)(lrow * 16) + ((uint32_t)min(b0 + lblk, nb - 1) << 10));
-    static_for<0, 4>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      sr[u][j] = mm_scale<ST, 16 * (j % T) * SB>(sbase + (long)min(b0 + j / T, nb - 1) * (PANEL * SB), so);
-    });
+    sr[u] = mm_scale<ST>(sbase, (uint32_t)(lrow * SB) + (uint32_t)min(b0 + lblk, nb - 1) * (PANEL * SB));
   };
   v4f acc[T];
 #pragma unroll
@@ -676,6 +682,7 @@ gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict_
     const int b0 = (wave + GEMV_WAVES * s) * BPS;
     if (b0 < nb) {
       const v4u w = transpose_rows(wr[u]);
+      const v4u sv = share_rows(sr[u]);
       v4f d[4];
       static_for<0, 4>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
@@ -686,7 +693,7 @@ gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict_
       static_for<0, 4>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         if (j / T == 0 || b0 + j / T < nb) {
-          const float sc = scale_value<ST>(sr[u][j]);
+          const float sc = scale_value<ST>(sv[j]);
 #pragma unroll
           for (int r = 0; r < 4; ++r) acc[j % T][r] = fmaf(sc, d[j][r], acc[j % T][r]);
         }
@@ -703,8 +710,7 @@ gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict_
       pin(wr[u]);
 #pragma unroll
       for (int i = 0; i < BPS; ++i) pin(xr[u][i]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) pin(sr[u][j]);
+      pin(sr[u]);
       use(u, s + u);
       issue(u, s + u + U);
     });
@@ -716,8 +722,7 @@ gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict_
     pin(wr[u]);
 #pragma unroll
     for (int i = 0; i < BPS; ++i) pin(xr[u][i]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) pin(sr[u][j]);
+    pin(sr[u]);
     use(u, s + u);
   });
 #pragma unroll
@@ -1000,6 +1005,16 @@ static int mm_split(int NP, int nblk) {
   if (v >= 1 && v <= 64) s = v;
   const int span = (nblk + s - 1) / s;
   return (nblk + span - 1) / span;  // no empty split
+}
+// K splits a launch uses (mm_split sizes the workspace): the partials and the
+// reduce launch cost more than filling the chip saves up to
+// GEMV_MM_UNSPLIT_BLOCKS blocks. 8 vectors, split / unsplit, per launch in a
+// graph: 4096 x 3840 7.0 / 5.8 us, 2048 x 3840 7.0 / 5.6, 8192 x 3840 7.3 / 6.4,
+// 3840 x 4096 7.0 / 5.6, 3840 x 8192 8.6 / 8.2, 3840 x 15360 11.6 / 13.1.
+constexpr int GEMV_MM_UNSPLIT_BLOCKS = 256;
+static int mm_launch_split(int NP, int nblk) {
+  if (tune_value(Q4_TUNE_GEMV_MM_SPLIT) < 0 && nblk <= GEMV_MM_UNSPLIT_BLOCKS) return 1;
+  return mm_split(NP, nblk);
 }
 static bool mm_deep() { return tune_value(Q4_TUNE_GEMV_MM_DEEP) > 0; }
 
@@ -1389,10 +1404,9 @@ int q4_gemv_multi_ws(const void* x, int M, const uint32_t* wq, const void* scale
   const int nblk = K / BLK;
   const float outscale = scale_fmt == Q4_SCALE_E4M3 ? inv * 256.0f : 1.0f;
   const size_t need = q4_gemv_multi_workspace_bytes(M, N, K);
-  const bool split = need && ws && ws_size >= need;
-  return gemv_mm_launch(x, M, wq, scales, scale_fmt, outscale, y, y_dtype, N, nblk,
-                        split ? mm_split(pad_rows(N), nblk) : 1, split ? reinterpret_cast<float*>(ws) : nullptr,
-                        as_stream(stream));
+  const int split = need && ws && ws_size >= need ? mm_launch_split(pad_rows(N), nblk) : 1;
+  return gemv_mm_launch(x, M, wq, scales, scale_fmt, outscale, y, y_dtype, N, nblk, split,
+                        split > 1 ? reinterpret_cast<float*>(ws) : nullptr, as_stream(stream));
 }
 
 int q4_gemv_multi(const void* x, int M, const uint32_t* wq, const void* scales, int scale_fmt, float inv, void* y,

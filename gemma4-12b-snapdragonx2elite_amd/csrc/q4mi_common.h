@@ -121,26 +121,6 @@ __device__ inline v2u ld8(const void* p) {
   asm volatile("global_load_dwordx2 %0, %1, off" : "=v"(r) : "v"(p));
   return r;
 }
-// Uniform base (SGPR pair) + per-lane 32-bit byte offset + immediate byte
-// offset OFF (-4096 .. 4095), streaming (read-once data).
-template <int OFF>
-__device__ inline uint32_t ld4_so_nt(const void* sbase, uint32_t voff) {
-  uint32_t r;
-  asm volatile("global_load_dword %0, %1, %2 offset:%3 nt" : "=v"(r) : "v"(voff), "s"(sbase), "n"(OFF));
-  return r;
-}
-template <int OFF>
-__device__ inline uint32_t ld2_so_off(const void* sbase, uint32_t voff) {
-  uint32_t r;
-  asm volatile("global_load_ushort %0, %1, %2 offset:%3" : "=v"(r) : "v"(voff), "s"(sbase), "n"(OFF));
-  return r;
-}
-template <int OFF>
-__device__ inline uint32_t ld1_so_off(const void* sbase, uint32_t voff) {
-  uint32_t r;
-  asm volatile("global_load_ubyte %0, %1, %2 offset:%3" : "=v"(r) : "v"(voff), "s"(sbase), "n"(OFF));
-  return r;
-}
 // (a & m) | c in one VALU operation. v_and_or_b32 takes no literal
 // constants and reads at most one SGPR: m comes in an SGPR, c in a VGPR
 // (both loop-invariant, so they are set up once).
@@ -174,6 +154,11 @@ __device__ inline v2u ld8_so(const void* sbase, uint32_t voff) {
 __device__ inline uint32_t ld2_so(const void* sbase, uint32_t voff) {
   uint32_t r;
   asm volatile("global_load_ushort %0, %1, %2" : "=v"(r) : "v"(voff), "s"(sbase));
+  return r;
+}
+__device__ inline uint32_t ld1_so(const void* sbase, uint32_t voff) {
+  uint32_t r;
+  asm volatile("global_load_ubyte %0, %1, %2" : "=v"(r) : "v"(voff), "s"(sbase));
   return r;
 }
 // Direct-to-LDS load at uniform base + per-lane offset (lds_dst as dma16).
