@@ -138,34 +138,52 @@ __device__ __forceinline__ void pa_q_split(const float (&qf)[NCH][8], int j0, v8
     }
 }
 
-// The keys of slots t0 .. t0 + 31 for row (T: its length, pos: its
-// position): -inf where masked (past the split's end kend, past the row's
-// length, or a ring slot a later token holds; rt = (last - t0) mod window).
-__device__ __forceinline__ void pa_mask(const v4f* sp, float (*sc)[4], int t0, int g, int kend, int T, int window,
-                                        int rt, uint32_t last, uint32_t pos) {
+// The keys of slots t0 .. t0 + 31 for a row: -inf where masked, which is at
+// or past lim (the split's end or the row's length, relative to t0), or in a
+// ring slot that a later token holds: slot t0 + i was written age = (rt - i)
+// mod window positions before the chunk's last one, and the row's token lies
+// `behind` positions before it.
+__device__ __forceinline__ void pa_mask(const v4f* sp, float (*sc)[4], int g, int lim, int window, int rt,
+                                        int behind) {
 #pragma unroll
   for (int st = 0; st < 2; ++st) {
     const v4f s = sp[st];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int i = 16 * st + 4 * g + e, slot = t0 + i;
-      bool ok = slot < kend && slot < T;
+      const int i = 16 * st + 4 * g + e;
+      bool ok = i < lim;
       if (window > 0) {
-        const int r = rt - i;  // (last - slot) mod window, for i < window
-        ok = ok && (long)last - (r >= 0 ? r : r + window) <= (long)pos;
+        const int r = rt - i;
+        ok = ok && (r >= 0 ? r : r + window) >= behind;
       }
       sc[st][e] = ok ? s[e] : -INFINITY;
     }
   }
 }
 
-// Keys below the returned slot are live for every row of a workgroup
-// (rows r0 ..): without a ring a row's keys are the slots below its length,
-// and the workgroup's first token has the shortest; with a ring, none is
-// taken as known.
-__device__ inline int pa_full_keys(int k0, int kend, int r0, int grp, uint32_t p0, int window, int stride) {
-  return window > 0 ? k0 : min(kend, att_len(p0 + (uint32_t)(r0 / grp), window, stride));
-}
+// Which tiles of a workgroup need no mask: their slots lie below the length
+// of the workgroup's first token (the shortest) and, in a ring, every one was
+// written at least as long ago as that token (the oldest): no wrap within the
+// tile and ages of at least rt - 31. rt (of the tile at hand) steps by one tile.
+struct PaLive {
+  int klim, behind, rt, window;
+  __device__ inline PaLive(int k0, int kend, int r0, int grp, uint32_t p0, int M, int window_, int stride)
+      : klim(min(kend, att_len(p0 + (uint32_t)(r0 / grp), window_, stride))),
+        behind(M - 1 - r0 / grp),
+        rt(window_ > 0 ? (int)(((long)p0 + M - 1 - k0) % window_) : 0),
+        window(window_) {
+    if (rt < 0) rt += window_;
+  }
+  __device__ inline bool full(int t0) const {
+    return t0 + PA_KT <= klim && (window == 0 || rt - (PA_KT - 1) >= behind);
+  }
+  __device__ inline void next() {
+    if (window > 0) {
+      rt -= PA_KT % window;
+      if (rt < 0) rt += window;
+    }
+  }
+};
 
 // Online softmax of a lane's 8 masked scores of the tile (row maximum and
 // sum across the row's 4 lanes) and the rescale of its accumulators: P in
@@ -251,7 +269,6 @@ pre_attn_kernel(const void* __restrict__ qin, int ldq, const float* __restrict__
   const int k0 = ks * ksl;
   if (k0 >= Tlast) return;  // no row of this workgroup has keys in this split (uniform)
   const int kend = min(k0 + ksl, Tlast);
-  const uint32_t last = p0 + (uint32_t)M - 1;  // the chunk's last position (all of its K/V are written)
 
   // ---- the next tile's K and V rows, loaded into registers one tile ahead.
   //      K chunks go to LDS row-major (lanes take consecutive chunks of a
@@ -306,7 +323,8 @@ pre_attn_kernel(const void* __restrict__ qin, int ldq, const float* __restrict__
 #pragma unroll
   for (int d = 0; d < NDT; ++d) oacc[d] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   float mrun = -INFINITY, lrun = 0.0f;
-  const int kfull = pa_full_keys(k0, kend, r0, grp, p0, window, stride);
+  PaLive live_keys(k0, kend, r0, grp, p0, M, window, stride);
+  const int klen = min(kend, T), behind = M - 1 - m;  // this row's (see pa_mask)
 
   for (int t0 = k0; t0 < kend; t0 += KT) {
     __syncthreads();  // every wave is done with the previous tile
@@ -317,9 +335,6 @@ pre_attn_kernel(const void* __restrict__ qin, int ldq, const float* __restrict__
     // ---- scores of the tile's keys for this lane's row: four independent
     //      MFMA chains (hi/lo x even/odd chunks) so consecutive MFMAs do not
     //      wait on each other's results ----
-    // ring slots t0 + i hold position last - ((last - t0 - i) mod window):
-    // one (uniform) division per tile
-    const int rt = window > 0 ? (int)(((long)last - t0) % window) : 0;
     v4f sp[2];
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
@@ -337,14 +352,15 @@ pre_attn_kernel(const void* __restrict__ qin, int ldq, const float* __restrict__
       sp[st] = (s0 + s1) + (s2 + s3);
     }
     float sc[2][4];
-    if (t0 + KT <= kfull) {  // every key of the tile is live for every row of the workgroup (uniform)
+    if (live_keys.full(t0)) {  // every key of the tile is live for every row of the workgroup (uniform)
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
         for (int e = 0; e < 4; ++e) sc[st][e] = sp[st][e];
     } else {
-      pa_mask(sp, sc, t0, g, kend, T, window, rt, last, pos);
+      pa_mask(sp, sc, g, klen - t0, window, live_keys.rt, behind);
     }
+    live_keys.next();
     const v8h pb = pa_softmax<NDT>(sc, mrun, lrun, oacc);
     // ---- O^T += V^T P^T, both subtiles in one K = 32 MFMA per output tile ----
 #pragma unroll
@@ -392,11 +408,14 @@ pre_attn_kernel(const void* __restrict__ qin, int ldq, const float* __restrict__
 // 32-key tiles, K direct loads and the K = 32 V product; 63.7 us with the
 // row address and mask changes; 58.5 us with the K rows loaded after the
 // exchange instead of with the V rows (the tile's loads all at once held
-// the score MFMAs back: 1.6k of ~7k cycles per tile). Not kept: the q
-// prologue (~10 us of the span) done once per row by a separate launch
-// (25 us for that launch), or reading qnw, cos and sin from LDS (67 us:
-// one more barrier, spills); the V rows loaded after the exchange too
-// (67 us: they no longer land before the next tile's store).
+// the score MFMAs back: 1.6k of ~7k cycles per tile); 97.4 us at 8128 keys before,
+// 95.5 (93.6 -> 90.2 us with the merge, untraced) with the rows prepared once
+// per workgroup and no spills. Not kept: the V
+// rows loaded after the exchange too (67 us: they no longer land before the
+// next tile's store); the V product of tile i - 1 beside the scores of tile i
+// (a second V^T tile; 97.4 -> 103.4 us at 8128 keys: the K rows then have only
+// the softmax to land); the rescale of the accumulators skipped when no row's
+// maximum moved (92.2 -> 94.7 us).
 constexpr int PA512_THREADS = 512;
 template <int QT>
 __global__ void __launch_bounds__(PA512_THREADS)
@@ -414,9 +433,14 @@ pre_attn512_kernel(const void* __restrict__ qin, int ldq, const float* __restric
   constexpr int VITEMS = (KT / 2) * CPR, VLD = VITEMS / NT;  // V key-pair chunks per tile, per thread
   constexpr int KPW = KT / WAVES;     // K rows each wave loads per tile
   static_assert(VITEMS % NT == 0 && KT % WAVES == 0 && NQC % 2 == 0, "tile shape");
-  __shared__ __attribute__((aligned(16))) uint8_t ksh[2][KT * KP];
-  __shared__ __attribute__((aligned(16))) uint8_t vsh[HD * VP];
-  __shared__ v4f xs[WAVES][2][64];  // each wave's partial scores of the tile
+  constexpr int QP = HD * 2 + 16;     // staged q row pitch (bytes)
+  constexpr int LOOPB = 2 * KT * KP + HD * VP + WAVES * 2 * 64 * 16, QB = 2 * PA_ROWS * QP;
+  // the q parts [2][PA_ROWS][QP] before the loop; then two K tiles, the V^T
+  // tile and each wave's partial scores of the tile
+  __shared__ __attribute__((aligned(16))) uint8_t lds[LOOPB > QB ? LOOPB : QB];
+  uint8_t(*ksh)[KT * KP] = reinterpret_cast<uint8_t(*)[KT * KP]>(lds);
+  uint8_t* const vsh = lds + 2 * KT * KP;
+  v4f(*xs)[2][64] = reinterpret_cast<v4f(*)[2][64]>(lds + 2 * KT * KP + HD * VP);
 
   const int kvh = blockIdx.x, ks = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
@@ -428,7 +452,6 @@ pre_attn512_kernel(const void* __restrict__ qin, int ldq, const float* __restric
   const int k0 = ks * ksl;
   if (k0 >= Tlast) return;  // uniform
   const int kend = min(k0 + ksl, Tlast);
-  const uint32_t last = p0 + (uint32_t)M - 1;
 
   // K rows of tile t0 -> ksh[b] (wave w loads rows w KPW .. + KPW - 1) and
   // the V rows of its key pairs -> registers. Away from the end of the cache
@@ -474,10 +497,55 @@ pre_attn512_kernel(const void* __restrict__ qin, int ldq, const float* __restric
     }
     kp += KT * HD;
   };
-  load_v(k0);
-  load_k(k0, 0);
 
-  // ---- this lane's query row: q-norm, RoPE, the hi/lo split of the wave's half ----
+  // ---- q-norm, RoPE and the hi/lo split, once per row: wave w prepares rows
+  //      8 w .. 8 w + 7 in row layout (lane l: elements 8 l ..; a row group's
+  //      lanes each loading their row's norm weights, cos and sin took 112
+  //      16-byte loads per wave and 9.5 us, now at most 42) and the parts
+  //      reach the waves of the row group through LDS ----
+  {
+    constexpr int RPW = PA_ROWS / WAVES;
+    float qf[RPW][8], w[8], cc[8], sv[8];
+    int mi[RPW];
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const int Ri = r0 + RPW * wave + i;
+      const bool ok = Ri < nrows;
+      mi[i] = ok ? Ri / grp : 0;
+      const int hi = kvh * grp + (ok ? Ri % grp : 0);
+      ld8f<QT>(qin, (long)mi[i] * ldq + (long)hi * HD + 8 * lane, qf[i]);
+    }
+    ld8f<Q4_DT_F32>(qnw, 8 * lane, w);
+    const bool lo = lane < 32;
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      if (i == 0 || mi[i] != mi[i - 1]) {  // (uniform) rows of one token share its cos and sin
+        ld8f<Q4_DT_F32>(cosM, (long)mi[i] * HD + 8 * lane, cc);
+        ld8f<Q4_DT_F32>(sinM, (long)mi[i] * HD + 8 * lane, sv);
+      }
+      float ss = 0.0f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) ss = fmaf(qf[i][u], qf[i][u], ss);
+      ss = reduce64<false>(ss);
+      const float inv = 1.0f / sqrtf(ss / (float)HD + PA_EPS);
+      float x[1][8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float y = __fmul_rn(__fmul_rn(qf[i][u], inv), w[u]);
+        const auto pr2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+        const float pr = __uint_as_float(lo ? pr2[1] : pr2[0]);  // element +- HD / 2
+        x[0][u] = __fadd_rn(__fmul_rn(y, cc[u]), __fmul_rn(lo ? -pr : pr, sv[u]));
+      }
+      v8h xh, xl;
+      pa_q_split<1>(x, 0, &xh, &xl);
+      *reinterpret_cast<v8h*>(lds + (RPW * wave + i) * QP + 16 * lane) = xh;
+      *reinterpret_cast<v8h*>(lds + (PA_ROWS + RPW * wave + i) * QP + 16 * lane) = xl;
+    }
+  }
+  load_v(k0);
+  __syncthreads();
+
+  // ---- this lane's query row, the wave's half of its elements ----
   const int R = r0 + 16 * rg + c;
   const bool live = R < nrows;
   const int m = live ? R / grp : 0;
@@ -485,19 +553,21 @@ pre_attn512_kernel(const void* __restrict__ qin, int ldq, const float* __restric
   const uint32_t pos = p0 + (uint32_t)m;
   const int T = att_len(pos, window, stride);
   v8h qh[NQC], ql[NQC];
-  {
-    float qf[NCH][8];
-    pa_q_row<HD, QT>(qin, (long)m * ldq + (long)h * HD, qnw, cosM + (long)m * HD, sinM + (long)m * HD, g, qf);
-    // a wave-uniform branch keeps the register indices static
-    if (dp == 0) pa_q_split<NQC>(qf, 0, qh, ql);
-    else pa_q_split<NQC>(qf, NQC, qh, ql);
+#pragma unroll
+  for (int j = 0; j < NQC; ++j) {
+    const uint8_t* qp = lds + (16 * rg + c) * QP + (4 * (dp * NQC + j) + g) * 16;
+    qh[j] = *reinterpret_cast<const v8h*>(qp);
+    ql[j] = *reinterpret_cast<const v8h*>(qp + PA_ROWS * QP);
   }
+  __syncthreads();  // the parts are read before the tiles take the LDS
+  load_k(k0, 0);
 
   v4f oacc[NDT];
 #pragma unroll
   for (int d = 0; d < NDT; ++d) oacc[d] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   float mrun = -INFINITY, lrun = 0.0f;
-  const int kfull = pa_full_keys(k0, kend, r0, grp, p0, window, stride);
+  PaLive live_keys(k0, kend, r0, grp, p0, M, window, stride);
+  const int klen = min(kend, T), behind = M - 1 - m;  // this row's (see pa_mask)
 
   int b = 0;
   for (int t0 = k0; t0 < kend; t0 += KT, b ^= 1) {
@@ -510,7 +580,6 @@ pre_attn512_kernel(const void* __restrict__ qin, int ldq, const float* __restric
     }
     const bool more = t0 + KT < kend;
     if (more) load_v(t0 + KT);  // the next tile's V rows run under this tile's math
-    const int rt = window > 0 ? (int)(((long)last - t0) % window) : 0;
     v4f sp[2];
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
@@ -535,14 +604,15 @@ pre_attn512_kernel(const void* __restrict__ qin, int ldq, const float* __restric
 #pragma unroll
     for (int st = 0; st < 2; ++st) sp[st] = xs[rg * DS][st][lane] + xs[rg * DS + 1][st][lane];
     float sc[2][4];
-    if (t0 + KT <= kfull) {  // uniform
+    if (live_keys.full(t0)) {  // uniform
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
         for (int e = 0; e < 4; ++e) sc[st][e] = sp[st][e];
     } else {
-      pa_mask(sp, sc, t0, g, kend, T, window, rt, last, pos);
+      pa_mask(sp, sc, g, klen - t0, window, live_keys.rt, behind);
     }
+    live_keys.next();
     const v8h pb = pa_softmax<NDT>(sc, mrun, lrun, oacc);
 #pragma unroll
     for (int d = 0; d < NDT; ++d) {

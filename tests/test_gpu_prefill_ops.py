@@ -223,3 +223,28 @@ def test_pre_attn_graph_replay_follows_p0(gpu):
         assert O.normwise_rel_err(got, ref) <= 2e-4, chunk
         rkc, rvc = _np(kc).copy(), _np(vc).copy()  # carry the device caches (fp16 rounding ties aside)
     g.destroy()
+
+
+@pytest.mark.parametrize("hd,nH,nkv,stride,window,M,p0", [
+    (256, 4, 2, 1024, 1024, 128, 1000),   # the chunk's slots wrap; whole tiles without a mask on both sides
+    (256, 4, 2, 1024, 1024, 128, 896),    # ends on the ring's last slot
+    (256, 4, 2, 1024, 1024, 97, 2013),    # odd length and position, several turns
+    (64, 2, 2, 100, 100, 33, 260),        # a window that is no multiple of the tile
+    (128, 2, 1, 48, 24, 20, 61),          # a window shorter than a tile
+    (512, 16, 1, 160, 96, 40, 200),       # hd 512 ring, rows of one token per 16
+    (512, 6, 2, 200, 0, 23, 100),         # hd 512, three heads per token: tokens change inside a wave's rows
+])
+def test_pre_attn_masks_and_rows(gpu, hd, nH, nkv, stride, window, M, p0):
+    """Ring ages, tiles that skip the mask and the row preparation of hd 512,
+    against the oracle (the bounds of test_pre_attn_vs_oracle)."""
+    rng = np.random.default_rng(hd + M + p0 + window)
+    Q, qnw, cosM, sinM, kc, vc = _attn_case(rng, M=M, nH=nH, nkv=nkv, hd=hd, stride=stride, window=window, p0=p0,
+                                            qdt=torch.float32, peaky=True)
+    ref = P.pre_attn_ref(Q, qnw, cosM, sinM, kc, vc, nH=nH, hd=hd, stride=stride, window=window, grp=nH // nkv,
+                         p0=p0)
+    out = gpu.pre_attn(_t(Q), _t(qnw), _t(cosM), _t(sinM), _t(kc, torch.float16), _t(vc, torch.float16), M=M,
+                       ldq=nH * hd, nH=nH, nkv=nkv, hd=hd, stride=stride, window=window, max_keys=window or stride,
+                       dyn=_dyn(p0, M), out_dtype=torch.float32)
+    got = _np(out).astype(np.float64)
+    for m in range(M):
+        assert O.normwise_rel_err(got[m], ref[m]) <= 2e-4, m
