@@ -408,9 +408,9 @@ pre_attn_kernel(const void* __restrict__ qin, int ldq, const float* __restrict__
 // 32-key tiles, K direct loads and the K = 32 V product; 63.7 us with the
 // row address and mask changes; 58.5 us with the K rows loaded after the
 // exchange instead of with the V rows (the tile's loads all at once held
-// the score MFMAs back: 1.6k of ~7k cycles per tile); 97.4 us at 8128 keys before,
-// 95.5 (93.6 -> 90.2 us with the merge, untraced) with the rows prepared once
-// per workgroup and no spills. Not kept: the V
+// the score MFMAs back: 1.6k of ~7k cycles per tile);
+// with the rows prepared once per workgroup and no spills, 128 tokens x 16
+// heads over 8128 keys 93.6 -> 90.2 us (merge included). Not kept: the V
 // rows loaded after the exchange too (67 us: they no longer land before the
 // next tile's store); the V product of tile i - 1 beside the scores of tile i
 // (a second V^T tile; 97.4 -> 103.4 us at 8128 keys: the K rows then have only
