@@ -591,7 +591,7 @@ gemv_multi_kernel(const uint16_t* __restrict__ X, int M, const uint4* __restrict
 // nibbles, mantissa bits 4-7: 64 + q), minus 1032 or 72, give q - 8
 // exactly; 9 VALU operations per 8 codes, whatever the number of vectors.
 //
-// A workgroup (4 waves) owns T tiles of 16 rows (16T rows of one 64-row
+// A workgroup (4 or 8 waves) owns T tiles of 16 rows (16T rows of one 64-row
 // panel). One step of a wave covers 4 (tile, block) pairs, 4/T blocks of
 // all T tiles: each lane loads one whole 16-byte unit (lane (c, g): tile
 // g % T, row c, block g / T of the step; 1 KB of contiguous weights per
@@ -600,9 +600,9 @@ gemv_multi_kernel(const uint16_t* __restrict__ X, int M, const uint4* __restrict
 // (c, g) word g of the 4 units of its column, one per MFMA. The lane loads its
 // unit's scale too (one load where every lane loaded the four scales of its
 // column), and three permlane swaps hand all four to each lane. Steps go to
-// the waves round-robin (the 4 waves read adjacent blocks together); U
+// the waves round-robin (the waves read adjacent blocks together); U
 // steps of loads stay in flight (x slices, the unit, its scale per step;
-// explicit wait counts as in the GEMV), and the 4 waves' partial sums meet
+// explicit wait counts as in the GEMV), and the waves' partial sums meet
 // in LDS in wave order (deterministic).
 __device__ inline v8h codes_to_h8(uint32_t w) {
   const uint32_t w8 = w >> 8;
@@ -640,15 +640,23 @@ __device__ inline uint32_t mm_scale(const uint8_t* sbase, uint32_t voff) {
   else return ld1_so(sbase, voff);
 }
 
+// Waves per workgroup of T tiles. 8 (two per SIMD) at T = 4, where a grid is
+// one workgroup per CU and a wave's transposes, dequant and dependent MFMAs
+// stall it between loads: 15360 x 3840, 8 vectors 9.75 -> 9.15 us, 3840 x 15360
+// in 4 splits 11.7 -> 11.4. With fewer tiles a wave has few steps: 4 (3840 x
+// 8192 8.2 us, 8.6 with 8 waves).
+__host__ __device__ constexpr int mm_waves(int T) { return T == 4 ? 8 : 4; }
+
 template <int T, int U, int ST, int YT>
-__global__ void __launch_bounds__(GEMV_THREADS)
+__global__ void __launch_bounds__(64 * mm_waves(T))
 gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict__ wq, const void* __restrict__ scv,
                float outscale, void* __restrict__ Y, int N, int nblk, int kspan, float* __restrict__ part) {
+  constexpr int W = mm_waves(T);                  // waves per workgroup
   constexpr int BPS = 4 / T;                      // blocks per step
   constexpr int L = BPS + 2;                      // loads per step: x slices, the unit and its scale
   constexpr int SB = ST == Q4_SCALE_F16 ? 2 : 1;  // scale bytes
   static_assert(U * L < 64, "vmcnt range");
-  __shared__ v4f red[GEMV_WAVES][T][64];
+  __shared__ v4f red[W][T][64];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: block indices and bases live in SGPRs
   const int c = lane & 15, g = lane >> 4;
@@ -663,11 +671,11 @@ gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict_
   const uint32_t xo = (uint32_t)min(c, M - 1) * (uint32_t)(nblk * BLK * 2) + g * 16;
   const int lrow = 16 * (g % T) + c, lblk = g / T;  // the unit lane (c, g) loads: row, block within the step
   const int nsteps = (nb + BPS - 1) / BPS;
-  const int rounds = ((nsteps + GEMV_WAVES - 1) / GEMV_WAVES + U - 1) / U;
+  const int rounds = ((nsteps + W - 1) / W + U - 1) / U;
   v4u xr[U][BPS], wr[U];
   uint32_t sr[U];
   auto issue = [&](int u, int s) {
-    const int b0 = (wave + GEMV_WAVES * s) * BPS;  // first block of the step
+    const int b0 = (wave + W * s) * BPS;  // first block of the step
     static_for<0, BPS>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
       xr[u][i] = ld16_so(xbase + (long)min(b0 + i, nb - 1) * (BLK * 2), xo);
@@ -679,7 +687,7 @@ gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict_
 #pragma unroll
   for (int t = 0; t < T; ++t) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   auto use = [&](int u, int s) {
-    const int b0 = (wave + GEMV_WAVES * s) * BPS;
+    const int b0 = (wave + W * s) * BPS;
     if (b0 < nb) {
       const v4u w = transpose_rows(wr[u]);
       const v4u sv = share_rows(sr[u]);
@@ -728,8 +736,10 @@ gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict_
 #pragma unroll
   for (int t = 0; t < T; ++t) red[wave][t][lane] = acc[t];
   __syncthreads();
-  for (int t = wave; t < T; t += GEMV_WAVES) {
-    const v4f y = ((red[0][t][lane] + red[1][t][lane]) + red[2][t][lane]) + red[3][t][lane];
+  for (int t = wave; t < T; t += W) {
+    v4f y = red[0][t][lane];
+#pragma unroll
+    for (int w = 1; w < W; ++w) y += red[w][t][lane];
     const int n = n0 + 16 * t + c;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -1351,14 +1361,14 @@ static int gemv_mm_launch(const void* x, int M, const uint32_t* wq, const void* 
   const int NP = pad_rows(N);
   if (split <= 1) {
     const int T = mm_tiles(NP);
-    hipLaunchKernelGGL(pick_mm(T, mm_deep(), scale_fmt, y_dtype), dim3(NP / (16 * T)), dim3(GEMV_THREADS), 0, st,
+    hipLaunchKernelGGL(pick_mm(T, mm_deep(), scale_fmt, y_dtype), dim3(NP / (16 * T)), dim3(64 * mm_waves(T)), 0, st,
                        reinterpret_cast<const uint16_t*>(x), M, reinterpret_cast<const uint8_t*>(wq), scales,
                        outscale, y, N, nblk, nblk, nullptr);
     Q4_LAUNCHED("gemv_mm");
     return Q4_OK;
   }
   const int span = (nblk + split - 1) / split;
-  hipLaunchKernelGGL(pick_mm(4, mm_deep(), scale_fmt, y_dtype), dim3(NP / 64, split), dim3(GEMV_THREADS), 0, st,
+  hipLaunchKernelGGL(pick_mm(4, mm_deep(), scale_fmt, y_dtype), dim3(NP / 64, split), dim3(64 * mm_waves(4)), 0, st,
                      reinterpret_cast<const uint16_t*>(x), M, reinterpret_cast<const uint8_t*>(wq), scales, outscale,
                      y, N, nblk, span, ws);
   Q4_LAUNCHED("gemv_mm split");
