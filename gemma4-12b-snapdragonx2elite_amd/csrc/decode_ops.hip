@@ -725,11 +725,15 @@ attn_split_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, 
 
 // The same split for 16 query heads of one KV head at hd 512 (the k == v
 // global layers), on the matrix cores: scores and p V are 16-row products and
-// the cache is read once for all 16 heads instead of once per 4. q and p stay
-// fp32 values: each is split into fp16 hi + lo parts (~22 bits) after an exact
-// power-of-two scaling (q: a head's largest element to [2^13, 2^14); p: 2^14),
-// so that both parts are normal numbers, and the two products with the fp16
-// cache are exact in the fp32 accumulators.
+// the cache is read once for all 16 heads instead of once per 4. The fp32 q
+// and p are each split into three fp16 parts (11 + 11 + 2 bits) after an
+// exact power-of-two scaling (q: a head's largest element to [2^13, 2^14); p:
+// 2^14): the parts sum to the fp32 value itself, except that bits below 2^-38
+// of the scale are rounded off, and their products with the fp16 cache are
+// exact in the fp32 accumulators. Zero parts and parts of both signs do not
+// multiply an Inf (in the cache) as their sum would: scores or sums that come
+// out not finite are taken again with fp32 operands (16x16x4), which gives an
+// Inf or NaN exactly where fp32 arithmetic does.
 //
 // Workgroup (g, sp): heads 16 g .., keys [32 sp, 32 sp + 32), 4 waves. All
 // loads come first (37 per wave, 64 KB of K and V per workgroup): this round
@@ -742,11 +746,13 @@ attn_split_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, 
 // wave's own 128 columns of V: column c of MFMA e is dim 8 c + e, so a lane's
 // 16-byte V loads of 8 keys hold the B operands of 8 MFMAs, transposed in the
 // lane by byte permutes, and its results are 8 consecutive dims.
-// Measured at 8101 keys (256 splits, 16.6 MB of cache per layer, kernel
-// trace): 22.6 us with the 4-head kernel, 14.7 with the same split on the
-// fp32 matrix instruction (16x16x4: 8 times the MFMA cycles, K and V widened
-// first, every lane loading the norm and RoPE rows), 12.1 us. Error against 64
-// bits with fp32 outputs, 8101 keys: 3.7e-7 (4 heads), 2.9e-7, 2.5e-7.
+// Measured at 8101 keys (256 splits, 16.6 MB of cache per layer), split and
+// merge of four layers: 160 us with the 4-head kernel, 71.0 (69.0 with two
+// parts per value and no check); the same split on the fp32 matrix
+// instruction alone (8 times the MFMA cycles, K and V widened first) took 2.6
+// us more per layer. Error against 64 bits with fp32 outputs, 2-norm, mean
+// over positions 1 to 8191 and score spreads of 0.25 to 4: 1.0e-7 to 6.8e-7
+// with the 4-head kernel, 1.0e-7 to 5.2e-7 here.
 template <bool PREP>
 __global__ void __launch_bounds__(256)
 attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, const float* __restrict__ cs,
@@ -756,8 +762,10 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
   constexpr int EPL = 8, HD = 512, KCH = 32, NW = 4, SST = KCH + 4;  // SST: score row stride (words)
   constexpr int QP = HD + 8;         // q row pitch (halves): 16 rows of a 16-byte column in distinct banks
   constexpr int HPW = ATT_MMH / NW;  // heads a wave prepares
+  constexpr int QF = HD + 4;         // fp32 q row pitch (floats), in the parts' place
   constexpr float PSC = 16384.0f;    // scale of p's parts
-  __shared__ __attribute__((aligned(16))) uint16_t qs[2][ATT_MMH][QP];  // hi, lo
+  static_assert(QF * 4 <= 3 * QP * 2, "fp32 q rows fit the parts");
+  __shared__ __attribute__((aligned(16))) uint16_t qs[3][ATT_MMH][QP];  // hi, mid, lo
   __shared__ __attribute__((aligned(16))) float sc[NW][ATT_MMH][SST];
   __shared__ __attribute__((aligned(16))) uint16_t fresh[PREP ? NW : 1][2][PREP ? HD : 8];
   __shared__ float qinv[ATT_MMH];    // inverse of each head's scale
@@ -801,15 +809,18 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
   // (2) q norm and RoPE of this wave's heads, their scaled parts to LDS; with
   //     the fresh slot in this split, this token's K and V through the wave's
   //     own LDS rows
-  auto halves = [](const float(&v)[8], v4u& hi, v4u& lo) {
-    v8h h, l;
+  auto parts = [](const float(&v)[8], v4u(&pt)[3]) {
+    v8h h, m, l;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       h[e] = (_Float16)v[e];
-      l[e] = (_Float16)(v[e] - (float)h[e]);
+      const float r = v[e] - (float)h[e];
+      m[e] = (_Float16)r;
+      l[e] = (_Float16)(r - (float)m[e]);
     }
-    hi = __builtin_bit_cast(v4u, h);
-    lo = __builtin_bit_cast(v4u, l);
+    pt[0] = __builtin_bit_cast(v4u, h);
+    pt[1] = __builtin_bit_cast(v4u, m);
+    pt[2] = __builtin_bit_cast(v4u, l);
   };
 #pragma unroll
   for (int i = 0; i < HPW; ++i) {
@@ -823,10 +834,10 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
     const float scale = __uint_as_float((uint32_t)ex << 23);
 #pragma unroll
     for (int e = 0; e < EPL; ++e) q[i][e] *= scale;
-    v4u hi, lo;
-    halves(q[i], hi, lo);
-    *reinterpret_cast<v4u*>(&qs[0][HPW * wave + i][EPL * lane]) = hi;
-    *reinterpret_cast<v4u*>(&qs[1][HPW * wave + i][EPL * lane]) = lo;
+    v4u pt[3];
+    parts(q[i], pt);
+#pragma unroll
+    for (int u = 0; u < 3; ++u) *reinterpret_cast<v4u*>(&qs[u][HPW * wave + i][EPL * lane]) = pt[u];
     if (lane == 0) qinv[HPW * wave + i] = __uint_as_float((uint32_t)(254 - ex) << 23);
   }
   if constexpr (PREP) {
@@ -862,11 +873,11 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
   }
 
   // (3) this wave's part of the scores: D column l % 16 = key, rows 4 (l / 16) .. = heads
-  v4f d[2][2] = {};  // [key tile][part]
+  v4f d[2][3] = {};  // [key tile][part]
 #pragma unroll
   for (int c = 0; c < 4; ++c)
 #pragma unroll
-    for (int pt = 0; pt < 2; ++pt) {
+    for (int pt = 0; pt < 3; ++pt) {
       const v8h a = *reinterpret_cast<const v8h*>(&qs[pt][li][sdim(c)]);
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
@@ -875,22 +886,58 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
 #pragma unroll
   for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float sum = d[kt][0][v] + d[kt][1][v];
-      sc[wave][4 * lg + v][16 * kt + li] = sum;
-    }
+    for (int v = 0; v < 4; ++v) sc[wave][4 * lg + v][16 * kt + li] = d[kt][0][v] + (d[kt][1][v] + d[kt][2][v]);
   __syncthreads();
 
   // (4) softmax over the split's keys: lane = head li, keys 8 lg .. + 7
-  const float qi = qinv[li];
   float p[8];
+  auto take_scores = [&](float scale) {  // the waves' sums; true where a live key's is not finite
+    bool odd = false;
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    v4f x = *reinterpret_cast<const v4f*>(&sc[0][li][8 * lg + 4 * b]);
+    for (int b = 0; b < 2; ++b) {
+      v4f x = *reinterpret_cast<const v4f*>(&sc[0][li][8 * lg + 4 * b]);
 #pragma unroll
-    for (int w = 1; w < NW; ++w) x += *reinterpret_cast<const v4f*>(&sc[w][li][8 * lg + 4 * b]);
+      for (int w = 1; w < NW; ++w) x += *reinterpret_cast<const v4f*>(&sc[w][li][8 * lg + 4 * b]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) p[4 * b + e] = 8 * lg + 4 * b + e < n ? x[e] * qi : -INFINITY;
+      for (int e = 0; e < 4; ++e) {
+        const bool live = 8 * lg + 4 * b + e < n;
+        p[4 * b + e] = live ? x[e] * scale : -INFINITY;
+        odd |= live && !(fabsf(x[e]) < INFINITY);
+      }
+    }
+    return odd;
+  };
+  if (__builtin_amdgcn_ballot_w64(take_scores(qinv[li]))) {  // workgroup-uniform: every wave adds the same sums
+    __syncthreads();  // the parts and the sums are read
+    float* const qf = reinterpret_cast<float*>(qs);
+    for (int i = 0; i < HPW; ++i) {
+      float x[EPL], w[EPL], c[EPL], s[EPL];
+      ld_row<EPL>(qkv + qoff + (long)(h0 + HPW * wave + i) * HD, x);
+      ld_row<EPL>(qnw, w);
+      ld_row<EPL>(cs, c);
+      ld_row<EPL>(sn, s);
+      row_norm_rope<EPL>(x, w, c, s);
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) qf[(HPW * wave + i) * QF + EPL * lane + e] = x[e];
+    }
+    __syncthreads();
+    v4f f[2] = {};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float a = qf[li * QF + sdim(c) + e];
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+          f[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, h2f((uint16_t)(ku[kt][c][e >> 1] >> (16 * (e & 1)))), f[kt], 0,
+                                                       0, 0);
+      }
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sc[wave][4 * lg + v][16 * kt + li] = f[kt][v];
+    __syncthreads();
+    take_scores(1.0f);
   }
   float m = p[0];
 #pragma unroll
@@ -907,23 +954,38 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
 
   // (5) unnormalised p V over the wave's 128 dims. Rows past the length are
   //     taken as zero (a never-written cache row may hold a NaN).
-  v4u ph, pl;
-  halves(p, ph, pl);
+  v4u pp[3];
+  parts(p, pp);
   if (n < KCH) {
 #pragma unroll
     for (int s = 0; s < 8; ++s)
       if (8 * lg + s >= n) vv[s] = v4u{0u, 0u, 0u, 0u};
   }
   v4f o[8];
+  float fin = 0.0f;  // stays zero while the sums are finite
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
     const int w = e >> 1;
     const v4u bt = {__builtin_amdgcn_perm(vv[1][w], vv[0][w], sel), __builtin_amdgcn_perm(vv[3][w], vv[2][w], sel),
                     __builtin_amdgcn_perm(vv[5][w], vv[4][w], sel), __builtin_amdgcn_perm(vv[7][w], vv[6][w], sel)};
-    const v8h bh = __builtin_bit_cast(v8h, bt);
-    o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, ph), bh, v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-    o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, pl), bh, o[e], 0, 0, 0);
+    o[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+      o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, pp[u]), __builtin_bit_cast(v8h, bt), o[e], 0,
+                                                    0, 0);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) fin = fmaf(o[e][v], 0.0f, fin);
+  }
+  if (__builtin_amdgcn_ballot_w64(fin != 0.0f)) {  // (a NaN is not equal to zero)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      o[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], h2f((uint16_t)(vv[s][e >> 1] >> (16 * (e & 1)))), o[e], 0, 0,
+                                                    0);
+    }
   }
 #pragma unroll
   for (int v = 0; v < 4; ++v) {

@@ -270,3 +270,41 @@ def test_prepkv_attn_many_heads_and_splits(gpu, nH, nkv, hd, stride, pos):
     ref = D.attn_ref(qkv, qnw, cs, sn, _np(kc1), _np(vc1), nH=nH, hd=hd, stride=stride, window=0, qoff=0,
                      grp=nH // nkv, pos=min(pos, stride - 1))
     assert O.normwise_rel_err(_np(o1), ref) <= 1e-4   # the bound of test_attn: fp32 sums over fp16 caches
+
+
+@pytest.mark.parametrize("nH,nkv,stride,window,pos", [
+    (16, 1, 64, 0, 20),         # one split, 11 of its 32 keys past the length
+    (16, 1, 300, 0, 250),       # eight splits, the last one partial
+    (32, 2, 96, 96, 250),       # a wrapped ring, two KV heads
+])
+@pytest.mark.parametrize("where", ["K", "V", "K and V"])
+def test_attn_infinities_in_the_cache(gpu, nH, nkv, stride, window, pos, where):
+    """16-head groups at hd 512 with an Inf in live cache rows give Inf and
+    NaN where fp32 arithmetic does: a key whose score is -Inf has weight 0
+    and leaves its head finite, one whose score is +Inf makes it NaN, and an
+    Inf in V reaches its own dim only. The other outputs keep test_attn's
+    bound."""
+    hd = 512
+    rng = np.random.default_rng(stride + pos)
+    qkv, qnw, cs, sn, kc, vc = _attn_case(rng, nH, nkv, hd, stride)
+    K, V = kc.reshape(nkv, stride, hd), vc.reshape(nkv, stride, hd)
+    with np.errstate(over="ignore"):
+        if "K" in where:
+            K[0, 3, 100] = np.inf
+            K[-1, 17, 511] = -np.inf
+        if "V" in where:
+            V[0, 5, 7] = np.inf
+            V[0, 19, 300] = -np.inf
+            V[-1, 6, 130], V[-1, 12, 130] = np.inf, -np.inf   # meet: NaN
+    dyn = torch.tensor([pos, pos + 1, 0, 0], dtype=torch.int32, device="cuda")
+    got = _np(gpu.attn(_t(qkv), _t(qnw), _t(cs), _t(sn), _t(kc, torch.float16), _t(vc, torch.float16), nH=nH, nkv=nkv,
+                       hd=hd, stride=stride, window=window, qoff=0, grp=nH // nkv, dyn=dyn))
+    with np.errstate(invalid="ignore"):
+        ref = D.attn_ref(qkv, qnw, cs, sn, kc, vc, nH=nH, hd=hd, stride=stride, window=window, qoff=0,
+                         grp=nH // nkv, pos=pos)
+    got, ref = got.reshape(-1), np.asarray(ref).reshape(-1)
+    assert np.isnan(ref).any() and np.isfinite(ref).any()
+    assert (np.isnan(got) == np.isnan(ref)).all()
+    assert (np.isinf(got) == np.isinf(ref)).all() and (got[np.isinf(ref)] == ref[np.isinf(ref)]).all()
+    ok = np.isfinite(ref)
+    assert O.normwise_rel_err(got[ok], ref[ok]) <= 1e-4
