@@ -1785,29 +1785,50 @@ static int w4a16_kgroups(int M, int N, int K, int split) {
 }
 
 // Launch plan of a W4A16 GEMM. `narrow`: two k-groups of two waves on 128 x
-// 128 tiles, taken where the wide plan would split K at one group: the groups
-// take the place of half the splits, each with at least W4A16_NARROW_KSTEPS
-// k-steps. The k-loop is the same per wave (~1600 cycles per k-step at the
-// 1.7 to 2.1 GHz the chip holds under it); the gain is in the partials, which
-// the GEMM writes and the next kernel reads at HBM speed. Per GEMM with its
-// reduction at M 128, wide / narrow: N 30720, K 3840 45.7 / 40.2 us, 8192 x 3840
-// 23.5 / 20.4, 3840 x 4096 20.8 / 18.7, 3840 x 15360 31.1 / 28.6; M 256, 15360 x
-// 3840 42.7 / 36.7; the gated gate/up GEMM (30720 x 3840) leaves no partials
-// and no second kernel (36.8 + 6.8 -> 41.0 us in a kernel trace).
-// Never more splits than the wide plan, whose partials size the workspace.
+// 128 tiles in place of splits of the wide plan (256 columns, one group). The
+// k-loop is about the same per wave (~1600 cycles per k-step at the 1.7 to 2.1
+// GHz the chip holds under it); the gain is in the partials, which the GEMM
+// writes and the next kernel reads at HBM speed. Per GEMM with its reduction at
+// M 128, wide / narrow: N 30720, K 3840 44.0 / 37.4 us, 8192 x 3840 24.5 / 21.5,
+// 3840 x 4096 22.6 / 20.2, 3840 x 15360 30.9 / 28.6; M 256, 15360 x 3840 43.2 /
+// 36.6; the gated gate/up GEMM (30720 x 3840) leaves no partials and no second
+// kernel (36.8 + 6.8 -> 41.0 us in a kernel trace).
+// Splits of the narrow plan, at most the wide plan's (whose partials size the
+// workspace):
+//  - one round: a workgroup's 131 KB of LDS fill a CU, so 256 workgroups run at
+//    a time (M 300, 4096 x 3840: 288 workgroups 34.6 us, 192 25.8, wide 26.3; M
+//    128, 10000 x 7040: 316 41.6 us, 237 31.1, wide 33.1);
+//  - groups of at least 8 k-steps, or 4 where partials are cheap: up to 48 rows
+//    (M 17, 4096 x 3840: 17.2 -> 15.3 us, wide 16.8), or for grids under 64
+//    workgroups of up to three splits, which then grow to 128 (M 77, 1000 x
+//    4032: 18.4 -> 15.4, wide 17.8; M 64, 6000 x 1600: 18.1 -> 16.4, wide
+//    17.8; from four splits on it loses: M 100, 1040 x 8000 19.5 -> 20.4). One
+//    split stays one where a second kernel would sum large partials whose odd
+//    rows are stored and read element by element (M 219, 2951 x 1120 16.0 ->
+//    20.0; M 68, 985 x 1920 20.0 -> 14.8).
+// The narrow plan is taken where its groups run fewer k-steps than the wide
+// plan's waves, where it leaves no second kernel, or where the partials it
+// saves (~0.1 us per split and 0.8 us per million fp32 values) are worth the
+// second read of A in its loop (~0.045 us per k-step): with few rows they are
+// not (M 1, 16000 x 8000 37.8 us, wide 35.9; even at M 64).
 struct W4Plan {
   int split, bm, kg;
   bool narrow;
 };
-constexpr int W4A16_NARROW_KSTEPS = 8;
 static W4Plan w4a16_plan(int M, int N, int K) {
   W4Plan p{w4a16_split(M, N, K), pick_bm(M, N), 1, false};
   p.kg = w4a16_kgroups(M, N, K, p.split);
   const bool tuned = tune_value(Q4_TUNE_W4A16_SPLIT) >= 0 || tune_value(Q4_TUNE_W4A16_KG) >= 0;
   if (!tuned && p.bm == 128 && p.kg == 1 && p.split > 1) {
     const int nk = (K / 32 + 1) / 2, t = ceil_div(M, 128) * ceil_div(N, 128);
-    const int s = min(ceil_div(240, t), nk / (2 * W4A16_NARROW_KSTEPS));
-    if (s >= 1 && s < p.split) p = W4Plan{s, 128, 2, true};
+    const int round = max(1, 256 / t);
+    int s = min(round, nk / (M <= 48 ? 8 : 16));
+    if (t * s < 64 && s < 4 && (s > 1 || N % 4 == 0 || (long)M * N <= 100000))
+      s = max(s, min(min(round, 128 / t), nk / 8));
+    s = min(s, p.split);
+    const bool shorter = 4 * s >= 3 * p.split;  // nk / (2 s) k-steps per group against nk / split
+    const long saved = ((long)M * N + 125000) * (p.split - s), reread = 56000L * ceil_div(nk, 2 * s);
+    if (shorter || s == 1 || saved >= reread) p = W4Plan{s, 128, 2, true};
   }
   return p;
 }

@@ -476,6 +476,34 @@ def test_w4a16_narrow_tiles(gpu, M, N, K, tune):
     assert np.abs(A - act).max() <= np.abs(act).max() * 2.0 ** -9
 
 
+@pytest.mark.parametrize("M,N,K", [(48, 1000, 4032),     # groups of 4 k-steps: seven splits, uneven
+                                   (49, 1000, 4032),     # a grid under 64 workgroups: the same
+                                   (65, 2000, 2048),     # under 64 workgroups grown to 64
+                                   (130, 5440, 3840),    # 86 tiles: two splits, 172 workgroups
+                                   (129, 10816, 1056),   # 170 tiles: one split, one round, half a last k-step
+                                   (300, 10752, 1024),   # 252 tiles: one split, the fullest round
+                                   (257, 11008, 1056)])  # 258 tiles: one split, two rounds
+@pytest.mark.parametrize("gated", [False, True])
+def test_w4a16_split_rules(gpu, M, N, K, gated, tune):
+    """Shapes on both sides of the rules that choose the splits, against the
+    256-column one-group plan (sums in another order: one fp16 step of the
+    largest output; the gated product of two such steps: two) and, per
+    element, the fp32 product."""
+    rng = np.random.default_rng(M + N + K)
+    q, s = synth_int4(rng, N, K)
+    wq, sc = upload_int4(q, s)
+    X = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float16)).cuda()
+    fn = gpu.gemm_w4a16_gated if gated else gpu.gemm_w4a16
+    Y = to_np(fn(X, wq, sc, N)).astype(np.float64)
+    tune("w4a16_kg", "1")
+    Y1 = to_np(fn(X, wq, sc, N)).astype(np.float64)
+    assert np.abs(Y - Y1).max() <= np.abs(Y1).max() * 2.0 ** (-8 if gated else -9)
+    if not gated:
+        W = ((torch.from_numpy(q).cuda().float() - 8) * torch.from_numpy(s).cuda().float().repeat_interleave(32, 1))
+        ref = (X.float() @ W.half().float().T).cpu().numpy().astype(np.float64)
+        assert np.abs(Y - ref).max() <= np.abs(ref).max() * 2.0 ** -9
+
+
 @pytest.mark.parametrize("M,N,K,fuse_norm", [(128, 3840, 4096, True), (128, 3840, 15360, True),
                                               (100, 320, 96, False), (37, 256, 224, True), (512, 1024, 1920, True)])
 def test_w4a16_normadd_equals_gemm_then_normadd(gpu, M, N, K, fuse_norm):
