@@ -640,18 +640,10 @@ __device__ inline uint32_t mm_scale(const uint8_t* sbase, uint32_t voff) {
   else return ld1_so(sbase, voff);
 }
 
-// Waves per workgroup of T tiles. 8 (two per SIMD) at T = 4, where a grid is
-// one workgroup per CU and a wave's transposes, dequant and dependent MFMAs
-// stall it between loads: 15360 x 3840, 8 vectors 9.75 -> 9.15 us, 3840 x 15360
-// in 4 splits 11.7 -> 11.4. With fewer tiles a wave has few steps: 4 (3840 x
-// 8192 8.2 us, 8.6 with 8 waves).
-__host__ __device__ constexpr int mm_waves(int T) { return T == 4 ? 8 : 4; }
-
-template <int T, int U, int ST, int YT>
-__global__ void __launch_bounds__(64 * mm_waves(T))
+template <int T, int U, int W, int ST, int YT>
+__global__ void __launch_bounds__(64 * W)
 gemv_mm_kernel(const uint16_t* __restrict__ X, int M, const uint8_t* __restrict__ wq, const void* __restrict__ scv,
                float outscale, void* __restrict__ Y, int N, int nblk, int kspan, float* __restrict__ part) {
-  constexpr int W = mm_waves(T);                  // waves per workgroup
   constexpr int BPS = 4 / T;                      // blocks per step
   constexpr int L = BPS + 2;                      // loads per step: x slices, the unit and its scale
   constexpr int SB = ST == Q4_SCALE_F16 ? 2 : 1;  // scale bytes
@@ -974,21 +966,35 @@ static gemv_multi_fn pick_mv(int R, int U, int mv, int st, int yt) {
 }
 
 typedef void (*gemv_mm_fn)(const uint16_t*, int, const uint8_t*, const void*, float, void*, int, int, int, float*);
-template <int T, int U>
+template <int T, int U, int W>
 static gemv_mm_fn pick_mm_sy(int st, int yt) {
   if (st == Q4_SCALE_E4M3)
-    return yt == Q4_DT_F16 ? gemv_mm_kernel<T, U, Q4_SCALE_E4M3, Q4_DT_F16> : gemv_mm_kernel<T, U, Q4_SCALE_E4M3, Q4_DT_F32>;
-  return yt == Q4_DT_F16 ? gemv_mm_kernel<T, U, Q4_SCALE_F16, Q4_DT_F16> : gemv_mm_kernel<T, U, Q4_SCALE_F16, Q4_DT_F32>;
+    return yt == Q4_DT_F16 ? gemv_mm_kernel<T, U, W, Q4_SCALE_E4M3, Q4_DT_F16>
+                           : gemv_mm_kernel<T, U, W, Q4_SCALE_E4M3, Q4_DT_F32>;
+  return yt == Q4_DT_F16 ? gemv_mm_kernel<T, U, W, Q4_SCALE_F16, Q4_DT_F16>
+                         : gemv_mm_kernel<T, U, W, Q4_SCALE_F16, Q4_DT_F32>;
 }
-// (T, U) pairs built: U = 4 or the deepest ring whose U (4/T + 5) loads
-// per step stay under the 63 the wait count can express (T = 1: 6,
-// T = 2: 8, T = 4: 10); the deeper one is the default.
-static gemv_mm_fn pick_mm(int T, bool deep, int st, int yt) {
+// (T, U) pairs built: U = 4 steps of 4 / T + 2 loads in flight, the default,
+// or a deeper ring (T = 1: 6, T = 2: 8, T = 4: 10), slower at every decode
+// shape (by 0.3 to 1.5 us).
+static gemv_mm_fn pick_mm(int T, int W, bool deep, int st, int yt) {
   switch (T) {
-    case 4: return deep ? pick_mm_sy<4, 10>(st, yt) : pick_mm_sy<4, 4>(st, yt);
-    case 2: return deep ? pick_mm_sy<2, 8>(st, yt) : pick_mm_sy<2, 4>(st, yt);
-    default: return deep ? pick_mm_sy<1, 6>(st, yt) : pick_mm_sy<1, 4>(st, yt);
+    case 4:
+      if (W == 8) return deep ? pick_mm_sy<4, 10, 8>(st, yt) : pick_mm_sy<4, 4, 8>(st, yt);
+      return deep ? pick_mm_sy<4, 10, 4>(st, yt) : pick_mm_sy<4, 4, 4>(st, yt);
+    case 2: return deep ? pick_mm_sy<2, 8, 4>(st, yt) : pick_mm_sy<2, 4, 4>(st, yt);
+    default: return deep ? pick_mm_sy<1, 6, 4>(st, yt) : pick_mm_sy<1, 4, 4>(st, yt);
   }
+}
+// Waves per workgroup: 8 (two per SIMD) at T = 4 where a grid is about one
+// workgroup per CU and a wave has enough steps: its transposes, dequant and
+// dependent MFMAs stall it between loads. 4 / 8 waves: 15360 x 3840 8.8 / 8.4 us
+// with 4 vectors, 9.05 / 8.8 with 12, 9.13 / 9.38 with 16 (the x reads bound it);
+// 15360 x 512 3.9 / 4.1; 3840 x 15360 in 4 splits 11.5 / 11.1; two workgroups per
+// CU have two waves per SIMD as it is (30720 x 3840 14.7 / 15.1; 4800 x 12288, 300
+// workgroups, 13.2 / 13.7). With fewer tiles a wave has few steps: 4.
+static int mm_waves(int T, int M, int blocks, int wgs) {
+  return T == 4 && M <= 12 && blocks >= 64 && wgs <= 256 ? 8 : 4;
 }
 // Row tiles of 16 per workgroup for NP padded rows: the largest T of 4, 2, 1
 // that still gives GEMV_MIN_WGS workgroups (about one per CU): the x slices
@@ -1002,29 +1008,27 @@ static int mm_tiles(int NP) {
   if (v == 1 || v == 2 || v == 4) T = v;
   return T;
 }
-// K splits for the small-M GEMV at T = 4 tiles: 1 where NP / 64 row groups
-// already give GEMV_MIN_WGS workgroups, else enough splits to reach it, each
-// split at least GEMV_MM_MIN_SPLIT_BLOCKS blocks (8 steps per wave).
+// K splits of the small-M GEMV (the workspace query and the launch both ask
+// here): 1 where NP / 64 row groups already give GEMV_MIN_WGS workgroups or K
+// is short, else enough splits at T = 4 tiles to reach them, each at least
+// GEMV_MM_MIN_SPLIT_BLOCKS blocks. Partials and the reduce launch cost more
+// than filling the chip saves up to 256 blocks; with more than 10 vectors (14
+// from 7680 rows on, where two tiles share the x), all of whose x every
+// workgroup reads, up to 128, and with few rows up to 192.
+// Split / unsplit, per launch in a graph: 4096 x 3840 7.2 / 5.7 us with 8 vectors,
+// 7.7 / 6.8 with 16; 2048 x 6144 7.8 / 6.8, 16: 8.0 / 8.6; 3840 x 8192 8.6 / 8.0, 12:
+// 8.6 / 9.2, 16: 8.9 / 10.4; 8192 x 8192, 12: 11.9 / 11.2; 512 x 6144 6.8 / 6.5; 512 x 8192 with 2 6.8 / 7.4;
+// 3840 x 15360 11.1 / 13.1.
 // The Q4_TUNE_GEMV_MM_SPLIT override (q4_tune_set) replaces it in tests and sweeps.
 constexpr int GEMV_MM_MIN_SPLIT_BLOCKS = 32;
-static int mm_split(int NP, int nblk) {
-  const int groups = NP / 64;
-  int s = groups >= GEMV_MIN_WGS ? 1 : (GEMV_MIN_WGS + groups - 1) / groups;
-  s = std::min(s, std::max(1, nblk / GEMV_MM_MIN_SPLIT_BLOCKS));
-  const int v = tune_value(Q4_TUNE_GEMV_MM_SPLIT);
+static int mm_split(int M, int NP, int nblk) {
+  const int groups = NP / 64, v = tune_value(Q4_TUNE_GEMV_MM_SPLIT);
+  int s = groups >= GEMV_MIN_WGS || nblk <= (M > (NP >= 7680 ? 14 : 10) ? 128 : NP >= 1024 ? 256 : 192)
+              ? 1
+              : std::min((GEMV_MIN_WGS + groups - 1) / groups, nblk / GEMV_MM_MIN_SPLIT_BLOCKS);
   if (v >= 1 && v <= 64) s = v;
   const int span = (nblk + s - 1) / s;
   return (nblk + span - 1) / span;  // no empty split
-}
-// K splits a launch uses (mm_split sizes the workspace): the partials and the
-// reduce launch cost more than filling the chip saves up to
-// GEMV_MM_UNSPLIT_BLOCKS blocks. 8 vectors, split / unsplit, per launch in a
-// graph: 4096 x 3840 7.0 / 5.8 us, 2048 x 3840 7.0 / 5.6, 8192 x 3840 7.3 / 6.4,
-// 3840 x 4096 7.0 / 5.6, 3840 x 8192 8.6 / 8.2, 3840 x 15360 11.6 / 13.1.
-constexpr int GEMV_MM_UNSPLIT_BLOCKS = 256;
-static int mm_launch_split(int NP, int nblk) {
-  if (tune_value(Q4_TUNE_GEMV_MM_SPLIT) < 0 && nblk <= GEMV_MM_UNSPLIT_BLOCKS) return 1;
-  return mm_split(NP, nblk);
 }
 static bool mm_deep() { return tune_value(Q4_TUNE_GEMV_MM_DEEP) > 0; }
 
@@ -1360,15 +1364,15 @@ static int gemv_mm_launch(const void* x, int M, const uint32_t* wq, const void* 
                           hipStream_t st) {
   const int NP = pad_rows(N);
   if (split <= 1) {
-    const int T = mm_tiles(NP);
-    hipLaunchKernelGGL(pick_mm(T, mm_deep(), scale_fmt, y_dtype), dim3(NP / (16 * T)), dim3(64 * mm_waves(T)), 0, st,
+    const int T = mm_tiles(NP), wgs = NP / (16 * T), W = mm_waves(T, M, nblk, wgs);
+    hipLaunchKernelGGL(pick_mm(T, W, mm_deep(), scale_fmt, y_dtype), dim3(wgs), dim3(64 * W), 0, st,
                        reinterpret_cast<const uint16_t*>(x), M, reinterpret_cast<const uint8_t*>(wq), scales,
                        outscale, y, N, nblk, nblk, nullptr);
     Q4_LAUNCHED("gemv_mm");
     return Q4_OK;
   }
-  const int span = (nblk + split - 1) / split;
-  hipLaunchKernelGGL(pick_mm(4, mm_deep(), scale_fmt, y_dtype), dim3(NP / 64, split), dim3(64 * mm_waves(4)), 0, st,
+  const int span = (nblk + split - 1) / split, W = mm_waves(4, M, span, NP / 64 * split);
+  hipLaunchKernelGGL(pick_mm(4, W, mm_deep(), scale_fmt, y_dtype), dim3(NP / 64, split), dim3(64 * W), 0, st,
                      reinterpret_cast<const uint16_t*>(x), M, reinterpret_cast<const uint8_t*>(wq), scales, outscale,
                      y, N, nblk, span, ws);
   Q4_LAUNCHED("gemv_mm split");
@@ -1402,7 +1406,7 @@ static int gemv_multi_check(const void* x, int M, const uint32_t* wq, const void
 size_t q4_gemv_multi_workspace_bytes(int M, int N, int K) {
   if (M < 1 || M > Q4_GEMV_MAX_VECTORS || N <= 0 || K <= 0 || K % BLK || N > (1 << 30) || (long)K > (1L << 24))
     return 0;
-  const int split = mm_split(pad_rows(N), K / BLK);
+  const int split = mm_split(M, pad_rows(N), K / BLK);
   return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
 }
 
@@ -1414,7 +1418,7 @@ int q4_gemv_multi_ws(const void* x, int M, const uint32_t* wq, const void* scale
   const int nblk = K / BLK;
   const float outscale = scale_fmt == Q4_SCALE_E4M3 ? inv * 256.0f : 1.0f;
   const size_t need = q4_gemv_multi_workspace_bytes(M, N, K);
-  const int split = need && ws && ws_size >= need ? mm_launch_split(pad_rows(N), nblk) : 1;
+  const int split = need && ws && ws_size >= need ? mm_split(M, pad_rows(N), nblk) : 1;
   return gemv_mm_launch(x, M, wq, scales, scale_fmt, outscale, y, y_dtype, N, nblk, split,
                         split > 1 ? reinterpret_cast<float*>(ws) : nullptr, as_stream(stream));
 }

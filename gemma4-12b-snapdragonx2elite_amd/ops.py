@@ -238,12 +238,12 @@ def gemv_multi(x: torch.Tensor, wq: torch.Tensor, scales: torch.Tensor, N: int, 
                ksplit: bool = True) -> torch.Tensor:
     """Y[m] = GEMV of x[m] for the M fp16 rows of ``x`` [M][K] (M <= 16),
     reading the weights once. ``exact``: every row bit-identical to
-    :func:`gemv` of that row when :func:`gemv` runs unsplit (VALU path, one
+    :func:`gemv` of that row for N >= 1920 (VALU path, one
     weight stream per 2-8 vectors); otherwise the MFMA path, equal to
     :func:`gemv` to fp32 rounding: one launch, or for matrices of fewer than
-    15360 rows and K >= 2048 a K-split launch into fp32 partials plus their
-    reduce — pass
-    ``ws`` (at least :func:`gemv_multi_workspace_bytes` bytes) or one is
+    15360 rows and a long K a K-split launch into fp32 partials plus their
+    reduce, where :func:`gemv_multi_workspace_bytes` is not 0 — pass
+    ``ws`` (at least that many bytes) or one is
     allocated here; capture code must pass its own. ``ksplit=False`` runs
     the MFMA path unsplit whatever the shape. Returns Y [M][N]."""
     if x.dtype != torch.float16:

@@ -97,6 +97,16 @@ def test_argument_errors_without_gpu(g4):
     assert lib.q4_gemv_multi_workspace_bytes(17, 3840, 15360) == 0
 
 
+@pytest.mark.parametrize("M,N,K,split", [(16, 3840, 4096, 1), (11, 3840, 4128, 4), (10, 3840, 4128, 1),
+                                         (10, 3840, 8192, 1), (10, 3840, 8224, 4), (10, 1024, 8192, 1),
+                                         (10, 960, 6144, 1), (10, 960, 6176, 6), (11, 3840, 8192, 4), (14, 7680, 8192, 1), (15, 7680, 8192, 2)])
+def test_small_m_workspace_follows_the_launch(g4, M, N, K, split):
+    """The workspace query names the splits that the launch uses: nothing
+    where K is not split, on both sides of each bound of the rule."""
+    need = g4._lib.lib().q4_gemv_multi_workspace_bytes(M, N, K)
+    assert need == (split * M * N * 4 if split > 1 else 0)
+
+
 def test_prefill_op_argument_errors_without_gpu(g4):
     lib = g4._lib.lib()
     p = C.c_void_p(1 << 20)

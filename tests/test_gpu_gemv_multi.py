@@ -207,3 +207,27 @@ def test_gemv_multi_ksplit_down_shape_reuses_workspace(gpu):
         ref = O.gemm_w4a16_ref(X, q, s)
         for m in range(M):
             assert O.normwise_rel_err(to_np(Y[m]), ref[m]) <= TOL[torch.float32], (M, m)
+
+
+@pytest.mark.parametrize("N,K,M", [(3840, 4096, 16), (3840, 4128, 11),    # the longest unsplit K above 10 vectors, and past it
+                                   (1024, 8192, 10), (960, 8192, 10),     # few rows split earlier
+                                   (3840, 8224, 10),                      # past the longest unsplit K
+                                   (15360, 2048, 12), (15360, 2048, 13),  # 8 and 4 waves
+                                   (15360, 2016, 5), (16400, 2080, 7),    # 63 blocks; 257 workgroups: 4 waves
+                                   (3840, 16384, 12), (3840, 16384, 16)]) # split spans of 128 blocks, 8 and 4 waves
+def test_gemv_multi_split_and_wave_rules(gpu, N, K, M):
+    """Both sides of the rules for K splits and waves per workgroup, fp16 and
+    e4m3 scales, against the single GEMV (TOL: fp32 sums in another order),
+    without a workspace and with the one the query names."""
+    rng = np.random.default_rng(N + K + M)
+    q, s = synth_int4(rng, N, K)
+    wq, sc = upload_int4(q, s)
+    sc8, inv = gpu.scales_e4m3(torch.from_numpy(s).cuda(), N, K)
+    Xd = torch.from_numpy(_x(rng, M, K)).cuda()
+    for kw in (dict(), dict(scale_fmt=gpu.SCALE_E4M3, inv=inv)):
+        sca = sc8 if kw else sc
+        ref = torch.stack([gpu.gemv(Xd[m].contiguous(), wq, sca, N, K, y_dtype=torch.float32, **kw) for m in range(M)])
+        for ks in (True, False):
+            Y = gpu.gemv_multi(Xd, wq, sca, N, K, y_dtype=torch.float32, ksplit=ks, **kw)
+            for m in range(M):
+                assert O.normwise_rel_err(to_np(Y[m]), to_np(ref[m])) <= TOL[torch.float32], (m, ks, kw)
