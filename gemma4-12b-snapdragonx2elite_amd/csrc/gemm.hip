@@ -1802,15 +1802,17 @@ static int w4a16_kgroups(int M, int N, int K, int split) {
 //    (M 17, 4096 x 3840: 17.2 -> 15.3 us, wide 16.8), or for grids under 64
 //    workgroups of up to three splits, which then grow to 128 (M 77, 1000 x
 //    4032: 18.4 -> 15.4, wide 17.8; M 64, 6000 x 1600: 18.1 -> 16.4, wide
-//    17.8; from four splits on it loses: M 100, 1040 x 8000 19.5 -> 20.4). One
-//    split stays one where a second kernel would sum large partials whose odd
-//    rows are stored and read element by element (M 219, 2951 x 1120 16.0 ->
-//    20.0; M 68, 985 x 1920 20.0 -> 14.8).
+//    17.8; from four splits on it loses: M 100, 1040 x 8000 19.5 -> 20.4).
+//    Partials of an N that is no multiple of 4 are stored and read element by
+//    element: above 40000 outputs their groups stay at 8 (M 41, 1274 x 7520
+//    20.5, with 4 22.8), and above 100000 one split stays one (M 219, 2951 x
+//    1120 16.0, two splits 20.0; M 68, 985 x 1920 20.0, three splits 14.8).
 // The narrow plan is taken where its groups run fewer k-steps than the wide
 // plan's waves, where it leaves no second kernel, or where the partials it
-// saves (~0.1 us per split and 0.8 us per million fp32 values) are worth the
-// second read of A in its loop (~0.045 us per k-step): with few rows they are
-// not (M 1, 16000 x 8000 37.8 us, wide 35.9; even at M 64).
+// saves (~0.1 us per split and 0.8 us per million fp32 values, element by
+// element 4 times that) are worth the second read of A in its loop (~0.045 us
+// per k-step): with few rows they are not (M 1, 16000 x 8000 37.8 us, wide
+// 35.9; even at M 64; M 20, 15042 x 7424 47.1, wide 50.2).
 struct W4Plan {
   int split, bm, kg;
   bool narrow;
@@ -1822,12 +1824,14 @@ static W4Plan w4a16_plan(int M, int N, int K) {
   if (!tuned && p.bm == 128 && p.kg == 1 && p.split > 1) {
     const int nk = (K / 32 + 1) / 2, t = ceil_div(M, 128) * ceil_div(N, 128);
     const int round = max(1, 256 / t);
-    int s = min(round, nk / (M <= 48 ? 8 : 16));
-    if (t * s < 64 && s < 4 && (s > 1 || N % 4 == 0 || (long)M * N <= 100000))
+    const long mn = (long)M * N;
+    const bool odd = N % 4 != 0;  // partials stored and read element by element
+    int s = min(round, nk / (M <= 48 && (!odd || mn <= 40000) ? 8 : 16));
+    if (t * s < 64 && s < 4 && (s > 1 || !odd || mn <= 100000))
       s = max(s, min(min(round, 128 / t), nk / 8));
     s = min(s, p.split);
     const bool shorter = 4 * s >= 3 * p.split;  // nk / (2 s) k-steps per group against nk / split
-    const long saved = ((long)M * N + 125000) * (p.split - s), reread = 56000L * ceil_div(nk, 2 * s);
+    const long saved = ((odd ? 4 : 1) * mn + 125000) * (p.split - s), reread = 56000L * ceil_div(nk, 2 * s);
     if (shorter || s == 1 || saved >= reread) p = W4Plan{s, 128, 2, true};
   }
   return p;
