@@ -11,42 +11,49 @@
 namespace q4 {
 
 // ---- int4 block quantizer (src/vk_engine.py:126-131) ---------------------
-// A workgroup quantizes 64 rows (one panel) x 8 blocks; each wave takes 16
-// rows, one row's 8 blocks (1 KB) per load, all 16 loads requested before the
-// first is used: lane l holds 4 consecutive elements of block l / 8, the
+// A workgroup quantizes 64 rows (one panel) x QB blocks; each wave takes 16
+// rows, 8 / QB rows' blocks (1 KB) per load, all 2 QB loads requested before
+// the first is used: 8 lanes hold a block, 4 consecutive elements each, the
 // block's maximum is an 8-lane reduction, and lane pairs join their nibbles
 // to device words. Units and fp16 scales go through LDS to the panel order
 // (64 rows of a block contiguous), fp32 scales are stored from the lanes.
-// Bound by the read of W: 15360 x 3840 (236 MB in, 41 MB out) 72.6 -> 59.6 us
+// Bound by the read of W: 15360 x 3840 (236 MB in, 41 MB out) 73.4 -> 63.2 us
 // against a thread per block, whose 16-byte loads of a wave lay 64 rows apart.
+// QB = 4 reads whole 512-byte runs of a row; with QB = 1 four times the
+// workgroups run a quarter of the chain each, better up to QUANT_SMALL values
+// (QB 4 / 1 / a thread per block, W not in cache: 64 x 3840 5.8 / 4.3 / 5.1 us, 1000
+// x 3840 8.5 / 7.1 / 7.3, 4000 x 3840 21.1 / 21.0 / 22.0, 8000 x 3840 34.6 / 38.4 /
+// 40.0).
 // The code is rint(v / sc) of the correctly rounded quotient; v times the
 // approximate reciprocal differs from it by less than 2e-6 (|v / sc| <= 7,
 // three roundings and the 1-ulp reciprocal), so only values that close to a
 // rounding tie, or not finite, take the division.
-constexpr int QB = 8;   // blocks per workgroup tile
+constexpr long QUANT_SMALL = 24L << 20;
+template <int QB>
 __global__ void __launch_bounds__(256) quantize_kernel(const float* __restrict__ W, int N, int K, int nblk,
                                                        uint4* __restrict__ wq, uint16_t* __restrict__ sc16,
                                                        float* __restrict__ sc32) {
-  constexpr int RW = 16;  // rows per wave
+  constexpr int LPR = 8 * QB, RL = 64 / LPR, NL = 16 / RL;  // lanes per row, rows per load, loads per wave
   __shared__ __attribute__((aligned(16))) uint32_t words[PANEL][QB * 4 + 4];
   __shared__ uint16_t scs[QB][PANEL];
   const int ct = ceil_div(nblk, QB);
   const int p = blockIdx.x / ct, b0 = (blockIdx.x % ct) * QB;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lb = lane >> 3;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lr = lane / LPR, lc = lane % LPR, lb = lc >> 3;  // the lane's row of a load, place in the row, block
   const int b = b0 + lb;
   const bool bok = b < nblk;
-  float4 v[RW];
+  float4 v[NL];
 #pragma unroll
-  for (int i = 0; i < RW; ++i) {
-    const int n = p * PANEL + wave * RW + i;
-    v[i] = bok && n < N ? *reinterpret_cast<const float4*>(W + (long)n * K + (long)b0 * BLK + 4 * lane)
+  for (int i = 0; i < NL; ++i) {
+    const int n = p * PANEL + wave * 16 + i * RL + lr;
+    v[i] = bok && n < N ? *reinterpret_cast<const float4*>(W + (long)n * K + (long)b0 * BLK + 4 * lc)
                         : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   }
   // nibble shifts of this lane's elements e = 4 (lane & 1) + c of its word
   const int odd = lane & 1;
 #pragma unroll
-  for (int i = 0; i < RW; ++i) {
-    const int r = wave * RW + i, n = p * PANEL + r;
+  for (int i = 0; i < NL; ++i) {
+    const int r = wave * 16 + i * RL + lr, n = p * PANEL + r;
     const float x[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
     const float amax = reduce8<true>(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
     const float sc = fmaxf(__fdiv_rn(amax, 7.0f), 1e-8f);
@@ -70,7 +77,7 @@ __global__ void __launch_bounds__(256) quantize_kernel(const float* __restrict__
     w <<= 8 * odd;   // elements 4..7 sit two nibbles above 0..3
     w |= __float_as_uint(dpp_f<DPP_XOR1>(__uint_as_float(w)));
     const bool live = n < N;
-    if (!odd) words[r][lane >> 1] = live ? w : 0x88888888u;   // padded row: code 8 (= weight 0), scale 0
+    if (!odd) words[r][lc >> 1] = live ? w : 0x88888888u;   // padded row: code 8 (= weight 0), scale 0
     if ((lane & 7) == 0) {
       scs[lb][r] = live ? f2h_after_f32(sc) : (uint16_t)0;
       if (sc32 && live && bok) sc32[(long)n * nblk + b] = sc;
@@ -375,10 +382,11 @@ int q4_quantize(const float* W, int N, int K, uint32_t* wq, uint16_t* sc16, floa
   Q4_ARG(W && wq && sc16, "null pointer");
   Q4_ARG(((uintptr_t)W & 15) == 0 && ((uintptr_t)wq & 15) == 0, "W and wq must be 16-byte aligned");
   const int nblk = K / BLK;
-  const long wgs = (long)(pad_rows(N) / PANEL) * ceil_div(nblk, QB);
+  const bool small = (long)N * K <= QUANT_SMALL;
+  const long wgs = (long)(pad_rows(N) / PANEL) * (small ? nblk : ceil_div(nblk, 4));
   Q4_ARG(wgs < (1L << 31), "matrix too large");
-  hipLaunchKernelGGL(quantize_kernel, dim3((unsigned)wgs), dim3(256), 0, as_stream(stream), W, N, K, nblk,
-                     reinterpret_cast<uint4*>(wq), sc16, sc32);
+  hipLaunchKernelGGL(small ? quantize_kernel<1> : quantize_kernel<4>, dim3((unsigned)wgs), dim3(256), 0,
+                     as_stream(stream), W, N, K, nblk, reinterpret_cast<uint4*>(wq), sc16, sc32);
   Q4_LAUNCHED("quantize");
   return Q4_OK;
 }

@@ -127,3 +127,24 @@ def test_quantizer_and_fold_edges_bit_exact(gpu, N, K, kind):
     e8, inv_ref, _ = O.e4m3_lift(sc)
     assert inv == inv_ref
     assert (to_np(sc8).reshape(-1) == O.scales_dev(e8).view(np.uint8).reshape(-1)).all()
+
+
+def test_quantizer_large_matrix_bit_exact(gpu):
+    """A matrix past the small tile's 24 M values: partial last panel and a
+    last tile of one block, with values on the rounding ties; codes and scales
+    equal numpy's bit for bit, and so does the same matrix cut into small ones."""
+    N, K = 6700, 4000
+    rng = np.random.default_rng(3)
+    W = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    W[:, 64:96] = np.round(W[:, 64:96] * 70) / 2   # multiples of 0.5 with a maximum of 7: ties
+    W[:, 64] = 7.0
+    q, sc = O.quant_codes(W)
+    wq, sc16, sc32 = gpu.quantize(torch.from_numpy(W).cuda())
+    assert (to_np(wq).view(np.uint32).reshape(-1) == O.pack_dev(q).view(np.uint32).reshape(-1)).all()
+    assert (to_np(sc32).view(np.uint32) == sc.view(np.uint32)).all()
+    assert (to_np(sc16).view(np.uint16).reshape(-1) == O.scales_dev(sc.astype(np.float16)).view(np.uint16).reshape(-1)).all()
+    for r0, r1 in ((0, 3328), (3328, 6700)):
+        w2, s2, _ = gpu.quantize(torch.from_numpy(W[r0:r1]).cuda())
+        u = K // 32 * 64   # units of a panel
+        p0, p1 = r0 // 64, -(-r1 // 64)
+        assert torch.equal(w2, wq[p0 * u * 4:p1 * u * 4]) and torch.equal(s2, sc16[p0 * u:p1 * u])
