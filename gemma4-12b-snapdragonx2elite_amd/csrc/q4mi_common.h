@@ -212,14 +212,15 @@ __device__ inline float reduce64(float v) {
   return red_op<MAX>(__uint_as_float(p[0]), __uint_as_float(p[1]));
 }
 
-// Sum (or max) over lanes l, l + R, l + 2R, .. (R = 4, 8, 16, 32, 64), valid
+// Sum (or max) over lanes l, l + R, l + 2R, .. (R = 2, 4, 8, 16, 32, 64), valid
 // in lanes l < R (with R = 16 or 32, in every lane): the xor-8, xor-16,
 // xor-32 pairings of a shuffle loop, each own + partner (so the bits equal
 // those of that loop), on VALU: DPP row rotate by 8 within 16 lanes, then
 // the permlane16 and permlane32 swaps.
 template <int R, bool MAX = false>
 __device__ inline float slot_reduce(float v) {
-  static_assert(R == 4 || R == 8 || R == 16 || R == 32 || R == 64, "slot width");
+  static_assert(R == 2 || R == 4 || R == 8 || R == 16 || R == 32 || R == 64, "slot width");
+  if constexpr (R <= 2) v = red_op<MAX>(v, dpp_f<0x122>(v));  // row_ror:2
   if constexpr (R <= 4) v = red_op<MAX>(v, dpp_f<0x124>(v));  // row_ror:4, with ror:8 below all four of a row
   if constexpr (R <= 8) v = red_op<MAX>(v, dpp_f<0x128>(v));  // row_ror:8 = lane ^ 8 within 16
   if constexpr (R <= 16) {

@@ -173,18 +173,23 @@ __global__ void __launch_bounds__(256) e4m3_lift_kernel(const float* __restrict_
 }
 
 // ---- W8A8 fold (src/vk_engine.py:152-157) --------------------------------
-// A workgroup folds 8 rows: thread (r = t % 8, block t / 8 + 32 i), so the 8
-// rows of a block are one 128-byte line of units, read by one workgroup (a
-// workgroup per row fetched every line into the L2 of all 8 XCDs). The row
-// maximum needs only the block's largest |code| (products round
-// monotonically). The 32 quotients of a block take 9 values: k s for k = 0..8
-// with either sign, so a thread rounds 8 quotients, packs the 16 codes' bytes
-// into 4 words and looks the codes up with byte permutes. W8 is row-major
+// A workgroup folds FR rows: thread (r = t % FR, block t / FR + 256 / FR i). With
+// FR = 8 the 8 rows of a block are one 128-byte line of units, read by one
+// workgroup (a workgroup per row fetched every line into the L2 of all 8
+// XCDs). The row maximum needs only the block's largest |code| (products
+// round monotonically). The 32 quotients of a block take 9 values: k s for k =
+// 0..8 with either sign, so a thread rounds 8 quotients, packs the 16 codes'
+// bytes into 4 words and looks the codes up with byte permutes. W8 is row-major
 // [N][K] or, PACKED, the layout of the packed W8A8 GEMM (1 KB per 32 rows x
 // 32 k: 16-byte chunk l is row l % 32, k half l / 32; rows padded to 32 and
 // K to 128 with zeros), which saves the pass that packs it.
 // 15360 x 3840: 59.6 us for the row-major fold and 18.3 for its packing
-// before, 24.1 us in one pass (96 MB).
+// before, 24.1 us in one pass (96 MB). Below FOLD_ROWS rows 8-row workgroups
+// do not fill the chip and each is a long chain of rounds: FR = 2 (8 / 2, and a
+// workgroup per row: 8 x 3840 6.4 / 4.3 / 4.8 us, 300 x 15360 18.9 / 7.7 / 11.3, 1000 x
+// 3840 7.1 / 5.8 / 9.4, 1000 x 15360 20.0 / 13.0 / 26.5, 2000 x 3840 7.9 / 7.5 / 13.2,
+// packed 7.5 / 8.7).
+constexpr int FOLD_ROWS = 1536;
 __device__ inline uint32_t fold_byte(float v) {
   return (uint32_t)(int)fminf(fmaxf(v, -127.0f), 127.0f) & 0xFFu;
 }
@@ -195,12 +200,12 @@ __device__ inline uint32_t fold_lookup(uint32_t c, const uint32_t (&t)[4]) {
   return __builtin_amdgcn_perm(hi, lo, ((c >> 1) & 0x04040404u) | 0x03020100u);  // byte i of hi where bit 3 is set
 }
 
-template <bool PACKED>
+template <bool PACKED, int FR>
 __global__ void __launch_bounds__(256) w8_fold_kernel(const uint4* __restrict__ wq, const float* __restrict__ sc32,
                                                       int N, int K, int nblk, int8_t* __restrict__ W8,
                                                       float* __restrict__ sw32, uint16_t* __restrict__ sw16,
                                                       int kslices) {
-  constexpr int FR = 8, FB = 256 / FR;
+  constexpr int FB = 256 / FR;
   __shared__ float red[4][FR];
   const int r = threadIdx.x & (FR - 1), n = blockIdx.x * FR + r, bt = threadIdx.x / FR;
   const bool live = n < N;
@@ -225,7 +230,7 @@ __global__ void __launch_bounds__(256) w8_fold_kernel(const uint4* __restrict__ 
     const int far = max(max((int)mx.x, (int)mx.y) - 8, 8 - min((int)mn.x, (int)mn.y));
     amax = fmaxf(amax, fabsf(__fmul_rn((float)far, s)));
   }
-  amax = slot_reduce<8, true>(amax);
+  amax = slot_reduce<FR, true>(amax);
   if ((threadIdx.x & 63) < FR) red[threadIdx.x >> 6][r] = amax;
   __syncthreads();
   amax = fmaxf(fmaxf(red[0][r], red[1][r]), fmaxf(red[2][r], red[3][r]));
@@ -415,8 +420,9 @@ int q4_w8_fold(const uint32_t* wq, const float* sc32, int N, int K, int8_t* W8, 
   if (int st = check_wk(N, K)) return st;
   Q4_ARG(wq && sc32 && W8, "null pointer");
   Q4_ARG(((uintptr_t)W8 & 15) == 0 && ((uintptr_t)wq & 15) == 0, "W8 and wq must be 16-byte aligned");
-  hipLaunchKernelGGL(w8_fold_kernel<false>, dim3(ceil_div(N, 8)), dim3(256), 0, as_stream(stream),
-                     reinterpret_cast<const uint4*>(wq), sc32, N, K, K / BLK, W8, sw32, sw16, 0);
+  const bool few = N < FOLD_ROWS;
+  hipLaunchKernelGGL((few ? w8_fold_kernel<false, 2> : w8_fold_kernel<false, 8>), dim3(ceil_div(N, few ? 2 : 8)),
+                     dim3(256), 0, as_stream(stream), reinterpret_cast<const uint4*>(wq), sc32, N, K, K / BLK, W8, sw32, sw16, 0);
   Q4_LAUNCHED("w8_fold");
   return Q4_OK;
 }
@@ -429,8 +435,9 @@ int q4_w8_fold_packed(const uint32_t* wq, const float* sc32, int N, int K, int8_
   Q4_ARG(((uintptr_t)W8p & 15) == 0 && ((uintptr_t)wq & 15) == 0, "W8p and wq must be 16-byte aligned");
   const int rows = ceil_div(N, 32) * 32;
   const int kslices = (int)(q4_w8_packed_bytes(N, K) / ((size_t)rows * 32));
-  hipLaunchKernelGGL(w8_fold_kernel<true>, dim3(rows / 8), dim3(256), 0, as_stream(stream),
-                     reinterpret_cast<const uint4*>(wq), sc32, N, K, K / BLK, W8p, sw32, sw16, kslices);
+  const bool few = N < FOLD_ROWS;
+  hipLaunchKernelGGL((few ? w8_fold_kernel<true, 2> : w8_fold_kernel<true, 8>), dim3(rows / (few ? 2 : 8)), dim3(256), 0,
+                     as_stream(stream), reinterpret_cast<const uint4*>(wq), sc32, N, K, K / BLK, W8p, sw32, sw16, kslices);
   Q4_LAUNCHED("w8_fold_packed");
   return Q4_OK;
 }

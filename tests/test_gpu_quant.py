@@ -148,3 +148,19 @@ def test_quantizer_large_matrix_bit_exact(gpu):
         u = K // 32 * 64   # units of a panel
         p0, p1 = r0 // 64, -(-r1 // 64)
         assert torch.equal(w2, wq[p0 * u * 4:p1 * u * 4]) and torch.equal(s2, sc16[p0 * u:p1 * u])
+
+
+@pytest.mark.parametrize("N,K", [(1, 15360), (7, 15392), (1535, 288), (1536, 288), (1543, 4160)])
+def test_fold_row_groups_bit_exact(gpu, N, K):
+    """Both sides of the fold's row bound, odd row counts and one block past
+    whole rounds of a workgroup (15360 / 32 = 480 blocks): numpy's bytes, and
+    the packed form equals fold then pack."""
+    rng = np.random.default_rng(N + K)
+    W = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    q, sc = O.quant_codes(W)
+    wq, _, sc32 = gpu.quantize(torch.from_numpy(W).cuda())
+    W8, sw = O.w8_fold(q, sc)
+    gW8, gsw32, gsw16 = gpu.w8_fold(wq, sc32, N, K)
+    assert (to_np(gW8) == W8).all() and (to_np(gsw32).view(np.uint32) == sw.view(np.uint32)).all()
+    pW8, psw32, psw16 = gpu.w8_fold_packed(wq, sc32, N, K)
+    assert torch.equal(pW8, gpu.w8_pack(gW8)) and torch.equal(psw32, gsw32) and torch.equal(psw16, gsw16)
