@@ -33,6 +33,7 @@ constexpr int NORM_THREADS = 1024;
 constexpr int ATT_THREADS = 256;
 constexpr int ATT_KPW = 8;        // keys per wave of an attention split (one K row per 8 lanes)
 constexpr int ATT_HPW = 4;        // query heads per attention workgroup (at most)
+constexpr int ATT_MERGE_PF = 8;   // splits per wave that the 8-wave merge loads before the position is known
 constexpr int ATT_MMH = 16;       // query heads per workgroup of the matrix-core attention split
 constexpr int ATT_MAX_HD = 512;   // head dims up to 512 (global layers)
 
@@ -477,9 +478,10 @@ __device__ inline HalfVec<E> ld_halves(const uint16_t* p) {
 // then lands in order with the kernel's other vector loads. As a scalar
 // load it shares lgkmcnt with the kernel-argument loads issued after it,
 // and their wait would put its round trip before every later load.
-__device__ inline uint32_t load_pos(const uint32_t* dyn) {
-  return __builtin_amdgcn_readfirstlane(__hip_atomic_load(dyn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+__device__ inline uint32_t load_pos_lane(const uint32_t* dyn) {
+  return __hip_atomic_load(dyn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ inline uint32_t load_pos(const uint32_t* dyn) { return __builtin_amdgcn_readfirstlane(load_pos_lane(dyn)); }
 
 // Partials of the attention splits: the unnormalised p V sums [nH][nsplit][hd],
 // then (m, l) pairs [nH][nsplit][2].
@@ -1003,15 +1005,21 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
 // Head blockIdx.x, dims 64 blockIdx.y .. + 63 (lane = dim), NW waves:
 // out = sum_c acc_c e^(m_c - M) / sum_c l_c e^(m_c - M), M = max_c m_c,
 // over the live splits c; wave w sums splits w, w + NW, .. in order, then the
-// waves' sums are added in order. The wave loads its dims of its first MB
-// splits and the (m, l) of splits lane, lane + 64, .. before the position
-// (which sets the live split count) arrives, takes M with a cross-lane
-// maximum (lane c holds split c, c + 64, ..); the weights e^(m_c - M) go
-// through LDS. One wave and no barrier up to 32 splits; 8 waves above, where
-// one wave's batches of 32 loads were a serial chain of memory round trips
-// (254 splits of 16 heads, hd 512: 17.4 -> 5.2 us).
+// waves' sums are added in order. Before the position (which sets the live
+// split count) arrives, the wave loads its dims of its first PF splits and the
+// (m, l) of splits lane, lane + 64, ..; the rest of its first MB splits follow
+// where they are live. M is a cross-lane maximum (lane c holds split c, c +
+// 64, ..); the weights e^(m_c - M) go through LDS. One wave and no barrier up
+// to 32 splits, all of them loaded at once; 8 waves above, where one wave's
+// batches of 32 loads were a serial chain of memory round trips (254 splits of
+// 16 heads, hd 512: 17.4 -> 5.2 us). There PF < MB: 32 splits per wave loaded
+// blindly are 8.4 MB of dead partials early in a long context (split and merge,
+// PF 32 / 8: 16 heads of 512, 8192 slots, 16.8 / 13.5 us at position 500 and 18.5 /
+// 18.5 at 8184; 16 heads of 256, 4096 slots, 12.8 / 12.4 and 13.2 / 12.8 at 4088,
+// with one wave 12.6 and 15.2; PF 4 loses where 8 just cover the context: 12.8
+// -> 13.4).
 // ml: nsplit floats of dynamic shared memory. out fp32 or fp16.
-template <int YT, int EPL, int MB, int NW>
+template <int YT, int EPL, int MB, int NW, int PF>
 __global__ void __launch_bounds__(64 * NW) attn_merge_kernel(const float* __restrict__ part, void* __restrict__ out,
                                                              int nsplit, int kch, int stride, int window,
                                                              const uint32_t* __restrict__ dyn) {
@@ -1024,14 +1032,21 @@ __global__ void __launch_bounds__(64 * NW) attn_merge_kernel(const float* __rest
   const float2* wml = reinterpret_cast<const float2*>(part + (long)gridDim.x * nsplit * HD) + (long)h * nsplit;
   // indices clamped to the workspace until the live split count is known
   float x[MB];
-  auto fetch = [&](int c0, int cmax) {
+  auto fetch = [&](auto lo, auto hi, int c0, int cmax) {
 #pragma unroll
-    for (int c = 0; c < MB; ++c) x[c] = w[(long)min(c0 + NW * c, cmax) * HD + d];
+    for (int c = decltype(lo)::value; c < decltype(hi)::value; ++c) x[c] = w[(long)min(c0 + NW * c, cmax) * HD + d];
   };
-  fetch(wave, nsplit - 1);
+  using C0 = std::integral_constant<int, 0>;
+  using CP = std::integral_constant<int, PF>;
+  using CM = std::integral_constant<int, MB>;
+  const uint32_t posv = load_pos_lane(dyn);  // requested first: the others arrive behind it
+  fetch(C0{}, CP{}, wave, nsplit - 1);
   const float2 ml_t = wml[min(t, nsplit - 1)];
-  const int T = att_len(load_pos(dyn), window, stride);
+  const int T = att_len(__builtin_amdgcn_readfirstlane(posv), window, stride);
   const int ns = (T + kch - 1) / kch;
+  if constexpr (PF < MB) {
+    if (wave + NW * PF < ns) fetch(CP{}, CM{}, wave, ns - 1);
+  }
   float M = t < ns ? ml_t.x : -INFINITY;
   for (int c = t + 64; c < ns; c += 64) M = fmaxf(M, wml[c].x);
   M = reduce64<true>(M);
@@ -1052,7 +1067,7 @@ __global__ void __launch_bounds__(64 * NW) attn_merge_kernel(const float* __rest
   }
   float acc = 0.0f;
   for (int c0 = wave; c0 < ns; c0 += MB * NW) {
-    if (c0 > wave) fetch(c0, ns - 1);
+    if (c0 > wave) fetch(C0{}, CM{}, c0, ns - 1);
 #pragma unroll
     for (int c = 0; c < MB; ++c)
       if (c0 + NW * c < ns) acc = fmaf(x[c], ml[c0 + NW * c], acc);
@@ -1270,16 +1285,16 @@ static int attn_launch(const float* qkv, const float* qnw, const float* cosb, co
                      qoff, grp, hpw, dyn, part, ns, knw, koff, voff)
   // the merge fetches its splits MB per wave at a time: one wave and the smallest of 8, 16, 32 that covers them all,
   // else 8 waves of 32
-#define Q4_MRG2(E, MB, W)                                                                                             \
-  if (h16) hipLaunchKernelGGL((attn_merge_kernel<Q4_DT_F16, E, MB, W>), dim3(nH, E), dim3(64 * W), msh, st, part, out, \
-                              ns, kch, stride, window, dyn);                                                         \
-  else hipLaunchKernelGGL((attn_merge_kernel<Q4_DT_F32, E, MB, W>), dim3(nH, E), dim3(64 * W), msh, st, part, out, ns, \
-                          kch, stride, window, dyn)
-#define Q4_MRG(E)                  \
-  if (ns <= 8) { Q4_MRG2(E, 8, 1); }  \
-  else if (ns <= 16) { Q4_MRG2(E, 16, 1); } \
-  else if (ns <= 32) { Q4_MRG2(E, 32, 1); } \
-  else { Q4_MRG2(E, 32, 8); }
+#define Q4_MRG2(E, MB, W, PF)                                                                                          \
+  if (h16) hipLaunchKernelGGL((attn_merge_kernel<Q4_DT_F16, E, MB, W, PF>), dim3(nH, E), dim3(64 * W), msh, st, part,   \
+                              out, ns, kch, stride, window, dyn);                                                      \
+  else hipLaunchKernelGGL((attn_merge_kernel<Q4_DT_F32, E, MB, W, PF>), dim3(nH, E), dim3(64 * W), msh, st, part, out,  \
+                          ns, kch, stride, window, dyn)
+#define Q4_MRG(E)                            \
+  if (ns <= 8) { Q4_MRG2(E, 8, 1, 8); }      \
+  else if (ns <= 16) { Q4_MRG2(E, 16, 1, 16); } \
+  else if (ns <= 32) { Q4_MRG2(E, 32, 1, 32); } \
+  else { Q4_MRG2(E, 32, 8, ATT_MERGE_PF); }
   switch (hd) {
     case 64: if (prep) { Q4_ATT(1, true, 8); } else { Q4_ATT(1, false, 8); } break;
     case 128: if (prep) { Q4_ATT(2, true, 8); } else { Q4_ATT(2, false, 8); } break;

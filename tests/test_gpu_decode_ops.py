@@ -308,3 +308,22 @@ def test_attn_infinities_in_the_cache(gpu, nH, nkv, stride, window, pos, where):
     assert (np.isinf(got) == np.isinf(ref)).all() and (got[np.isinf(ref)] == ref[np.isinf(ref)]).all()
     ok = np.isfinite(ref)
     assert O.normwise_rel_err(got[ok], ref[ok]) <= 1e-4
+
+
+@pytest.mark.parametrize("nsplit_live", [1, 63, 64, 65, 120, 256, 257, 300])
+@pytest.mark.parametrize("odt", [torch.float32, torch.float16])
+def test_attn_merge_of_many_splits(gpu, nsplit_live, odt):
+    """Live split counts around what the 8-wave merge loads before and after
+    it knows the position (64 and 256), in a cache of 300 splits whose dead
+    partials are NaN, against the oracle (test_attn's bound, or the fp16
+    output's half step)."""
+    nH, nkv, hd = 4, 2, 64
+    stride, pos = 300 * 64, nsplit_live * 64 - 3   # 64-key splits
+    rng = np.random.default_rng(nsplit_live)
+    qkv, qnw, cs, sn, kc, vc = _attn_case(rng, nH, nkv, hd, stride)
+    ws = torch.full_like(gpu.attn_workspace(nH, hd, stride), float("nan"))
+    dyn = torch.tensor([pos, pos + 1, 0, 0], dtype=torch.int32, device="cuda")
+    got = _np(gpu.attn(_t(qkv), _t(qnw), _t(cs), _t(sn), _t(kc, torch.float16), _t(vc, torch.float16), nH=nH, nkv=nkv,
+                       hd=hd, stride=stride, window=0, qoff=0, grp=nH // nkv, dyn=dyn, ws=ws, out_dtype=odt))
+    ref = D.attn_ref(qkv, qnw, cs, sn, kc, vc, nH=nH, hd=hd, stride=stride, window=0, qoff=0, grp=nH // nkv, pos=pos)
+    assert O.normwise_rel_err(got.astype(np.float64), ref) <= (1e-4 if odt == torch.float32 else 1e-3)
