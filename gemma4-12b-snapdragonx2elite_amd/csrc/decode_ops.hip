@@ -486,6 +486,9 @@ __device__ inline uint32_t load_pos(const uint32_t* dyn) { return __builtin_amdg
 // Partials of the attention splits: the unnormalised p V sums [nH][nsplit][hd],
 // then (m, l) pairs [nH][nsplit][2].
 __device__ inline float* attn_ml(float* part, int nH, int nsplit, int hd) { return part + (long)nH * nsplit * hd; }
+struct SplitMl {  // (one load of a pair; the workspace is float-aligned, which float2 is not)
+  float m, l;
+};
 
 // Decode attention, split along the keys (vk/attn.comp:18-53,
 // flash-decoding). Workgroup (g, s): head group g = hpw query heads of one
@@ -1029,7 +1032,7 @@ __global__ void __launch_bounds__(64 * NW) attn_merge_kernel(const float* __rest
   const int h = blockIdx.x, t = threadIdx.x & 63, d = blockIdx.y * 64 + t;
   const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
   const float* w = part + (long)h * nsplit * HD;
-  const float2* wml = reinterpret_cast<const float2*>(part + (long)gridDim.x * nsplit * HD) + (long)h * nsplit;
+  const SplitMl* wml = reinterpret_cast<const SplitMl*>(part + (long)gridDim.x * nsplit * HD) + (long)h * nsplit;
   // indices clamped to the workspace until the live split count is known
   float x[MB];
   auto fetch = [&](auto lo, auto hi, int c0, int cmax) {
@@ -1041,21 +1044,21 @@ __global__ void __launch_bounds__(64 * NW) attn_merge_kernel(const float* __rest
   using CM = std::integral_constant<int, MB>;
   const uint32_t posv = load_pos_lane(dyn);  // requested first: the others arrive behind it
   fetch(C0{}, CP{}, wave, nsplit - 1);
-  const float2 ml_t = wml[min(t, nsplit - 1)];
+  const SplitMl ml_t = wml[min(t, nsplit - 1)];
   const int T = att_len(__builtin_amdgcn_readfirstlane(posv), window, stride);
   const int ns = (T + kch - 1) / kch;
   if constexpr (PF < MB) {
     if (wave + NW * PF < ns) fetch(CP{}, CM{}, wave, ns - 1);
   }
-  float M = t < ns ? ml_t.x : -INFINITY;
-  for (int c = t + 64; c < ns; c += 64) M = fmaxf(M, wml[c].x);
+  float M = t < ns ? ml_t.m : -INFINITY;
+  for (int c = t + 64; c < ns; c += 64) M = fmaxf(M, wml[c].m);
   M = reduce64<true>(M);
   float L = 0.0f;
   for (int c = threadIdx.x; c < ns; c += 64 * NW) {
-    const float2 mc = c == t ? ml_t : wml[c];
-    const float wc = expf(mc.x - M);
+    const SplitMl mc = c == t ? ml_t : wml[c];
+    const float wc = expf(mc.m - M);
     ml[c] = wc;
-    L = fmaf(mc.y, wc, L);
+    L = fmaf(mc.l, wc, L);
   }
   L = reduce64<false>(L);
   if constexpr (NW > 1) {

@@ -166,9 +166,8 @@ __global__ void __launch_bounds__(256) e4m3_lift_kernel(const float* __restrict_
   __syncthreads();
   for (int i = threadIdx.x; i < TB * 16; i += 256) {
     const int bb = i >> 4, w = i & 15;
-    if (b0 + bb < nblk)
-      *reinterpret_cast<uint32_t*>(sc8 + ((long)p * nblk + b0 + bb) * PANEL + 4 * w) =
-          *reinterpret_cast<const uint32_t*>(&out[bb][4 * w]);
+    if (b0 + bb < nblk)  // one 4-byte store, at any alignment of sc8
+      __builtin_memcpy(sc8 + ((long)p * nblk + b0 + bb) * PANEL + 4 * w, &out[bb][4 * w], 4);
   }
 }
 

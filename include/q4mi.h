@@ -99,7 +99,7 @@ int q4_quantize(const float* W, int N, int K, uint32_t* wq, uint16_t* sc16,
                 float* sc32, void* stream);
 
 /* fp32 scales sc32 [N][K/32] -> e4m3 scales (panel-64 bytes) with the
- * per-tensor power-of-two lift; writes inv = 2^-shift to *inv_dev (device
+ * per-tensor power-of-two lift, into sc8 at any address; writes inv = 2^-shift to *inv_dev (device
  * float) and the max scale bits to *work (device uint32, caller-owned,
  * zeroed by this call). src/vk_engine.py:133-137. */
 int q4_scales_e4m3(const float* sc32, int N, int K, uint8_t* sc8,
@@ -445,8 +445,8 @@ int q4_prepkv(const float* qkv, const float* knw, const float* cosb, const float
  * of KV head h/grp: softmax(q.k) weighted sum of V into out[nH*hd] (fp32
  * or fp16, out_dtype). Split along the keys (two launches: the splits of
  * each group of query heads sharing a KV head, then their merge); ws:
- * q4_attn_workspace_bytes(nH, hd, stride) bytes, no initialisation needed.
- * hd 64, 128, 256 or 512; qkv, qnw, cosb, sinb (and knw), kc and vc 16-byte
+ * q4_attn_workspace_bytes(nH, hd, stride) bytes at any float's address, no
+ * initialisation needed. hd 64, 128, 256 or 512; qkv, qnw, cosb, sinb (and knw), kc and vc 16-byte
  * aligned, qoff (koff, voff) multiples of 4.
  * vk/attn.comp:18-53 (d_attn, src/vk_engine.py:238-239). */
 size_t q4_attn_workspace_bytes(int nH, int hd, int stride);

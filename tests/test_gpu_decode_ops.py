@@ -327,3 +327,22 @@ def test_attn_merge_of_many_splits(gpu, nsplit_live, odt):
                        hd=hd, stride=stride, window=0, qoff=0, grp=nH // nkv, dyn=dyn, ws=ws, out_dtype=odt))
     ref = D.attn_ref(qkv, qnw, cs, sn, kc, vc, nH=nH, hd=hd, stride=stride, window=0, qoff=0, grp=nH // nkv, pos=pos)
     assert O.normwise_rel_err(got.astype(np.float64), ref) <= (1e-4 if odt == torch.float32 else 1e-3)
+
+
+@pytest.mark.parametrize("nH,nkv,hd,stride", [(16, 1, 512, 100), (16, 1, 512, 2000), (4, 2, 64, 300), (4, 2, 128, 3000)])
+def test_attn_workspace_at_any_float(gpu, nH, nkv, hd, stride):
+    """A workspace that starts 4 bytes past a 16-byte boundary gives the bits
+    of an aligned one, for both splits and both merges, and nothing before
+    or behind it is written."""
+    rng = np.random.default_rng(stride)
+    qkv, qnw, cs, sn, kc, vc = _attn_case(rng, nH, nkv, hd, stride)
+    dyn = torch.tensor([stride - 2, stride - 1, 0, 0], dtype=torch.int32, device="cuda")
+    n = gpu.attn_workspace(nH, hd, stride).numel()
+    outs = []
+    for off in (0, 1):
+        buf = torch.full((n + 8,), 3.0, device="cuda")
+        outs.append(gpu.attn(_t(qkv), _t(qnw), _t(cs), _t(sn), _t(kc, torch.float16), _t(vc, torch.float16), nH=nH,
+                             nkv=nkv, hd=hd, stride=stride, window=0, qoff=0, grp=nH // nkv, dyn=dyn,
+                             ws=buf[off:off + n]))
+        assert bool((buf[:off] == 3.0).all()) and bool((buf[off + n:] == 3.0).all())
+    assert torch.equal(*outs)

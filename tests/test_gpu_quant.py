@@ -164,3 +164,17 @@ def test_fold_row_groups_bit_exact(gpu, N, K):
     assert (to_np(gW8) == W8).all() and (to_np(gsw32).view(np.uint32) == sw.view(np.uint32)).all()
     pW8, psw32, psw16 = gpu.w8_fold_packed(wq, sc32, N, K)
     assert torch.equal(pW8, gpu.w8_pack(gW8)) and torch.equal(psw32, gsw32) and torch.equal(psw16, gsw16)
+
+
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_scales_e4m3_into_an_unaligned_buffer(gpu, off):
+    """The e4m3 scales are bytes: any start address gives the same ones, and
+    nothing around them is written."""
+    N, K = 130, 416
+    sc32 = torch.rand(N, K // 32, device="cuda")
+    ref, inv = gpu.scales_e4m3(sc32, N, K)
+    buf = torch.full((ref.numel() + 8,), 77, dtype=torch.uint8, device="cuda")
+    inv_d, work = torch.empty(1, device="cuda"), torch.empty(1, dtype=torch.int32, device="cuda")
+    gpu.call("q4_scales_e4m3", gpu._p(sc32), N, K, gpu._p(buf[off:]), gpu._p(inv_d), gpu._p(work), gpu._stream())
+    assert torch.equal(buf[off:off + ref.numel()], ref) and float(inv_d.item()) == inv
+    assert bool((buf[:off] == 77).all()) and bool((buf[off + ref.numel():] == 77).all())
