@@ -99,9 +99,9 @@ int q4_quantize(const float* W, int N, int K, uint32_t* wq, uint16_t* sc16,
                 float* sc32, void* stream);
 
 /* fp32 scales sc32 [N][K/32] -> e4m3 scales (panel-64 bytes) with the
- * per-tensor power-of-two lift, into sc8 at any address; writes inv = 2^-shift to *inv_dev (device
- * float) and the max scale bits to *work (device uint32, caller-owned,
- * zeroed by this call). src/vk_engine.py:133-137. */
+ * per-tensor power-of-two lift, into sc8 at any address; writes inv =
+ * 2^-shift to *inv_dev (device float) and the max scale bits to *work (device
+ * uint32, caller-owned, zeroed by this call). src/vk_engine.py:133-137. */
 int q4_scales_e4m3(const float* sc32, int N, int K, uint8_t* sc8,
                    float* inv_dev, uint32_t* work, void* stream);
 
@@ -144,14 +144,19 @@ int q4_repack_w8_ref(const int8_t* w8_kn, int N, int K, int8_t* w8_nk,
  * (vk/gemv_fp8.comp:20-40) as recorded by gemv_ds()/gemv()
  * (src/vk_engine.py:214-226, 270-272).
  * x: x_dtype [K]; y: y_dtype [N]. split = number of workgroups sharing one
- * 64-row panel along K (0 = choose automatically). When the effective split
- * is > 1 a workspace of q4_workspace_bytes(Q4_OP_GEMV, N, K, split) bytes is
- * required; it must be zero-filled once before first use (q4_workspace_init)
- * and is left ready for the next call. One workspace per stream. */
+ * 64-row panel along K (0 = choose automatically: matrices of few rows, which
+ * would need a split to fill the GPU, run unsplit in groups of 4 or 8 rows where
+ * x fits a workgroup's staging, K <= 32768 for fp16 x and K <= 16384 for fp32).
+ * Where q4_workspace_bytes(Q4_OP_GEMV, N, K, split) is not 0 a workspace of that
+ * many bytes is required, also by a call with split 0 that then runs unsplit;
+ * it must be zero-filled once before first use (q4_workspace_init) and is left
+ * ready for the next call. One workspace per stream. */
 size_t q4_workspace_bytes(int op, int N, int K, int split);
 int q4_workspace_init(void* ws, size_t bytes, void* stream);
-/* The split the library uses for an N x K GEMV when asked for split = 0
- * (the MI355X counterpart of src/vk_engine.py:143-148). */
+/* The split that sizes the workspace of an N x K GEMV with split = 0 (the
+ * MI355X counterpart of src/vk_engine.py:143-148). Asked for as an explicit split
+ * it is used as it is; split = 0 may run unsplit instead (above), with the
+ * sums in another order. */
 int q4_gemv_auto_split(int N, int K);
 
 int q4_gemv(const void* x, int x_dtype, const uint32_t* wq,
@@ -446,8 +451,8 @@ int q4_prepkv(const float* qkv, const float* knw, const float* cosb, const float
  * or fp16, out_dtype). Split along the keys (two launches: the splits of
  * each group of query heads sharing a KV head, then their merge); ws:
  * q4_attn_workspace_bytes(nH, hd, stride) bytes at any float's address, no
- * initialisation needed. hd 64, 128, 256 or 512; qkv, qnw, cosb, sinb (and knw), kc and vc 16-byte
- * aligned, qoff (koff, voff) multiples of 4.
+ * initialisation needed. hd 64, 128, 256 or 512; qkv, qnw, cosb, sinb (and
+ * knw), kc and vc 16-byte aligned, qoff (koff, voff) multiples of 4.
  * vk/attn.comp:18-53 (d_attn, src/vk_engine.py:238-239). */
 size_t q4_attn_workspace_bytes(int nH, int hd, int stride);
 int q4_attn(const float* qkv, const float* qnw, const float* cosb, const float* sinb,

@@ -146,3 +146,28 @@ def test_record_once_token_graph(E):
         q, sc = O.quant_codes(lmW)
         assert O.normwise_rel_err(y, O.gemv_ref(q, sc.astype(np.float16).astype(np.float32), x[:H])) <= 2e-5
     graph.destroy()
+
+
+@pytest.mark.parametrize("xdt", [torch.float32, torch.float16])
+def test_few_row_descriptors_run_the_automatic_plan(E, gpu, xdt):
+    """A quantized matrix of few rows stores the library's split; its
+    descriptor, and the fused gate/up one, give the bits of the automatic
+    plan (one unsplit launch), while another stored split runs as stored."""
+    rng = np.random.default_rng(44)
+    N, K = 512, 3840
+    qw = E.quant(_w(rng, N, K), fp8=False, prefill_i8=False)
+    qu = E.quant(_w(rng, N, K), fp8=False, prefill_i8=False)
+    assert qw.split == gpu.auto_split(N, K) > 3
+    x = torch.from_numpy(rng.standard_normal(K).astype(np.float32)).cuda().to(xdt)
+    inbuf, outbuf, act = E.Buf(tensor=x), E.Buf(N * 4), E.Buf(N * 4)
+    for stored, split in ((qw.split, 0), (3, 3)):
+        E.gemv(E.gemv_ds((qw._replace(split=stored), (N, K)), inbuf, outbuf, x_dtype=xdt))
+        y = gpu.gemv(x, qw.bw.t, qw.bs.t, N, K, y_dtype=torch.float32, split=split)
+        torch.cuda.synchronize()
+        assert torch.equal(outbuf.view(torch.float32, N), y), stored
+    d = E.gate_up_ds((qw, (N, K)), (qu, (N, K)), inbuf, act, x_dtype=xdt)
+    d.fn(*d.args, **d.kw)
+    a = gpu.gemv_gated(x, *gpu.interleave_rows(qw.bw.t, qw.bs.t, qu.bw.t, qu.bs.t, N, K), 2 * N, K,
+                       act_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert torch.equal(act.view(torch.float32, N), a)
