@@ -229,47 +229,58 @@ def test_prepkv_attn_fused_equals_separate(gpu, nH, nkv, hd, stride, window, pos
         assert torch.equal(o1, o2) and torch.equal(kc1, kc2) and torch.equal(vc1, vc2), odt
 
 
-@pytest.mark.parametrize("nH,nkv,hd,stride,pos", [
-    (16, 1, 512, 64, 0),        # one key
-    (16, 1, 512, 64, 15),       # a whole 16-key tile
-    (16, 1, 512, 64, 16),
-    (16, 1, 512, 64, 31),       # a whole split
-    (16, 1, 512, 64, 32),       # one key in the second split
-    (16, 1, 512, 100, 99),      # last slot of a depth that is no multiple of the split
-    (16, 1, 512, 100, 130),     # past the cache depth: nothing written
-    (32, 2, 512, 300, 250),     # two KV heads
-    (32, 1, 512, 300, 40),      # two head groups of one KV head: the first writes the cache
-    (16, 1, 512, 8200, 8150),   # 255 live splits of 257: every wave of the merge has work
-    (16, 1, 512, 33000, 32999),  # 1032 splits: several batches per wave of the merge
-    (2, 2, 64, 2200, 2111),     # 33 splits: the first count with the 8-wave merge
+@pytest.mark.parametrize("nH,nkv,hd,stride,window,pos,keqv", [
+    (16, 1, 512, 64, 0, 0, False),        # one key
+    (16, 1, 512, 64, 0, 15, False),       # a whole 16-key tile
+    (16, 1, 512, 64, 0, 16, True),
+    (16, 1, 512, 64, 0, 31, False),       # a whole split
+    (16, 1, 512, 64, 0, 32, False),       # one key in the second split
+    (16, 1, 512, 100, 0, 99, False),      # last slot of a depth that is no multiple of the split
+    (16, 1, 512, 100, 0, 130, False),     # past the cache depth: nothing written
+    (32, 2, 512, 300, 0, 250, False),     # two KV heads
+    (32, 1, 512, 300, 0, 40, True),       # two head groups of one KV head: the first writes the cache
+    (16, 1, 512, 100, 96, 250, False),    # a wrapped ring: the fresh slot in a split with live keys on both sides
+    (32, 1, 512, 100, 96, 287, True),     # its last slot
+    (32, 2, 512, 100, 90, 180, False),    # its first slot, a window that is no multiple of the split
+    (16, 1, 512, 8200, 0, 8150, True),    # 255 live splits of 257: every wave of the merge has work
+    (16, 1, 512, 33000, 0, 32999, False),  # 1032 splits: several batches per wave of the merge
+    (2, 2, 64, 2200, 0, 2111, False),     # 33 splits: the first count with the 8-wave merge
 ])
-def test_prepkv_attn_many_heads_and_splits(gpu, nH, nkv, hd, stride, pos):
+@pytest.mark.parametrize("qoff", [0, 1024])
+def test_prepkv_attn_many_heads_and_splits(gpu, nH, nkv, hd, stride, window, pos, keqv, qoff):
     """16-head groups at hd 512 (matrix-core split) and more than 32 splits
-    (8-wave merge), against the oracle; NaN in the rows past the position must
-    not reach the result; caches and output equal q4_prepkv + q4_attn's."""
+    (8-wave merge), against the oracle; NaN in the rows that no token has
+    written must not reach the result; caches and output, fp32 and fp16,
+    equal q4_prepkv + q4_attn's."""
     rng = np.random.default_rng(stride + pos)
     qkv, qnw, cs, sn, kc, vc = _attn_case(rng, nH, nkv, hd, stride)
+    qkv = np.concatenate([np.full(qoff, 1e4, np.float32), qkv])
     knw = (rng.random(hd) + 0.5).astype(np.float32)
-    kc.reshape(nkv, stride, hd)[:, pos + 1:] = np.nan
-    vc.reshape(nkv, stride, hd)[:, pos + 1:] = np.nan
+    kc.reshape(nkv, stride, hd)[:, min(pos + 1, window or stride):] = np.nan
+    vc.reshape(nkv, stride, hd)[:, min(pos + 1, window or stride):] = np.nan
     dyn = torch.tensor([pos, pos + 1, 0, 0], dtype=torch.int32, device="cuda")
     t = dict(qkv=_t(qkv), knw=_t(knw), qnw=_t(qnw), cs=_t(cs), sn=_t(sn))
-    kc1, vc1 = _t(kc, torch.float16), _t(vc, torch.float16)
-    kc2, vc2 = kc1.clone(), vc1.clone()
-    kw = dict(nH=nH, nkv=nkv, hd=hd, stride=stride, window=0, qoff=0, grp=nH // nkv, dyn=dyn)
-    koff, voff = nH * hd, nH * hd + nkv * hd
-    gpu.prepkv(t["qkv"], t["knw"], t["cs"], t["sn"], kc1, vc1, nkv=nkv, hd=hd, koff=koff, voff=voff, keqv=False,
-               stride=stride, window=0, dyn=dyn)
-    o1 = gpu.attn(t["qkv"], t["qnw"], t["cs"], t["sn"], kc1, vc1, **kw)
-    o2 = gpu.prepkv_attn(t["qkv"], t["knw"], t["qnw"], t["cs"], t["sn"], kc2, vc2, koff=koff, voff=voff, keqv=False,
-                         **kw)
-    torch.cuda.synchronize()
-    assert torch.equal(o1, o2)
-    assert torch.equal(kc1.view(torch.int16), kc2.view(torch.int16))
-    assert torch.equal(vc1.view(torch.int16), vc2.view(torch.int16))
-    ref = D.attn_ref(qkv, qnw, cs, sn, _np(kc1), _np(vc1), nH=nH, hd=hd, stride=stride, window=0, qoff=0,
-                     grp=nH // nkv, pos=min(pos, stride - 1))
-    assert O.normwise_rel_err(_np(o1), ref) <= 1e-4   # the bound of test_attn: fp32 sums over fp16 caches
+    kw = dict(nH=nH, nkv=nkv, hd=hd, stride=stride, window=window, qoff=qoff, grp=nH // nkv, dyn=dyn)
+    koff = qoff + nH * hd
+    voff = koff if keqv else koff + nkv * hd
+    outs = {}
+    for odt in (torch.float32, torch.float16):
+        kc1, vc1 = _t(kc, torch.float16), _t(vc, torch.float16)
+        kc2, vc2 = kc1.clone(), vc1.clone()
+        gpu.prepkv(t["qkv"], t["knw"], t["cs"], t["sn"], kc1, vc1, nkv=nkv, hd=hd, koff=koff, voff=voff, keqv=keqv,
+                   stride=stride, window=window, dyn=dyn)
+        o1 = gpu.attn(t["qkv"], t["qnw"], t["cs"], t["sn"], kc1, vc1, out_dtype=odt, **kw)
+        o2 = gpu.prepkv_attn(t["qkv"], t["knw"], t["qnw"], t["cs"], t["sn"], kc2, vc2, koff=koff, voff=voff, keqv=keqv,
+                             out_dtype=odt, **kw)
+        torch.cuda.synchronize()
+        assert torch.equal(o1, o2)
+        assert torch.equal(kc1.view(torch.int16), kc2.view(torch.int16))
+        assert torch.equal(vc1.view(torch.int16), vc2.view(torch.int16))
+        outs[odt] = o1
+    assert torch.equal(outs[torch.float16], outs[torch.float32].half())
+    ref = D.attn_ref(qkv, qnw, cs, sn, _np(kc1), _np(vc1), nH=nH, hd=hd, stride=stride, window=window, qoff=qoff,
+                     grp=nH // nkv, pos=pos if window else min(pos, stride - 1))
+    assert O.normwise_rel_err(_np(outs[torch.float32]), ref) <= 1e-4   # the bound of test_attn: fp32 sums over fp16 caches
 
 
 @pytest.mark.parametrize("nH,nkv,stride,window,pos", [

@@ -442,10 +442,10 @@ def test_w4a16_gated_equals_separate_gemms_and_gelumul(gpu, M, I, K, dev_interle
     assert np.abs(A.astype(np.float64) - act).max() <= np.abs(act).max() * 2.0 ** -9
 
 
-@pytest.mark.parametrize("M,N,K", [(100, 660, 1056),     # unsplit, 9 and 8 k-steps, the last one half a step
-                                   (37, 14, 4096),       # one partial column tile, four splits
+@pytest.mark.parametrize("M,N,K", [(100, 660, 1056),     # two splits, 5 and 4 k-steps, the last one half a step
+                                   (37, 14, 4096),       # one partial column tile, eight splits
                                    (128, 3848, 4096),    # a last tile of 8 columns
-                                   (300, 520, 2080),     # three row tiles, two splits
+                                   (300, 520, 2080),     # three row tiles, four splits
                                    (128, 30720, 3840)])  # the chunk's gate/up, unsplit
 def test_w4a16_narrow_tiles(gpu, M, N, K, tune):
     """128-column tiles of two k-groups (the automatic plan of these shapes)

@@ -196,21 +196,23 @@ def test_gemv_output_offset_and_untouched_neighbours(gpu):
 
 
 def test_gemv_graph_replay_matches_eager(gpu):
-    """A captured sequence of split-K GEMVs sharing one workspace replays
+    """A captured sequence of unsplit and split-K GEMVs (explicit splits, and
+    one automatic: K past the staging) sharing one workspace replays
     bit-identically to eager execution, replay after replay."""
     rng = np.random.default_rng(7)
-    shapes = [(4096, 3840), (512, 3840), (2048, 3840), (256, 15360), (3840, 4096), (3840, 15360), (15360, 3840)]
+    shapes = [(4096, 3840, 0), (512, 3840, 7), (2048, 3840, 3), (256, 15360, 30), (512, 3840, 0), (64, 33024, 0),
+              (3840, 4096, 0), (3840, 15360, 2), (15360, 3840, 0)]
     mats = []
-    for N, K in shapes:
+    for N, K, split in shapes:
         q, s = synth_int4(rng, N, K)
         wq, sc = upload_int4(q, s)
         x = torch.from_numpy(rng.standard_normal(K).astype(np.float16)).cuda()
-        mats.append((N, K, wq, sc, x, torch.empty(N, device="cuda")))
-    ws = gpu.Workspace(max(gpu.Workspace.bytes_for(N, K) for N, K in shapes))
+        mats.append((N, K, wq, sc, x, torch.empty(N, device="cuda"), split))
+    ws = gpu.Workspace(max(gpu.Workspace.bytes_for(*s) for s in shapes))
 
     def body():
-        for N, K, wq, sc, x, y in mats:
-            gpu.gemv(x, wq, sc, N, K, y=y, ws=ws)
+        for N, K, wq, sc, x, y, split in mats:
+            gpu.gemv(x, wq, sc, N, K, y=y, ws=ws, split=split)
 
     body()
     torch.cuda.synchronize()
@@ -314,8 +316,8 @@ def test_gemv_batch_e4m3(gpu):
 def test_gemv_gated_vs_oracle(gpu, I, K, xdt, adt):
     """Interleaved gate/up rows and the gelumul epilogue: act = gelu_tanh(W_g x)
     * (W_u x) against the oracle's GEMVs and gelumul (normwise <= 5e-5 fp32,
-    the product doubles the GEMVs' relative error; <= 1e-3 fp16). I = 64 and
-    96 take the split-K path."""
+    the product doubles the GEMVs' relative error; <= 1e-3 fp16); the smaller
+    ones also with an explicit K split."""
     from oracle import decode_ops_oracle as D
     rng = np.random.default_rng(I + K)
     qg, sg = synth_int4(rng, I, K)
@@ -331,10 +333,11 @@ def test_gemv_gated_vs_oracle(gpu, I, K, xdt, adt):
     assert np.array_equal(codes[0::2], qg) and np.array_equal(codes[1::2], qu)
     sc = O.unscales_dev(to_np(so), 2 * I, K // 32)
     assert np.array_equal(sc[0::2], sg.astype(np.float16)) and np.array_equal(sc[1::2], su.astype(np.float16))
-    act = gpu.gemv_gated(torch.from_numpy(xin).cuda(), wo, so, 2 * I, K, act_dtype=adt)
-    assert act.numel() == I and act.dtype == adt
     tol = 1e-3 if adt == torch.float16 else 5e-5
-    assert O.normwise_rel_err(to_np(act).astype(np.float64), ref) <= tol
+    for split in (0, 3) if I < 1000 else (0,):
+        act = gpu.gemv_gated(torch.from_numpy(xin).cuda(), wo, so, 2 * I, K, act_dtype=adt, split=split)
+        assert act.numel() == I and act.dtype == adt
+        assert O.normwise_rel_err(to_np(act).astype(np.float64), ref) <= tol, split
 
 
 @pytest.mark.parametrize("N,K,rows", [(15360, 3840, None), (30720, 3840, None), (1024, 4096, "16"), (4096, 15360, "32"),
@@ -393,6 +396,10 @@ def test_gemv_few_rows(gpu, N, K):
         assert O.normwise_rel_err(to_np(y8), O.gemv_ref(q, s8, xin, inv)) <= TOL_F32
         yh = gpu.gemv(xt, wq, sc, N, K, y_dtype=torch.float16)
         assert torch.equal(yh, y.half())
+        yn = torch.empty_like(y)
+        gpu.call("q4_gemv_noalloc", gpu._p(xt), gpu._dt(xt), gpu._p(wq), gpu._p(sc), gpu.SCALE_F16, 1.0, gpu._p(yn),
+                 gpu.DT_F32, N, K, 0, gpu._stream())
+        assert torch.equal(yn, y)
         act = gpu.gemv_gated(xt, wq, sc, N, K, act_dtype=torch.float32)
         g, u = y[0::2].double(), y[1::2].double()
         ref = 0.5 * g * (1 + torch.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3))) * u

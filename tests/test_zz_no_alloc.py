@@ -2,7 +2,8 @@
 device array instead of a caller buffer) against q4_gemv with a caller
 workspace: bit-identical outputs, through the C ABI, for two calls in a
 row (the second smaller, reusing the array's previous contents), split-K
-and unsplit plans, fp16 and e4m3 scales; and against the oracle."""
+(explicit, and automatic where x is longer than the staging) and unsplit
+plans, fp16 and e4m3 scales; and against the oracle."""
 import ctypes as C
 
 import numpy as np
@@ -33,9 +34,11 @@ def test_noalloc_matches_workspace_gemv(g4, gpu, e4m3):
     rng = np.random.default_rng(31 + int(e4m3))
     fmt = gpu.SCALE_E4M3 if e4m3 else gpu.SCALE_F16
     # first a split-K plan with many row groups, then a smaller one (fewer groups, other split):
-    # the second call must not see the first call's partials or tickets; then two unsplit shapes
-    for N, K in [(1792, 3840), (320, 2048), (64, 256), (2048, 4096), (4096, 3840)]:
-        print(f"noalloc N={N} K={K} e4m3={e4m3} split={gpu.auto_split(N, K)}", flush=True)
+    # the second call must not see the first call's partials or tickets; a K past the staging of
+    # fp16 x splits by itself; then unsplit shapes, with few rows and with many
+    for N, K, split in [(1792, 3840, 5), (320, 2048, 3), (64, 33024, 0), (1792, 3840, 0), (320, 2048, 0), (64, 256, 0),
+                        (2048, 4096, 0), (4096, 3840, 0)]:
+        print(f"noalloc N={N} K={K} e4m3={e4m3} split={split}", flush=True)
         q, s = synth_int4(rng, N, K)
         wq, sc = upload_int4(q, s)
         inv = 1.0
@@ -47,12 +50,13 @@ def test_noalloc_matches_workspace_gemv(g4, gpu, e4m3):
             s_used = O.e4m3_decode(e8).astype(np.float32)
         xh = rng.standard_normal(K).astype(np.float16)
         x = torch.from_numpy(xh).cuda()
-        ws = torch.zeros(max(256, gpu.Workspace.bytes_for(N, K)), dtype=torch.uint8, device="cuda")
+        need = gpu.Workspace.bytes_for(N, K, split)
+        ws = torch.zeros(max(256, need), dtype=torch.uint8, device="cuda")
         y_ref = torch.full((N,), float("nan"), dtype=torch.float32, device="cuda")
         y_na = torch.full((N,), float("nan"), dtype=torch.float32, device="cuda")
-        assert _call_ws(lib, x, wq, sc, fmt, inv, y_ref, N, K, ws) == 0, lib.q4_last_error()
+        assert _call_ws(lib, x, wq, sc, fmt, inv, y_ref, N, K, ws, split) == 0, lib.q4_last_error()
         for rep in range(2):
-            assert _call_noalloc(lib, x, wq, sc, fmt, inv, y_na, N, K) == 0, lib.q4_last_error()
+            assert _call_noalloc(lib, x, wq, sc, fmt, inv, y_na, N, K, split) == 0, lib.q4_last_error()
             torch.cuda.synchronize()
             assert (to_np(y_na).view(np.uint32) == to_np(y_ref).view(np.uint32)).all(), (N, K, rep)
         ref = O.gemv_ref(q, s_used, xh, inv)
