@@ -17,10 +17,12 @@
 //  * Attention is split along the cached keys (flash-decoding): workgroup
 //    (head group, split) serves up to 4 query heads of one KV head over 32
 //    keys (8 per wave), with every K and V row it needs in flight from the
-//    start; a second kernel merges the splits' (max, sum, accumulator)
-//    triples. The grid covers the cache capacity and splits past the current
-//    length exit at once, so the launch shape does not depend on the
-//    position; a 1024-key window of 8 KV heads with 2 query heads each is
+//    start (hd 512 with whole groups of 16 query heads per KV head: 16 heads
+//    at a time, on the matrix cores); a second kernel merges the splits'
+//    (max, sum, accumulator) triples. The grid covers the cache capacity, so
+//    the launch shape does not depend on the position: splits past the
+//    current length run through with every key masked, and the merge leaves
+//    them out; a 1024-key window of 8 KV heads with 2 query heads each is
 //    256 workgroups. Per-head vector work (q/k norms, RoPE) runs once per
 //    wave in row layout (EPL elements per lane: 64-lane sums, the RoPE
 //    partner from lane l ^ 32), not once per key row: the kernel is bound by
@@ -509,8 +511,8 @@ struct SplitMl {  // (one load of a pair; the workspace is float-aligned, which 
 // the p of its own keys by lane broadcast) and after the waves' p V
 // partials. Per head the split's maximum m, sum l of exp(s - m) and
 // unnormalised p V go to the workspace for attn_merge_kernel. Splits past
-// the length exit at once (the grid covers the cache depth, so a captured
-// graph replays every position).
+// the length run with every key masked (the grid covers the cache depth, so a
+// captured graph replays every position).
 //
 // With PREP (prepkv folded in, vk/prepkv.comp:16-30): the split holding this
 // token's slot forms its K and V with fresh_kv (the same bits as

@@ -1104,15 +1104,15 @@ __global__ void __launch_bounds__(256) w8q_kernel(const GemmArgs g) {
 // count leaves a last k-step with one block: the other block's scales read
 // as zero, and its (clamped, stale) A chunks add nothing. With split > 1,
 // blockIdx.y selects a contiguous range of k-steps and fp32 partials go to P.
-// KG = 2 runs two groups of 4 waves (512 threads, two waves per SIMD, each
-// with its own A ring) over the two halves of the workgroup's k-steps: one
-// wave per SIMD is bound by its own instruction issue (dequant, A reads,
-// addresses between the MFMAs), and a second wave issues while the first
-// one's MFMAs run. Both groups run the same number of k-steps (barriers stay
-// paired): for an odd count the second group runs one k-step fewer and
-// then joins the first group's last barrier without any MFMA, so no
-// operand is multiplied that a one-group launch would not multiply (a
-// surplus step on zero scales would turn an Inf in X into NaN). The groups
+// KG = 2 runs two groups of NWV waves, each with its own A ring, over the two
+// halves of the workgroup's k-steps. With NWV = 4 these are 512 threads, two
+// waves per SIMD: one wave per SIMD is bound by its own instruction issue
+// (dequant, A reads, addresses between the MFMAs), and a second wave issues
+// while the first one's MFMAs run. Both groups pass the same barriers: for an
+// odd count the second group runs one k-step fewer and then joins the first
+// group's last barrier without any MFMA, so no operand is multiplied that a
+// one-group launch would not multiply (a surplus step on zero scales would
+// turn an Inf in X into NaN). The groups
 // then exchange halves of their accumulators through LDS, add them (acc0 +
 // acc1) and each runs the epilogue of its half.
 // NWV = 2 (with KG = 2) narrows the tile to 128 columns: two waves per group,
@@ -1853,7 +1853,14 @@ static void launch_w4a16(const GemmArgs& g, const W4Plan& p, hipStream_t st) {
 // W4A8 tile: the largest of 128 x 64, 128 x 32, 64 x 64, 64 x 32 (64-row tiles
 // alone up to 64 rows) whose grid gives at least W4A8_MIN_WGS workgroups,
 // else 64 x 32: one 128-row workgroup fills a CU, and a smaller tile repeats
-// the requantization (fewer rows) or the loads of A (fewer columns).
+// the requantization (fewer rows) or the loads of A (fewer columns). 128 x 64 /
+// 128 x 32 / 64 x 64 / 64 x 32, us (* the rule's): M 128, 15360 x 3840 20.6* / 26.1 /
+// 24.5 / 26.1; M 512, 16000 x 8000 108* / 166 / 137 / 170; M 180, 3840 x 15360 44.8 /
+// 35.4* / 34.2 / 40.3; M 128, 2000 x 2048 13.1 / 10.2 / 10.3 / 9.2*. It looks at one
+// round of workgroups only: where a tile leaves a short second round, a larger
+// one is better (M 384, 3840 x 15360 51.5 / 75.3* / 61.2 / 62.9; M 256, 6000 x 1600
+// 13.6 / 15.8* / 15.8 / 13.2). The 256-column tiles before took 45 us at K 1024 to
+// 540 at K 15360 whatever M up to 512: every shape tried gained 2 times or more.
 constexpr int W4A8_MIN_WGS = 192;
 template <int BM, int BN>
 static bool launch_w4a8(const GemmArgs& g, bool force, hipStream_t st) {

@@ -116,11 +116,6 @@ __device__ inline v4u ld16(const void* p) {
   asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(r) : "v"(p));
   return r;
 }
-__device__ inline v2u ld8(const void* p) {
-  v2u r;
-  asm volatile("global_load_dwordx2 %0, %1, off" : "=v"(r) : "v"(p));
-  return r;
-}
 // (a & m) | c in one VALU operation. v_and_or_b32 takes no literal
 // constants and reads at most one SGPR: m comes in an SGPR, c in a VGPR
 // (both loop-invariant, so they are set up once).
