@@ -735,8 +735,8 @@ attn_split_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, 
 // the cache is read once for all 16 heads instead of once per 4. The fp32 q
 // and p are each split into three fp16 parts (11 + 11 + 2 bits) after an
 // exact power-of-two scaling (q: a head's largest element to [2^13, 2^14); p:
-// 2^14): the parts sum to the fp32 value itself, except that bits below 2^-38
-// of the scale are rounded off, and their products with the fp16 cache are
+// 2^14): the parts sum to the fp32 value itself, except that bits below 2^-37
+// of the scale are cut off, and their products with the fp16 cache are
 // exact in the fp32 accumulators. Zero parts and parts of both signs do not
 // multiply an Inf (in the cache) as their sum would: scores or sums that come
 // out not finite are taken again with fp32 operands (16x16x4), which gives an
@@ -754,12 +754,14 @@ attn_split_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, 
 // 16-byte V loads of 8 keys hold the B operands of 8 MFMAs, transposed in the
 // lane by byte permutes, and its results are 8 consecutive dims.
 // Measured at 8101 keys (256 splits, 16.6 MB of cache per layer), split and
-// merge of four layers: 160 us with the 4-head kernel, 71.0 (69.0 with two
-// parts per value and no check); the same split on the fp32 matrix
-// instruction alone (8 times the MFMA cycles, K and V widened first) took 2.6
-// us more per layer. Error against 64 bits with fp32 outputs, 2-norm, mean
-// over positions 1 to 8191 and score spreads of 0.25 to 4: 1.0e-7 to 6.8e-7
-// with the 4-head kernel, 1.0e-7 to 5.2e-7 here.
+// merge of four layers: 160 us with the 4-head kernel, 69.8 (68.6 with two
+// parts per value and no check; 70.6 with parts rounded to nearest, two
+// conversions more per value); the same split on the fp32 matrix instruction
+// alone (8 times the MFMA cycles, K and V widened first) took 2.6 us more per
+// layer. Error against 64 bits with fp32 outputs, 2-norm, mean over positions
+// up to 64, 2000 and 8191: 1.9e-7, 2.6e-7 and 3.3e-7 with the 4-head kernel,
+// 1.5e-7, 2.1e-7 and 2.4e-7 here; with scores 4 times as large 3.7e-7, 4.7e-7
+// and 6.4e-7, here 2.5e-7, 3.6e-7 and 4.9e-7.
 template <bool PREP>
 __global__ void __launch_bounds__(256)
 attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qnw, const float* __restrict__ cs,
@@ -816,18 +818,20 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
   // (2) q norm and RoPE of this wave's heads, their scaled parts to LDS; with
   //     the fresh slot in this split, this token's K and V through the wave's
   //     own LDS rows
+  // (towards zero, two values per conversion: what is left over is exact, so
+  // the rounding of the first two parts does not matter)
   auto parts = [](const float(&v)[8], v4u(&pt)[3]) {
-    v8h h, m, l;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      h[e] = (_Float16)v[e];
-      const float r = v[e] - (float)h[e];
-      m[e] = (_Float16)r;
-      l[e] = (_Float16)(r - (float)m[e]);
+    for (int e = 0; e < 4; ++e) {
+      float a = v[2 * e], b = v[2 * e + 1];
+#pragma unroll
+      for (int u = 0; u < 3; ++u) {
+        const v2h h = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(a, b));
+        pt[u][e] = __builtin_bit_cast(uint32_t, h);
+        a = fmaf((float)h[0], -1.0f, a);
+        b = fmaf((float)h[1], -1.0f, b);
+      }
     }
-    pt[0] = __builtin_bit_cast(v4u, h);
-    pt[1] = __builtin_bit_cast(v4u, m);
-    pt[2] = __builtin_bit_cast(v4u, l);
   };
 #pragma unroll
   for (int i = 0; i < HPW; ++i) {
@@ -969,7 +973,7 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
       if (8 * lg + s >= n) vv[s] = v4u{0u, 0u, 0u, 0u};
   }
   v4f o[8];
-  float fin = 0.0f;  // stays zero while the sums are finite
+  v4f fin = {};  // stays zero while the sums are finite
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
@@ -978,13 +982,13 @@ attn_split_mm_kernel(const float* __restrict__ qkv, const float* __restrict__ qn
                     __builtin_amdgcn_perm(vv[5][w], vv[4][w], sel), __builtin_amdgcn_perm(vv[7][w], vv[6][w], sel)};
     o[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int u = 0; u < 3; ++u)
+    for (int u = 2; u >= 0; --u)  // the small products first: one rounding at the sums' size
       o[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, pp[u]), __builtin_bit_cast(v8h, bt), o[e], 0,
                                                     0, 0);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) fin = fmaf(o[e][v], 0.0f, fin);
+    for (int v = 0; v < 4; ++v) fin[v] = fmaf(o[e][v], 0.0f, fin[v]);
   }
-  if (__builtin_amdgcn_ballot_w64(fin != 0.0f)) {  // (a NaN is not equal to zero)
+  if (__builtin_amdgcn_ballot_w64((fin[0] + fin[1]) + (fin[2] + fin[3]) != 0.0f)) {  // (a NaN is not equal to zero)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       o[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
