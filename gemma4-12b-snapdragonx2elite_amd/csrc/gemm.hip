@@ -1805,9 +1805,10 @@ static int w4a16_kgroups(int M, int N, int K, int split) {
 //    4032: 18.4 -> 15.4, wide 17.8; M 64, 6000 x 1600: 18.1 -> 16.4, wide
 //    17.8; from four splits on it loses: M 100, 1040 x 8000 19.5 -> 20.4).
 //    Partials of an N that is no multiple of 4 are stored and read element by
-//    element: above 40000 outputs their groups stay at 8 (M 41, 1274 x 7520
-//    20.5, with 4 22.8), and above 100000 one split stays one (M 219, 2951 x
-//    1120 16.0, two splits 20.0; M 68, 985 x 1920 20.0, three splits 14.8).
+//    element: above 40000 outputs few rows alone do not shorten their groups
+//    (M 41, 1274 x 7520 20.5, with 4 22.8), and above 100000 neither does a small
+//    grid (M 219, 2951 x 1120 16.0, two splits 20.0; M 347, 849 x 3200 21.8, six
+//    splits 22.9; but M 68, 985 x 1920 20.0, three splits 14.8).
 // The narrow plan is taken where its groups run fewer k-steps than the wide
 // plan's waves, where it leaves no second kernel, or where the partials it
 // saves (~0.1 us per split and 0.8 us per million fp32 values, element by
@@ -1828,8 +1829,7 @@ static W4Plan w4a16_plan(int M, int N, int K) {
     const long mn = (long)M * N;
     const bool odd = N % 4 != 0;  // partials stored and read element by element
     int s = min(round, nk / (M <= 48 && (!odd || mn <= 40000) ? 8 : 16));
-    if (t * s < 64 && s < 4 && (s > 1 || !odd || mn <= 100000))
-      s = max(s, min(min(round, 128 / t), nk / 8));
+    if (t * s < 64 && s < 4 && (!odd || mn <= 100000)) s = max(s, min(min(round, 128 / t), nk / 8));
     s = min(s, p.split);
     const bool shorter = 4 * s >= 3 * p.split;  // nk / (2 s) k-steps per group against nk / split
     const long saved = ((odd ? 4 : 1) * mn + 125000) * (p.split - s), reread = 56000L * ceil_div(nk, 2 * s);

@@ -319,6 +319,18 @@ def test_attn_infinities_in_the_cache(gpu, nH, nkv, stride, window, pos, where):
     assert (np.isinf(got) == np.isinf(ref)).all() and (got[np.isinf(ref)] == ref[np.isinf(ref)]).all()
     ok = np.isfinite(ref)
     assert O.normwise_rel_err(got[ok], ref[ok]) <= 1e-4
+    # and with this token's K and V formed in the same launch
+    koff, voff = nH * hd, nH * hd + nkv * hd
+    kw = dict(nkv=nkv, hd=hd, koff=koff, voff=voff, keqv=False, stride=stride, window=window, dyn=dyn)
+    knw = _t((rng.random(hd) + 0.5).astype(np.float32))
+    kc1, vc1 = _t(kc, torch.float16), _t(vc, torch.float16)
+    kc2, vc2 = kc1.clone(), vc1.clone()
+    gpu.prepkv(_t(qkv), knw, _t(cs), _t(sn), kc1, vc1, **kw)
+    o1 = gpu.attn(_t(qkv), _t(qnw), _t(cs), _t(sn), kc1, vc1, nH=nH, nkv=nkv, hd=hd, stride=stride, window=window, qoff=0,
+                  grp=nH // nkv, dyn=dyn)
+    o2 = gpu.prepkv_attn(_t(qkv), knw, _t(qnw), _t(cs), _t(sn), kc2, vc2, nH=nH, qoff=0, grp=nH // nkv, **kw)
+    assert torch.equal(o1.isnan(), o2.isnan()) and torch.equal(o1.nan_to_num(), o2.nan_to_num())
+    assert bool(o1.isnan().any()) and bool(o1.isfinite().any())
 
 
 @pytest.mark.parametrize("nsplit_live", [1, 63, 64, 65, 120, 256, 257, 300])
